@@ -139,6 +139,28 @@ struct mi_ctx {
   int64_t quad_entries = 0;
   bool use_quad() const { return quad_enable && quad_ent.p != nullptr; }
   void build_quad_table(const uint32_t* d_perm, int64_t n, const int64_t* d_famoff);
+  // back projection by image tiles with the runs in LDS (pmrt_tile.hip), the
+  // default where build_tile_table accepts the geometry
+  bool use_tile = false;
+  int64_t tile_entries = 0;
+  DBuf<uint32_t> tile_phase_off, tile_row;
+  DBuf<uint4> tile_hdr;
+  DBuf<int32_t> tile_off, tile_order;
+  DBuf<float> tile_w;
+  DBuf<int2> tile_rng, tile_segs;
+  mi::TileArgs tile{};
+  void release_tile() {
+    use_tile = false;
+    tile_entries = 0;
+    tile_phase_off.release(); tile_hdr.release(); tile_row.release(); tile_segs.release(); tile_off.release(); tile_order.release();
+    tile_w.release(); tile_rng.release();
+    tile = mi::TileArgs{};
+  }
+  int64_t tile_bytes() const {
+    return static_cast<int64_t>(tile_phase_off.bytes() + tile_hdr.bytes() + tile_row.bytes() + tile_off.bytes() +
+                                tile_order.bytes() + tile_w.bytes());
+  }
+  bool build_tile_table();
   std::vector<mi::Family> h_fams;
   std::unordered_map<int64_t, int> fam_lookup;  // (seg,view,tang,a0) -> family
   int64_t num_basic_elements = 0;
@@ -351,6 +373,9 @@ struct mi_ctx {
     else if (use_slab)
       mi::launch_back_project_slab(mode, slab, subset_begin(subset), subset_end(subset), d_proj, d_img, dims, data,
                                    st);
+    else if (use_tile)
+      mi::launch_back_project_tile(mode, tile, subset_begin(subset), subset_end(subset), d_proj, d_img, dims, data,
+                                   st);
     else if (use_quad())
       mi::launch_back_project_quad(mode, quad_off.p, quad_ent.p, subset_begin(subset), subset_end(subset), d_proj,
                                    d_img, dims, data, bp_tuning, st, block_bins);
@@ -378,6 +403,8 @@ struct mi_ctx {
       bp_bytes = img_bytes + proj_bytes + static_cast<int64_t>(tof_bp_rec.bytes() + list_off.bytes());
     else if (use_quad())
       bp_bytes = img_bytes + proj_bytes + static_cast<int64_t>(quad_ent.bytes() + quad_off.bytes());
+    else if (use_tile)
+      bp_bytes = img_bytes + proj_bytes + tile_bytes();
     else
       bp_bytes = img_bytes + proj_bytes +
                  static_cast<int64_t>(entries.bytes() + list_off.bytes() + entry_d.bytes() + slab_hdr.bytes() +
@@ -645,6 +672,12 @@ void mi_ctx::build_table() {
     return;
   }
   release_slab();
+  release_tile();
+  if (build_tile_table()) {
+    use_tile = true;
+    return;
+  }
+  release_tile();
   const int nsub = plan->num_subsets();
   const int ncols = dims.ncols;
   // entry offsets per family (family order == subset order)
@@ -1055,11 +1088,206 @@ bool mi_ctx::build_slab_table() {
   return true;
 }
 
+// The tile table (pmrt_tile.hip) of a non-TOF matrix whose families cover
+// whole runs; false where the geometry does not qualify (the column table is
+// built instead). Images of up to 32 planes stay with the column kernels,
+// which pack them better than a wave of 64 planes.
+bool mi_ctx::build_tile_table() {
+  const mi_geometry& g = plan->geometry();
+  if (!slab_allowed || slab_enable || quad_enable || ntof > 1 || dims.nz <= 32 || h_fams.empty()) return false;
+  const auto& keys = plan->family_keys();
+  const int nsub = plan->num_subsets(), nfam = static_cast<int>(h_fams.size()), ntang = g.num_tangential_poss;
+  // units: the (segment, view) viewgrams, ntang consecutive families each
+  if (nfam % ntang || int64_t{g.num_views} * ntang >= (1 << 24) || plan->nseg() > 255) return false;
+  const int nunits = nfam / ntang;
+  std::vector<int4> hunits(nunits);
+  std::vector<int2> hpos(nfam), hsegs(256, make_int2(0, 1 << 16));
+  int longest = 0;
+  for (int u = 0; u < nunits; ++u) {
+    const auto& k0 = keys[static_cast<size_t>(u) * ntang];
+    const mi::Family& f0 = h_fams[static_cast<size_t>(u) * ntang];
+    const int64_t seg_off = plan->segment_offset(k0.seg);
+    for (int i = 0; i < ntang; ++i) {
+      const int fi = u * ntang + i;
+      const mi::Family& f = h_fams[fi];
+      if (keys[fi].a0 != 0 || keys[fi].seg != k0.seg || keys[fi].view != k0.view ||
+          keys[fi].tang != g.min_tangential_pos_num + i || f.nax != plan->num_axial(k0.seg) || f.ppa < 1 ||
+          f.ppa != f0.ppa || f.sino_base != seg_off + (int64_t{k0.view} * ntang + i) * f.nax)
+        return false;
+      hpos[fi] = make_int2(k0.view, i);
+    }
+    const int slot = k0.seg - g.min_segment_num, len = f0.ppa * (f0.nax - 1) + 1;
+    hsegs[slot] = make_int2(static_cast<int>(seg_off), f0.nax | f0.ppa << 16);
+    hunits[u] = make_int4(slot, len, 0, k0.view);
+    longest = std::max(longest, len);
+  }
+  const int nslot = (dims.nz + 63) / 64;
+  if (longest > 64 * nslot) return false;
+  std::vector<int32_t> hunit_off(nsub + 1);
+  for (int s = 0; s <= nsub; ++s) {
+    if (plan->subset_family_begin(s) % ntang) return false;
+    hunit_off[s] = plan->subset_family_begin(s) / ntang;
+  }
+  const int ntx = (dims.nx + mi::kTileSide - 1) / mi::kTileSide, nty = (dims.ny + mi::kTileSide - 1) / mi::kTileSide;
+  const int ntiles = ntx * nty;
+  auto upload = [&](auto& buf, const auto& v) {
+    buf.alloc(v.size());
+    HIPCHECK(hipMemcpyAsync(buf.p, v.data(), buf.bytes(), hipMemcpyHostToDevice, stream));
+  };
+  DBuf<int4> d_units;
+  DBuf<int2> d_pos;
+  DBuf<int32_t> d_unit_off;
+  upload(d_units, hunits);
+  upload(d_pos, hpos);
+  upload(d_unit_off, hunit_off);
+  // pass 1: tangential ranges and the zeros a row needs
+  tile_rng.alloc(static_cast<size_t>(ntiles) * g.num_views);
+  mi::launch_fill_int2(tile_rng.p, static_cast<int64_t>(tile_rng.n), make_int2(0x7fffffff, -1), stream);
+  DBuf<int> d_need;  // planes after a run's start, planes up to its end, flag
+  d_need.alloc(3);
+  HIPCHECK(hipMemsetAsync(d_need.p, 0, d_need.bytes(), stream));
+  mi::launch_tile_range(fams.p, d_pos.p, nfam, pool.p, dims, ntx, g.num_views, tile_rng.p, d_need.p, stream);
+  HIPCHECK(hipGetLastError());
+  int need[3];
+  HIPCHECK(hipMemcpyAsync(need, d_need.p, sizeof(need), hipMemcpyDeviceToHost, stream));
+  HIPCHECK(hipStreamSynchronize(stream));
+  if (need[1] <= 0) return false;  // no element reaches the image
+  mi::TileArgs A{};
+  A.ntx = ntx;
+  A.ntiles = ntiles;
+  A.nsub = nsub;
+  A.nviews = g.num_views;
+  A.stride = std::max({need[0], need[1], (longest + 63) / 64 * 64});  // rows are written 64 lanes at a time
+  A.lead = std::max(A.stride, 64 * nslot);  // also the zeros that padding entries read
+  A.longest = longest;
+  const int rows = (mi::kTileLdsBytes / 4 - A.lead - 64 * nslot) / A.stride;
+  if (rows < 32) return false;
+  A.lds_floats = mi::kTileLdsBytes / 4;
+  // pass 2: phases
+  const int64_t nst = static_cast<int64_t>(nsub) * ntiles;
+  DBuf<uint32_t> slot, nphase, nrow, row_off, phase_row;
+  slot.alloc(static_cast<size_t>(ntiles) * nunits);
+  nphase.alloc(nst + 1);
+  nrow.alloc(nst + 1);
+  HIPCHECK(hipMemsetAsync(nphase.p + nst, 0, sizeof(uint32_t), stream));
+  HIPCHECK(hipMemsetAsync(nrow.p + nst, 0, sizeof(uint32_t), stream));
+  mi::launch_tile_phases(d_units.p, d_unit_off.p, nsub, ntiles, nunits, ntang, g.num_views, tile_rng.p, rows, slot.p,
+                         nphase.p, nrow.p, d_need.p + 2, stream);
+  auto scan = [&](const DBuf<uint32_t>& in, DBuf<uint32_t>& out, int64_t n) {  // n counts, then the total
+    out.alloc(n);
+    size_t tb = 0;
+    HIPCHECK(mi::exclusive_scan_u32(nullptr, tb, in.p, out.p, static_cast<int>(n), stream));
+    DBuf<char> tmp;
+    tmp.alloc(std::max<size_t>(tb, 1));
+    HIPCHECK(mi::exclusive_scan_u32(tmp.p, tb, in.p, out.p, static_cast<int>(n), stream));
+    HIPCHECK(hipStreamSynchronize(stream));
+  };
+  scan(nphase, tile_phase_off, nst + 1);
+  scan(nrow, row_off, nst + 1);
+  uint32_t totals[2];
+  HIPCHECK(hipMemcpy(&totals[0], tile_phase_off.p + nst, sizeof(uint32_t), hipMemcpyDeviceToHost));
+  HIPCHECK(hipMemcpy(&totals[1], row_off.p + nst, sizeof(uint32_t), hipMemcpyDeviceToHost));
+  HIPCHECK(hipMemcpy(need, d_need.p, sizeof(need), hipMemcpyDeviceToHost));
+  if (need[2]) return false;
+  const uint32_t total_rows = totals[1];
+  const int64_t nph = totals[0], nlists = nph * mi::kTileCols;
+  if (nlists >= (int64_t{1} << 31) - 2) return false;
+  upload(tile_segs, hsegs);
+  tile_row.alloc(static_cast<size_t>(total_rows) + mi::kTileRowSlack);
+  HIPCHECK(hipMemsetAsync(tile_row.p + total_rows, 0, mi::kTileRowSlack * sizeof(uint32_t), stream));
+  phase_row.alloc(nph);
+  mi::launch_tile_rows(d_units.p, d_unit_off.p, nsub, ntiles, nunits, ntang, g.num_views, tile_rng.p, rows,
+                       tile_phase_off.p, row_off.p, tile_row.p, phase_row.p, d_need.p + 2, stream);
+  A.phase_off = tile_phase_off.p;
+  A.row = tile_row.p;
+  A.segs = tile_segs.p;
+  A.rng = tile_rng.p;
+  // pass 3: entries per list, in groups of 4
+  DBuf<uint32_t> counts, groups, list_start, group_off;
+  counts.alloc(nlists + 1);
+  HIPCHECK(hipMemsetAsync(counts.p, 0, counts.bytes(), stream));
+  for (int s = 0; s < nsub; ++s)
+    mi::launch_tile_count(fams.p, d_pos.p, plan->subset_family_begin(s), plan->subset_family_begin(s + 1), ntang, pool.p,
+                          s, dims, A, nunits, slot.p, counts.p, stream);
+  groups.alloc(nlists + 1);
+  mi::launch_tile_groups(counts.p, nlists + 1, groups.p, d_need.p + 2, stream);
+  HIPCHECK(hipGetLastError());
+  scan(counts, list_start, nlists + 1);
+  scan(groups, group_off, nlists + 1);
+  counts.release();
+  HIPCHECK(hipMemcpy(&totals[0], list_start.p + nlists, sizeof(uint32_t), hipMemcpyDeviceToHost));
+  HIPCHECK(hipMemcpy(&totals[1], group_off.p + nlists, sizeof(uint32_t), hipMemcpyDeviceToHost));
+  HIPCHECK(hipMemcpy(need, d_need.p, sizeof(need), hipMemcpyDeviceToHost));
+  const int64_t nent = totals[0], nslots = 4 * static_cast<int64_t>(totals[1]);
+  if (need[2]) return false;
+  tile_hdr.alloc((nph + mi::kTileHdrSlack) * mi::kTileWaves);
+  mi::launch_tile_headers(groups.p, group_off.p, phase_row.p, total_rows, nph, tile_hdr.p, stream);
+  // pass 4: every element's list and entry, sorted by list, to its place
+  std::vector<int64_t> fam_off(nfam + 1, 0);
+  for (int i = 0; i < nfam; ++i) fam_off[i + 1] = fam_off[i] + h_fams[i].row_len;
+  const int64_t n = fam_off.back();
+  if (n >= (int64_t{1} << 31)) throw ApiError(MI_ERR_ARGUMENT, "back-projection table above 2^31 entries");
+  DBuf<int64_t> d_fam_off;
+  upload(d_fam_off, fam_off);
+  tile_off.alloc(nslots + mi::kTileEntSlack);
+  tile_w.alloc(nslots + mi::kTileEntSlack);
+  HIPCHECK(hipMemsetAsync(tile_off.p, 0, tile_off.bytes(), stream));  // padding: weight 0 times the leading zeros
+  HIPCHECK(hipMemsetAsync(tile_w.p, 0, tile_w.bytes(), stream));
+  DBuf<uint32_t> keys_in, keys_out, vals_in, vals_out;
+  DBuf<int2> raw;
+  keys_in.alloc(n);
+  raw.alloc(n);
+  for (int s = 0; s < nsub; ++s)
+    mi::launch_tile_make(fams.p, d_pos.p, plan->subset_family_begin(s), plan->subset_family_begin(s + 1), ntang, pool.p,
+                         s, dims, A, nunits, slot.p, static_cast<uint32_t>(nlists), d_fam_off.p, keys_in.p, raw.p,
+                         stream);
+  keys_out.alloc(n);
+  vals_in.alloc(n);
+  vals_out.alloc(n);
+  mi::launch_iota(vals_in.p, n, stream);
+  int end_bit = 1;
+  while ((int64_t{1} << end_bit) <= nlists) ++end_bit;
+  {
+    size_t tb = 0;
+    HIPCHECK(mi::radix_sort_pairs(nullptr, tb, keys_in.p, keys_out.p, vals_in.p, vals_out.p, static_cast<int>(n), end_bit,
+                                  stream));
+    DBuf<char> tmp;
+    tmp.alloc(std::max<size_t>(tb, 1));
+    HIPCHECK(mi::radix_sort_pairs(tmp.p, tb, keys_in.p, keys_out.p, vals_in.p, vals_out.p, static_cast<int>(n), end_bit,
+                                  stream));
+    HIPCHECK(hipStreamSynchronize(stream));
+  }
+  mi::launch_tile_place(keys_out.p, vals_out.p, raw.p, list_start.p, group_off.p, nent, tile_off.p, tile_w.p, stream);
+  HIPCHECK(hipGetLastError());
+  // launch order: the tiles with the most entries first, so that the last
+  // workgroups to run are short ones
+  DBuf<uint32_t> d_work;
+  d_work.alloc(ntiles);
+  mi::launch_tile_work(group_off.p, tile_phase_off.p, nsub, ntiles, d_work.p, stream);
+  std::vector<uint32_t> work(ntiles);
+  HIPCHECK(hipMemcpyAsync(work.data(), d_work.p, d_work.bytes(), hipMemcpyDeviceToHost, stream));
+  HIPCHECK(hipStreamSynchronize(stream));
+  std::vector<int32_t> order(ntiles);
+  for (int t = 0; t < ntiles; ++t) order[t] = t;
+  std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return work[a] > work[b]; });
+  upload(tile_order, order);
+  HIPCHECK(hipStreamSynchronize(stream));
+  HIPCHECK(mi::tile_allow_lds(mi::kTileLdsBytes));
+  A.hdr = tile_hdr.p;
+  A.off = tile_off.p;
+  A.w = tile_w.p;
+  A.order = tile_order.p;
+  tile = A;
+  tile_entries = n;
+  return true;
+}
+
 void mi_ctx::set_up(const mi_geometry& g, int nsub) {
   HIPCHECK(hipSetDevice(device));
   // release everything of a previous set-up
   pool.release(); pool_ops.release(); fams.release(); tasks.release(); list_off.release(); entries.release();
   release_slab();
+  release_tile();
   img.release(); img2.release(); sino.release(); ratio.release(); stage_img.release(); stage_sino.release();
   y.release(); add.release(); mult.release(); ones.release(); vg_small.release(); x.release(); sens.clear();
   vg_off.release(); vg_len.release(); partial.release(); prior_partial.release();
@@ -1201,7 +1429,7 @@ int mi_get_info(mi_ctx* ctx, mi_info* out) {
     out->num_basic_elements = ctx->num_basic_elements;
     out->num_families = static_cast<int64_t>(ctx->h_fams.size());
     out->num_matrix_elements = ctx->num_matrix_elements;
-    out->num_table_entries = static_cast<int64_t>(ctx->use_slab ? ctx->slab_ent.n : ctx->entries.n);
+    out->num_table_entries = static_cast<int64_t>(ctx->use_slab ? ctx->slab_ent.n : ctx->use_tile ? ctx->tile_entries : ctx->entries.n);
     out->num_nonzeros = ctx->num_nonzeros;
     out->device_bytes = static_cast<int64_t>(ctx->pool.bytes() + ctx->pool_ops.bytes() + ctx->fams.bytes() + ctx->tasks.bytes() +
                                              ctx->list_off.bytes() + ctx->entries.bytes() + ctx->img.bytes() +
@@ -1211,7 +1439,7 @@ int mi_get_info(mi_ctx* ctx, mi_info* out) {
                                              ctx->slab_hdr.bytes() + ctx->slab_ent.bytes() + ctx->slab_rng.bytes() +
                                              ctx->slab_tiles.bytes() + ctx->lors.bytes() + ctx->entry_d.bytes() +
                                              ctx->erf_tab.bytes() + ctx->tof_fp_rec.bytes() +
-                                             ctx->tof_bp_rec.bytes());
+                                             ctx->tof_bp_rec.bytes()) + ctx->tile_bytes();
     for (auto& s : ctx->sens) out->device_bytes += static_cast<int64_t>(s->bytes());
     out->num_subsets = ctx->plan->num_subsets();
     ctx->plan->symmetry_flags(out->symmetry_flags);

@@ -80,20 +80,20 @@ __global__ void __launch_bounds__(64) make_entries_kernel(const Family* __restri
 __global__ void __launch_bounds__(64) count_nonzeros_kernel(const Family* __restrict__ fams, int nfam,
                                                             const int2* __restrict__ pool, ImageDims d,
                                                             unsigned long long* __restrict__ total) {
-  const int fi = blockIdx.x;
-  if (fi >= nfam) return;
-  const Family f = fams[fi];
   unsigned long long cnt = 0;
-  for (int e = threadIdx.x; e < f.row_len; e += blockDim.x) {
-    int x, y, z;
-    decode(pool[f.row_start + e].x, x, y, z);
-    const int k = f.zsign * z + f.zadd0 - d.min_z;  // image z of axial position 0
-    // ppa*a in [-k, nz-1-k]
-    const int lo_num = -k, hi_num = d.nz - 1 - k;
-    int lo = lo_num <= 0 ? 0 : (lo_num + f.ppa - 1) / f.ppa;
-    int hi = hi_num < 0 ? -1 : hi_num / f.ppa;
-    if (hi > f.nax - 1) hi = f.nax - 1;
-    if (hi >= lo) cnt += static_cast<unsigned long long>(hi - lo + 1);
+  for (int fi = blockIdx.x; fi < nfam; fi += gridDim.x) {  // one atomic per workgroup, not per family
+    const Family f = fams[fi];
+    for (int e = threadIdx.x; e < f.row_len; e += blockDim.x) {
+      int x, y, z;
+      decode(pool[f.row_start + e].x, x, y, z);
+      const int k = f.zsign * z + f.zadd0 - d.min_z;  // image z of axial position 0
+      // ppa*a in [-k, nz-1-k]
+      const int lo_num = -k, hi_num = d.nz - 1 - k;
+      int lo = lo_num <= 0 ? 0 : (lo_num + f.ppa - 1) / f.ppa;
+      int hi = hi_num < 0 ? -1 : hi_num / f.ppa;
+      if (hi > f.nax - 1) hi = f.nax - 1;
+      if (hi >= lo) cnt += static_cast<unsigned long long>(hi - lo + 1);
+    }
   }
   for (int off = 32; off > 0; off >>= 1) cnt += __shfl_xor(cnt, off, 64);
   if (threadIdx.x == 0) atomicAdd(total, cnt);
@@ -139,7 +139,7 @@ void launch_make_entries(const Family* d_fams, int fam_begin, int fam_end, const
 void launch_count_nonzeros(const Family* d_fams, int nfam, const int2* d_pool, const ImageDims& dims,
                            unsigned long long* d_total, hipStream_t stream) {
   if (nfam <= 0) return;
-  hipLaunchKernelGGL(count_nonzeros_kernel, dim3(nfam), dim3(64), 0, stream, d_fams, nfam, d_pool, dims, d_total);
+  hipLaunchKernelGGL(count_nonzeros_kernel, dim3(nfam < 16384 ? nfam : 16384), dim3(64), 0, stream, d_fams, nfam, d_pool, dims, d_total);
 }
 
 void launch_iota(uint32_t* d_vals, int64_t n, hipStream_t stream) {

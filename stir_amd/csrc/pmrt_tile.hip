@@ -1,0 +1,542 @@
+// Back projection by image tiles, projection-data runs staged in LDS.
+//
+// What bounds it, and why it is built this way. A back projection gathers one
+// projection-data run (up to 127 floats) per table entry and adds it to one
+// image column. Read straight from memory (bp_kernel) nearly every gather
+// misses L1 and, starting at any 4-byte address, moves three 128-byte lines:
+// 7.2 cycles of a CU's L2 path for 64 lanes, against 2.3 for a run read from
+// LDS at any alignment. So one workgroup owns a tile of 8 x 8 columns, copies
+// the runs that cross it into LDS once and lets all 64 columns read them
+// there (each staged run is used by about nine entries at mMR size).
+//
+// Measured at mMR size (4.2e8 entries, 837 x 252 x 344 bins, 344 x 344 x 127
+// voxels): 10.8 ms with the column kernel, 6.4 ms with this one, which then
+// issues vector instructions in 76 % of the cycles (2.8e9 of them, 2.55e9 in
+// the entry loop), reads LDS in 47 % and fetches 17 GB from beyond L2. With
+// the copies left out it takes 4.8 ms, with the entries left out 2.4 ms: the
+// two overlap only in part. Half the waves per workgroup: 7.2 ms; three
+// workgroups of 8 waves and 53 KB per CU: 6.3 ms, four of 40 KB: 6.8 ms
+// (shorter lists, more padding).
+//
+// Work: phases. The (segment, view) viewgrams of a subset are taken in family
+// order; consecutive ones form a phase as long as the tangential positions
+// that cross the tile fill no more than `rows` LDS rows. Per phase the
+// workgroup copies the rows (loads that write LDS directly, all in flight at
+// once), then every wave walks its columns' entries. Two workgroups share a
+// CU, so one computes while the other waits for its rows.
+//
+// LDS rows: `stride` floats per run, the run spread to one value per image
+// plane (ppa planes per axial position: zeros between) and followed by zeros.
+// An entry holds the byte offset of plane 0 in its run's row, so lane l of
+// slot q reads plane 64 q + l; the stride is chosen so that planes the run
+// does not reach fall on zeros (of its own row, or of the end of the row
+// before it): no test, clamp or select, and the sum is the column table's,
+// term by term and bit for bit.
+//
+// Entries: per (phase, column) a list padded to groups of 4 with entries that
+// read the leading zeros with weight 0. Offsets and weights are two arrays;
+// each row of 16 lanes loads the same 16 consecutive entries and a group
+// takes its four by DPP broadcast inside the add and the multiply, so an entry
+// costs one address add, one two-slot LDS read, and a multiply and an add per
+// slot: 5 vector instructions for 128 planes, no scalar ones.
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+
+#include "pmrt_device.hpp"
+#include "pmrt_kernels.hpp"
+
+namespace mi {
+
+namespace {
+
+using namespace dev;
+
+constexpr int kTileCpw = kTileCols / kTileWaves;  // columns per wave
+
+// The matrix element of a family as the tile table sees it: tile, column of
+// the tile, plane of axial position 0; false when it reaches no image plane.
+struct TileElem {
+  int t, c, k;
+};
+__device__ inline bool tile_elem(const Family& f, int coords, const ImageDims& d, int ntx, TileElem& E) {
+  int x, y, z, xo, yo;
+  decode(coords, x, y, z);
+  inplane_any_op(f.inplane, x, y, xo, yo);
+  const int cx = xo - d.min_x, cy = yo - d.min_y;
+  E.k = f.zsign * z + f.zadd0 - d.min_z;
+  const int last = E.k + f.ppa * (f.nax - 1);
+  if (cx < 0 || cx >= d.nx || cy < 0 || cy >= d.ny || last < 0 || E.k >= d.nz) return false;
+  E.t = (cy / kTileSide) * ntx + cx / kTileSide;
+  E.c = (cy % kTileSide) * kTileSide + cx % kTileSide;
+  return true;
+}
+
+// pass 1, one wave per family: the tangential positions of every (tile, view)
+// and, over all elements, the most planes a row needs after a run's start
+// (rows[0]: nz - k) and before its end (rows[1]: run length + k)
+__global__ void __launch_bounds__(kWave) tile_range_kernel(const Family* __restrict__ fams,
+                                                           const int2* __restrict__ fam_pos, int nfam,
+                                                           const int2* __restrict__ pool, ImageDims d, int ntx,
+                                                           int nviews, int2* __restrict__ rng, int* __restrict__ need) {
+  const int fi = blockIdx.x;
+  if (fi >= nfam) return;
+  const Family f = fams[fi];
+  const int2 pos = fam_pos[fi];  // view, tangential index
+  const int lane = static_cast<int>(threadIdx.x);
+  int after = 0, before = 0;
+  for (int e0 = 0; e0 < f.row_len; e0 += kWave) {
+    const int e = e0 + lane;
+    TileElem E;
+    const bool ok = e < f.row_len && tile_elem(f, pool[f.row_start + (e < f.row_len ? e : 0)].x, d, ntx, E);
+    const int t = ok ? E.t : -1;
+    if (ok) {
+      after = max(after, d.nz - E.k);
+      before = max(before, f.ppa * (f.nax - 1) + 1 + E.k);
+    }
+    // neighbouring elements of a row lie mostly in one tile: one update per run of them
+    const int prev = __shfl_up(t, 1, kWave);
+    if (ok && (lane == 0 || prev != t)) {
+      int2* r = rng + static_cast<int64_t>(t) * nviews + pos.x;
+      atomicMin(&r->x, pos.y);
+      atomicMax(&r->y, pos.y);
+    }
+  }
+  for (int o = kWave / 2; o > 0; o >>= 1) {
+    after = max(after, __shfl_xor(after, o, kWave));
+    before = max(before, __shfl_xor(before, o, kWave));
+  }
+  // most families do not raise the maxima: read them first (a stale value
+  // only costs the atomic), or every wave would queue on one address
+  if (lane == 0 && before > 0) {
+    if (after > __hip_atomic_load(need, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(need, after);
+    if (before > __hip_atomic_load(need + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(need + 1, before);
+  }
+}
+
+// pass 2, one thread per (tile, subset): its units dealt to phases. FILL 0:
+// slot[tile][unit] = phase within (tile, subset) << 16 | first row, and the
+// numbers of phases and rows; 1: the rows and the first row of every phase. A
+// run's planes before its start fall on the end of the row before it: after a
+// longer run (of another segment) a row of zeros lies between.
+template <bool FILL>
+__global__ void tile_phase_kernel(const int4* __restrict__ units, const int32_t* __restrict__ unit_off, int nsub,
+                                  int ntiles, int nunits, int ntang, int nviews, const int2* __restrict__ rng, int rows,
+                                  uint32_t* __restrict__ slot, uint32_t* __restrict__ nphase,
+                                  uint32_t* __restrict__ nrow, const uint32_t* __restrict__ phase_off,
+                                  const uint32_t* __restrict__ row_off, uint32_t* __restrict__ row,
+                                  uint32_t* __restrict__ phase_row, int* __restrict__ bad) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= nsub * ntiles) return;
+  const int t = i / nsub, s = i - t * nsub;
+  int ph = -1, used = 0, prev = 0;
+  uint32_t n = 0;
+  for (int u = unit_off[s]; u < unit_off[s + 1]; ++u) {
+    const int4 U = units[u];  // segment slot, run length in planes, -, view
+    const int2 r = rng[static_cast<int64_t>(t) * nviews + U.w];
+    const int T = r.y - r.x + 1;
+    if (r.y < r.x) continue;
+    int gap = prev > U.y;
+    if (T > rows) *bad = 1;
+    if (ph < 0 || used + gap + T > rows) {
+      ++ph;
+      used = gap = 0;
+      if (FILL) phase_row[phase_off[i] + ph] = row_off[i] + n;
+    }
+    prev = U.y;
+    if (FILL) {
+      uint32_t* o = row + row_off[i] + n;
+      if (gap) *o++ = kTileZeroRow;
+      const uint32_t first = static_cast<uint32_t>(U.x) << 24 | static_cast<uint32_t>(U.w * ntang + r.x);
+      for (int k = 0; k < T; ++k) o[k] = first + k;
+    } else {
+      slot[static_cast<int64_t>(t) * nunits + u] = static_cast<uint32_t>(ph) << 16 | (used + gap);
+    }
+    used += gap + T;
+    n += gap + T;
+  }
+  if (!FILL) {
+    nphase[i] = ph + 1;
+    nrow[i] = n;
+    if (ph + 1 > 65535) *bad = 1;
+  }
+}
+
+// passes 3 and 4, one wave per family of subset s: the number of entries of
+// every (phase, column), then every element's key and entry in family order,
+// element order (elements without an image plane get the last key)
+template <bool COUNT>
+__global__ void __launch_bounds__(kWave) tile_entries_kernel(const Family* __restrict__ fams,
+                                                             const int2* __restrict__ fam_pos, int fam_begin,
+                                                             int fam_end, int ntang, const int2* __restrict__ pool,
+                                                             int subset, ImageDims d, TileArgs A, int nunits,
+                                                             const uint32_t* __restrict__ slot,
+                                                             uint32_t* __restrict__ counts, uint32_t none,
+                                                             const int64_t* __restrict__ fam_entry_off,
+                                                             uint32_t* __restrict__ keys, int2* __restrict__ raw) {
+  const int fi = fam_begin + blockIdx.x;
+  if (fi >= fam_end) return;
+  const Family f = fams[fi];
+  const int2 pos = fam_pos[fi];
+  const int unit = fi / ntang;
+  const int64_t base = COUNT ? 0 : fam_entry_off[fi];
+  for (int e = threadIdx.x; e < f.row_len; e += kWave) {
+    const int2 el = pool[f.row_start + e];
+    TileElem E;
+    uint32_t key = none;
+    int off4 = 0;
+    if (tile_elem(f, el.x, d, A.ntx, E)) {
+      const uint32_t sl = slot[static_cast<int64_t>(E.t) * nunits + unit];
+      const uint32_t ph = A.phase_off[static_cast<int64_t>(E.t) * A.nsub + subset] + (sl >> 16);
+      key = ph * kTileCols + E.c;
+      if (COUNT) {
+        atomicAdd(&counts[key], 1U);
+      } else {
+        const int row = static_cast<int>(sl & 0xffff) + pos.y - A.rng[static_cast<int64_t>(E.t) * A.nviews + pos.x].x;
+        off4 = 4 * (A.lead + row * A.stride - E.k);
+      }
+    }
+    if (!COUNT) {
+      keys[base + e] = key;
+      raw[base + e] = make_int2(off4, el.y);
+    }
+  }
+}
+
+// groups of 4 entries of every list
+__global__ void tile_groups_kernel(const uint32_t* __restrict__ counts, int64_t n, uint32_t* __restrict__ groups,
+                                   int* __restrict__ bad) {
+  for (int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; i < n;
+       i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+    groups[i] = (counts[i] + 3) / 4;
+    if (groups[i] > 255) *bad = 1;
+  }
+}
+
+// per (phase, wave): first group, the group counts of its columns (one byte
+// each) and the phase's first row; `slack` more phases without groups close
+// the list
+__global__ void tile_headers_kernel(const uint32_t* __restrict__ groups, const uint32_t* __restrict__ group_off,
+                                    const uint32_t* __restrict__ phase_row, uint32_t total_rows, int64_t nphase,
+                                    int64_t slack, uint4* __restrict__ hdr) {
+  for (int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; i < (nphase + slack) * kTileWaves;
+       i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+    const int64_t p = i / kTileWaves;
+    if (p >= nphase) {
+      hdr[i] = make_uint4(0, 0, 0, total_rows);
+      continue;
+    }
+    uint32_t c[2] = {0, 0};
+    for (int j = 0; j < kTileCpw; ++j) c[j / 4] |= groups[i * kTileCpw + j] << (8 * (j % 4));
+    hdr[i] = make_uint4(group_off[i * kTileCpw], c[0], c[1], phase_row[p]);
+  }
+}
+
+// groups of every tile (its work)
+__global__ void tile_work_kernel(const uint32_t* __restrict__ group_off, const uint32_t* __restrict__ phase_off, int nsub,
+                                 int ntiles, uint32_t* __restrict__ work) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= ntiles) return;
+  const int64_t a = phase_off[static_cast<int64_t>(t) * nsub], b = phase_off[static_cast<int64_t>(t + 1) * nsub];
+  work[t] = group_off[b * kTileCols] - group_off[a * kTileCols];
+}
+
+// sorted element r -> its place: 4 x its list's first group + its rank in the list
+__global__ void tile_place_kernel(const uint32_t* __restrict__ keys, const uint32_t* __restrict__ idx,
+                                  const int2* __restrict__ raw, const uint32_t* __restrict__ list_start,
+                                  const uint32_t* __restrict__ group_off, int64_t n, int32_t* __restrict__ off,
+                                  float* __restrict__ w) {
+  for (int64_t r = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; r < n;
+       r += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+    const uint32_t key = keys[r];
+    const int2 E = raw[idx[r]];
+    const int64_t at = 4 * static_cast<int64_t>(group_off[key]) + (r - list_start[key]);
+    off[at] = E.x;
+    w[at] = __int_as_float(E.y);
+  }
+}
+
+// lane j of the row of 16 lanes, in every lane of the row
+template <int J>
+__device__ inline int row_bcast(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, 0x150 + J, 0xf, 0xf, true);
+}
+// lane (i + 4) % 16 of the row of 16 lanes
+__device__ inline int row_next4(int v) { return __builtin_amdgcn_update_dpp(0, v, 0x120 + 12, 0xf, 0xf, true); }
+
+// p times lane J's w of the row. The multiply takes the broadcast itself (the
+// compiler moves it to a register first when two slots share the weight). A
+// DPP read needs two wait states after a VALU write of w, which the compiler
+// does not count across asm: the first multiply of a group brings them.
+template <int J>
+__device__ inline float mul_bcast(int w, float p) {
+  float r;
+  if constexpr (J == 0)
+    asm("s_nop 1\n\tv_mul_f32_dpp %0, %1, %2 row_newbcast:0 row_mask:0xf bank_mask:0xf" : "=v"(r) : "v"(w), "v"(p));
+  else if constexpr (J == 1)
+    asm("v_mul_f32_dpp %0, %1, %2 row_newbcast:1 row_mask:0xf bank_mask:0xf" : "=v"(r) : "v"(w), "v"(p));
+  else if constexpr (J == 2)
+    asm("v_mul_f32_dpp %0, %1, %2 row_newbcast:2 row_mask:0xf bank_mask:0xf" : "=v"(r) : "v"(w), "v"(p));
+  else
+    asm("v_mul_f32_dpp %0, %1, %2 row_newbcast:3 row_mask:0xf bank_mask:0xf" : "=v"(r) : "v"(w), "v"(p));
+  return r;
+}
+
+// an ordered (not invariant) load: it stays behind the copy of the registers it overwrites
+__device__ inline int entry_word(const char* base, unsigned off) {
+  return *(const MI_AS_GLOBAL int*)((const MI_AS_GLOBAL char*)base + off);
+}
+
+// the next four entries (lanes 0-3 of every row hold them) added to one column
+template <int NSLOT>
+__device__ inline void tile_group(int off, int w, const char* lds, int lane4, float (&acc)[NSLOT]) {
+  const int o[4] = {row_bcast<0>(off), row_bcast<1>(off), row_bcast<2>(off), row_bcast<3>(off)};
+  float v[4][NSLOT];
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int q = 0; q < NSLOT; ++q) v[j][q] = *reinterpret_cast<const float*>(lds + (lane4 + o[j]) + 256 * q);
+#pragma unroll
+  for (int q = 0; q < NSLOT; ++q) acc[q] = acc[q] + mul_bcast<0>(w, v[0][q]);
+#pragma unroll
+  for (int q = 0; q < NSLOT; ++q) acc[q] = acc[q] + mul_bcast<1>(w, v[1][q]);
+#pragma unroll
+  for (int q = 0; q < NSLOT; ++q) acc[q] = acc[q] + mul_bcast<2>(w, v[2][q]);
+#pragma unroll
+  for (int q = 0; q < NSLOT; ++q) acc[q] = acc[q] + mul_bcast<3>(w, v[3][q]);
+}
+
+template <int MODE, int NSLOT>
+__global__ void __launch_bounds__(kWave* kTileWaves) bp_tile_kernel(TileArgs A, int sb, int se,
+                                                                    const float* __restrict__ proj,
+                                                                    float* __restrict__ img, ImageDims d, BpData data,
+                                                                    int chunk) {
+  extern __shared__ float tile_lds[];
+  const int b = xcd_chunk_remap(static_cast<int>(blockIdx.x), chunk);
+  if (b >= A.ntiles) return;
+  const int t = as_const(A.order)[b];
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
+  const int lane = static_cast<int>(threadIdx.x % kWave);
+  const int lane4 = 4 * lane;
+  for (int i = threadIdx.x; i < A.lds_floats; i += kWave * kTileWaves) tile_lds[i] = 0.F;
+  float acc[kTileCpw][NSLOT];
+#pragma unroll
+  for (int c = 0; c < kTileCpw; ++c)
+#pragma unroll
+    for (int q = 0; q < NSLOT; ++q) acc[c][q] = 0.F;
+#if defined(__HIP_DEVICE_COMPILE__)
+  const char* lds = reinterpret_cast<const char*>(tile_lds);
+  const int l16 = lane % 16;
+  const uint32_t p0 = as_const(A.phase_off)[static_cast<int64_t>(t) * A.nsub + sb];
+  const uint32_t p1 = as_const(A.phase_off)[static_cast<int64_t>(t) * A.nsub + se];
+  // headers two phases ahead and rows one phase ahead, by vector loads (scalar
+  // loads in flight would make every LDS wait a full wait); lane l has the
+  // wave's row l
+  int zero = 0;
+  asm volatile("" : "+v"(zero));
+  const uint4* hp = A.hdr + static_cast<int64_t>(p0) * kTileWaves + wave + zero;
+  uint4 h = hp[0], h1 = hp[kTileWaves];
+  uint32_t rw = A.row[h.w + wave + kTileWaves * lane];
+  for (uint32_t p = p0; p < p1; ++p) {
+    const uint32_t group0 = __builtin_amdgcn_readfirstlane(h.x);
+    const uint32_t cnt[2] = {static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(h.y)),
+                             static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(h.z))};
+    const int nrow = static_cast<int>(__builtin_amdgcn_readfirstlane(h1.w) - __builtin_amdgcn_readfirstlane(h.w));
+    const int2 sg = A.segs[rw >> 24];  // device offset, nax | ppa << 16
+    const int base = sg.x + static_cast<int>(rw & 0xffffff) * (sg.y & 0xffff);
+    const char* po = reinterpret_cast<const char*>(A.off + 4 * static_cast<int64_t>(group0));
+    const char* pw = reinterpret_cast<const char*>(A.w + 4 * static_cast<int64_t>(group0));
+    unsigned at = 4 * l16;  // byte offset of this lane's entry
+    __syncthreads();        // the previous phase's rows have been read
+    float* dst = tile_lds + A.lead + wave * A.stride;
+    for (int l = 0, r = wave; r < nrow; ++l, r += kTileWaves, dst += kTileWaves * A.stride) {
+      const int np = __builtin_amdgcn_readlane(sg.y, l);
+      const __amdgpu_buffer_rsrc_t run =
+          run_buffer(as_const(proj), static_cast<unsigned>(__builtin_amdgcn_readlane(base, l)), np & 0xffff);
+#pragma unroll
+      for (int q = 0; q < NSLOT; ++q) {
+        // this lane's plane in the run; outside [0, 4 nax) the buffer reads 0
+        const int z = kWave * q + lane;
+        int v = 4 * z;
+        if ((np >> 16) == 2) v = z & 1 ? -4 : 2 * z;
+        else if ((np >> 16) > 2) v = z % (np >> 16) ? -4 : z / (np >> 16) * 4;
+        if (kWave * q < A.longest)
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(run, (__attribute__((address_space(3))) void*)(dst + kWave * q), 4,
+                                                   whole_offset(v), 0, 0, 0);
+      }
+    }
+    h = h1;
+    hp += kTileWaves;
+    h1 = hp[kTileWaves];
+    rw = A.row[h.w + wave + kTileWaves * lane];
+    int off = entry_word(po, at), w = entry_word(pw, at);
+    at += 64;
+    int off1 = entry_word(po, at), w1 = entry_word(pw, at);
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's rows are in LDS
+    __syncthreads();
+    int left = 4;  // groups left in the current chunk
+#pragma unroll
+    for (int c = 0; c < kTileCpw; ++c) {
+      for (uint32_t n = (cnt[c / 4] >> (8 * (c % 4))) & 255; n > 0; --n) {
+        tile_group<NSLOT>(off, w, lds, lane4, acc[c]);
+        if (--left == 0) {
+          // copied by hand, so that the next chunk's loads, requested after it,
+          // can write off1 and w1 themselves (a copy that the compiler places
+          // comes after the loads and waits for them)
+          asm volatile("v_mov_b32 %0, %2\n\tv_mov_b32 %1, %3\n\ts_nop 1"
+                       : "=&v"(off), "=&v"(w)
+                       : "v"(off1), "v"(w1)
+                       : "memory");
+          at += 64;
+          off1 = entry_word(po, at);
+          w1 = entry_word(pw, at);
+          left = 4;
+        } else {
+          off = row_next4(off);
+          w = row_next4(w);
+        }
+      }
+    }
+  }
+#endif
+  const int x0 = (t % A.ntx) * kTileSide, y0 = (t / A.ntx) * kTileSide;
+#pragma unroll
+  for (int c = 0; c < kTileCpw; ++c) {
+    const int cc = wave * kTileCpw + c;
+    const int cx = x0 + cc % kTileSide, cy = y0 + cc / kTileSide;
+    if (cx >= d.nx || cy >= d.ny) continue;
+    const int col = cy * d.nx + cx;
+#pragma unroll
+    for (int q = 0; q < NSLOT; ++q) {
+      const int z = lane + kWave * q;
+      if (z >= d.nzp) continue;
+      const int64_t idx = static_cast<int64_t>(col) * d.nzp + z;
+      if constexpr (MODE == BP_PLAIN) {
+        as_global(img)[idx] = z < d.nz ? acc[c][q] : 0.F;
+      } else {
+        if (z < d.nz) {
+          const float u = osem_factor(acc[c][q], as_const(data.sens)[idx], data.threshold, data.thr_lo, data.thr_hi);
+          as_global(data.estimate)[idx] = as_global(data.estimate)[idx] * u;
+          if (data.update) as_global(data.update)[idx] = u;
+        }
+      }
+    }
+  }
+}
+
+unsigned grid_of(int64_t n) {
+  int64_t b = (n + 255) / 256;
+  if (b > 65536) b = 65536;
+  if (b < 1) b = 1;
+  return static_cast<unsigned>(b);
+}
+
+}  // namespace
+
+void launch_tile_range(const Family* d_fams, const int2* d_fam_pos, int nfam, const int2* d_pool, const ImageDims& dims,
+                       int ntx, int nviews, int2* d_rng, int* d_need, hipStream_t stream) {
+  if (nfam <= 0) return;
+  hipLaunchKernelGGL(tile_range_kernel, dim3(nfam), dim3(kWave), 0, stream, d_fams, d_fam_pos, nfam, d_pool, dims, ntx,
+                     nviews, d_rng, d_need);
+}
+
+void launch_tile_phases(const int4* d_units, const int32_t* d_unit_off, int nsub, int ntiles, int nunits, int ntang,
+                        int nviews, const int2* d_rng, int rows, uint32_t* d_slot, uint32_t* d_nphase, uint32_t* d_nrow,
+                        int* d_bad, hipStream_t stream) {
+  hipLaunchKernelGGL(tile_phase_kernel<false>, dim3((nsub * ntiles + 63) / 64), dim3(64), 0, stream, d_units, d_unit_off,
+                     nsub, ntiles, nunits, ntang, nviews, d_rng, rows, d_slot, d_nphase, d_nrow, nullptr, nullptr,
+                     nullptr, nullptr, d_bad);
+}
+
+void launch_tile_rows(const int4* d_units, const int32_t* d_unit_off, int nsub, int ntiles, int nunits, int ntang,
+                      int nviews, const int2* d_rng, int rows, const uint32_t* d_phase_off, const uint32_t* d_row_off,
+                      uint32_t* d_row, uint32_t* d_phase_row, int* d_bad, hipStream_t stream) {
+  hipLaunchKernelGGL(tile_phase_kernel<true>, dim3((nsub * ntiles + 63) / 64), dim3(64), 0, stream, d_units, d_unit_off,
+                     nsub, ntiles, nunits, ntang, nviews, d_rng, rows, nullptr, nullptr, nullptr, d_phase_off, d_row_off,
+                     d_row, d_phase_row, d_bad);
+}
+
+void launch_tile_count(const Family* d_fams, const int2* d_fam_pos, int fam_begin, int fam_end, int ntang,
+                       const int2* d_pool, int subset, const ImageDims& dims, const TileArgs& A, int nunits,
+                       const uint32_t* d_slot, uint32_t* d_counts, hipStream_t stream) {
+  if (fam_end <= fam_begin) return;
+  hipLaunchKernelGGL(tile_entries_kernel<true>, dim3(fam_end - fam_begin), dim3(kWave), 0, stream, d_fams, d_fam_pos,
+                     fam_begin, fam_end, ntang, d_pool, subset, dims, A, nunits, d_slot, d_counts, 0U, nullptr, nullptr,
+                     nullptr);
+}
+
+void launch_tile_make(const Family* d_fams, const int2* d_fam_pos, int fam_begin, int fam_end, int ntang,
+                      const int2* d_pool, int subset, const ImageDims& dims, const TileArgs& A, int nunits,
+                      const uint32_t* d_slot, uint32_t none, const int64_t* d_fam_entry_off, uint32_t* d_keys,
+                      int2* d_raw, hipStream_t stream) {
+  if (fam_end <= fam_begin) return;
+  hipLaunchKernelGGL(tile_entries_kernel<false>, dim3(fam_end - fam_begin), dim3(kWave), 0, stream, d_fams, d_fam_pos,
+                     fam_begin, fam_end, ntang, d_pool, subset, dims, A, nunits, d_slot, nullptr, none, d_fam_entry_off,
+                     d_keys, d_raw);
+}
+
+void launch_tile_groups(const uint32_t* d_counts, int64_t n, uint32_t* d_groups, int* d_bad, hipStream_t stream) {
+  hipLaunchKernelGGL(tile_groups_kernel, dim3(grid_of(n)), dim3(256), 0, stream, d_counts, n, d_groups, d_bad);
+}
+
+void launch_tile_headers(const uint32_t* d_groups, const uint32_t* d_group_off, const uint32_t* d_phase_row,
+                         uint32_t total_rows, int64_t nphase, uint4* d_hdr, hipStream_t stream) {
+  const int64_t n = (nphase + kTileHdrSlack) * kTileWaves;
+  hipLaunchKernelGGL(tile_headers_kernel, dim3(grid_of(n)), dim3(256), 0, stream, d_groups, d_group_off, d_phase_row,
+                     total_rows, nphase, int64_t{kTileHdrSlack}, d_hdr);
+}
+
+void launch_tile_work(const uint32_t* d_group_off, const uint32_t* d_phase_off, int nsub, int ntiles, uint32_t* d_work,
+                      hipStream_t stream) {
+  hipLaunchKernelGGL(tile_work_kernel, dim3((ntiles + 255) / 256), dim3(256), 0, stream, d_group_off, d_phase_off, nsub,
+                     ntiles, d_work);
+}
+
+void launch_tile_place(const uint32_t* d_keys, const uint32_t* d_idx, const int2* d_raw, const uint32_t* d_list_start,
+                       const uint32_t* d_group_off, int64_t n, int32_t* d_off, float* d_w, hipStream_t stream) {
+  if (n <= 0) return;
+  hipLaunchKernelGGL(tile_place_kernel, dim3(grid_of(n)), dim3(256), 0, stream, d_keys, d_idx, d_raw, d_list_start,
+                     d_group_off, n, d_off, d_w);
+}
+
+void launch_back_project_tile(BpMode mode, const TileArgs& A, int subset_begin, int subset_end, const float* d_proj,
+                              float* d_img, const ImageDims& dims, const BpData& data, hipStream_t stream) {
+  const int nslot = (dims.nz + kWave - 1) / kWave;
+  const int chunk = kTileXcdChunk, round = kNumXcd * chunk;
+  const dim3 grid((A.ntiles + round - 1) / round * round), block(kWave * kTileWaves);
+  const size_t lds = static_cast<size_t>(A.lds_floats) * sizeof(float);
+#define MI_TILE(M, S)                                                                                                 \
+  hipLaunchKernelGGL((bp_tile_kernel<M, S>), grid, block, lds, stream, A, subset_begin, subset_end, d_proj, d_img, dims, \
+                     data, chunk)
+#define MI_TILE_S(M)             \
+  switch (nslot) {               \
+    case 1: MI_TILE(M, 1); break; \
+    case 2: MI_TILE(M, 2); break; \
+    case 3: MI_TILE(M, 3); break; \
+    default: MI_TILE(M, 4); break; \
+  }
+  if (mode == BP_PLAIN) { MI_TILE_S(BP_PLAIN) }
+  else { MI_TILE_S(BP_OSEM_UPDATE) }
+#undef MI_TILE_S
+#undef MI_TILE
+}
+
+// LDS above 64 KB per workgroup needs the kernels' dynamic limit raised on
+// every device they run on
+hipError_t tile_allow_lds(int bytes) {
+  const void* k[] = {reinterpret_cast<const void*>(&bp_tile_kernel<BP_PLAIN, 1>),
+                     reinterpret_cast<const void*>(&bp_tile_kernel<BP_PLAIN, 2>),
+                     reinterpret_cast<const void*>(&bp_tile_kernel<BP_PLAIN, 3>),
+                     reinterpret_cast<const void*>(&bp_tile_kernel<BP_PLAIN, 4>),
+                     reinterpret_cast<const void*>(&bp_tile_kernel<BP_OSEM_UPDATE, 1>),
+                     reinterpret_cast<const void*>(&bp_tile_kernel<BP_OSEM_UPDATE, 2>),
+                     reinterpret_cast<const void*>(&bp_tile_kernel<BP_OSEM_UPDATE, 3>),
+                     reinterpret_cast<const void*>(&bp_tile_kernel<BP_OSEM_UPDATE, 4>)};
+  for (const void* f : k) {
+    const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
+}  // namespace mi
