@@ -29,7 +29,11 @@ void launch_fill_int2(int2* d, int64_t n, int2 v, hipStream_t stream);
 
 namespace {
 
-constexpr int kRowSlack = 16;  // elements after the row copies: the forward kernel reads a group ahead
+// Mean axial positions per family up to which the forward projection runs row
+// groups (milliseconds, row groups against tasks): 8 rings, mean 7: 0.083 / 0.358;
+// 16 rings, span 1, mean 8: 0.47 / 1.23; 24 rings, span 3, mean 24: 0.50 / 0.59;
+// 32 rings, span 7, mean 38: 0.60 / 0.52; 40 rings, span 9, mean 47: 0.77 / 0.62.
+constexpr int kRowsMeanAxial = 28;
 
 thread_local std::string g_last_error;
 
@@ -108,6 +112,13 @@ struct mi_ctx {
   std::vector<int> task_group;                          // forward task -> group
   std::vector<std::vector<int>> subset_groups;          // subset of the table -> its groups, ascending
   std::vector<mi::FpTask> h_tasks;
+  // forward projection by row groups (pmrt_rows.hip), for short families
+  bool use_rows = false;
+  std::vector<int> item_off;  // per subset, size nsub+1
+  DBuf<mi::RowGroup> row_groups;
+  DBuf<int32_t> row_fams;
+  DBuf<int2> row_items;
+  void build_row_groups();
   DBuf<mi::FpTask> sel_tasks;  // forward tasks of a view-segment request
   bool have_image = false;     // ctx->img holds the image of mi_set_image
   DBuf<int64_t> list_off;
@@ -301,7 +312,21 @@ struct mi_ctx {
   // ---- projections on device-layout buffers
   void fp(mi::FpMode mode, const float* d_img, float* d_out, int subset, const mi::FpData& data, hipStream_t st) {
     const int tb = task_off[subset_begin(subset)], te = task_off[subset_end(subset)];
-    fp_tasks(mode, tasks.p + tb, te - tb, d_img, d_out, data, st);
+    if (!use_rows) {
+      fp_tasks(mode, tasks.p + tb, te - tb, d_img, d_out, data, st);
+      return;
+    }
+    hipEvent_t e0 = nullptr, e1 = nullptr;
+    if (timing) { e0 = take_event(); e1 = take_event(); HIPCHECK(hipEventRecord(e0, st)); }
+    const int ib = item_off[subset_begin(subset)], ie = item_off[subset_end(subset)];
+    mi::launch_forward_project_rows(mode, row_items.p + ib, ie - ib, row_groups.p, row_fams.p, fams.p, pool.p, d_img,
+                                    d_out, dims, data, st);
+    if (timing) { HIPCHECK(hipEventRecord(e1, st)); fp_events.emplace_back(e0, e1); }
+  }
+  // log-likelihood partial sums that fp() of a subset writes
+  int num_partials(int subset) const {
+    const std::vector<int>& off = use_rows ? item_off : task_off;
+    return off[subset_end(subset)] - off[subset_begin(subset)];
   }
   void fp_tasks(mi::FpMode mode, const mi::FpTask* d_tasks, int ntasks, const float* d_img, float* d_out,
                 const mi::FpData& data, hipStream_t st) {
@@ -540,7 +565,8 @@ void mi_ctx::build_rows() {
   sk.release();
   sw.release();
   if (total >= (int64_t(1) << 31)) throw ApiError(MI_ERR_ARGUMENT, "more than 2^31 basic-row elements");
-  pool.alloc(std::max<int64_t>(total, 1));
+  pool.alloc(total + mi::kRowSlack);
+  HIPCHECK(hipMemsetAsync(pool.p + total, 0, mi::kRowSlack * sizeof(int2), stream));
   for (auto& ch : chunks)
     if (ch.size > 0)
       HIPCHECK(hipMemcpyAsync(pool.p + ch.global_start, ch.data->p, ch.size * sizeof(int2), hipMemcpyDeviceToDevice, stream));
@@ -550,8 +576,8 @@ void mi_ctx::build_rows() {
   pool_ops.release();
   if (ntof == 1 && total > 0) {
     // 8 copies, then slack for the forward kernel's read-ahead of one element group
-    pool_ops.alloc(8 * total + kRowSlack);
-    HIPCHECK(hipMemsetAsync(pool_ops.p + 8 * total, 0, kRowSlack * sizeof(int2), stream));
+    pool_ops.alloc(8 * total + mi::kRowSlack);
+    HIPCHECK(hipMemsetAsync(pool_ops.p + 8 * total, 0, mi::kRowSlack * sizeof(int2), stream));
     mi::launch_expand_rows(pool.p, total, dims, pool_ops.p, stream);
     HIPCHECK(hipGetLastError());
   }
@@ -659,10 +685,68 @@ void mi_ctx::build_tasks() {
     v.erase(std::unique(v.begin(), v.end()), v.end());
   }
   h_tasks = h;
+  build_row_groups();
   tasks.alloc(h.size());
   HIPCHECK(hipMemcpyAsync(tasks.p, h.data(), h.size() * sizeof(mi::FpTask), hipMemcpyHostToDevice, stream));
-  partial.alloc(std::max<size_t>(h.size(), 1));
+  partial.alloc(std::max<size_t>({h.size(), row_items.n, 1}));
   HIPCHECK(hipStreamSynchronize(stream));
+}
+
+// Row groups (pmrt_rows.hip) where the families are short (kRowsMeanAxial).
+void mi_ctx::build_row_groups() {
+  use_rows = false;
+  item_off.clear();
+  row_groups.release();
+  row_fams.release();
+  row_items.release();
+  // (the image is read as one buffer of less than 2^31 bytes)
+  if (ntof > 1 || h_fams.empty() || static_cast<int64_t>(dims.ncols) * dims.nzp >= (int64_t{1} << 28)) return;
+  int64_t bins = 0;
+  for (const mi::Family& f : h_fams) bins += f.nax;
+  if (bins > int64_t{kRowsMeanAxial} * static_cast<int64_t>(h_fams.size())) return;
+  const int nsub = plan->num_subsets();
+  std::vector<mi::RowGroup> groups;
+  std::vector<int32_t> list;
+  std::vector<int2> items;
+  item_off.assign(nsub + 1, 0);
+  std::vector<int> order;
+  for (int s = 0; s < nsub; ++s) {
+    item_off[s] = static_cast<int>(items.size());
+    // the subset's families by basic row (an empty row starts where the next
+    // row does); a row's families are one segment or +-pair: one length
+    order.clear();
+    for (int f = plan->subset_family_begin(s); f < plan->subset_family_begin(s + 1); ++f) order.push_back(f);
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
+      const mi::Family &A = h_fams[a], &B = h_fams[b];
+      if (A.row_start != B.row_start) return A.row_start < B.row_start;
+      if (A.row_len != B.row_len) return A.row_len < B.row_len;
+      return A.nax < B.nax;
+    });
+    for (size_t i = 0; i < order.size();) {
+      const mi::Family& F = h_fams[order[i]];
+      mi::RowGroup G{F.row_start, F.row_len, static_cast<int32_t>(list.size()), 0, F.nax, 0, {0, 0}};
+      for (; i < order.size(); ++i) {
+        const mi::Family& f = h_fams[order[i]];
+        if (f.row_start != F.row_start || f.row_len != F.row_len || f.nax != F.nax) break;
+        list.push_back(order[i]);
+        ++G.nfam;
+      }
+      for (int b = 0; b < G.nfam * G.nax; b += 64) items.push_back(make_int2(static_cast<int>(groups.size()), b));
+      groups.push_back(G);
+    }
+  }
+  item_off[nsub] = static_cast<int>(items.size());
+  auto upload = [&](auto& buf, const auto& v) {
+    buf.alloc(v.size());
+    HIPCHECK(hipMemcpyAsync(buf.p, v.data(), buf.bytes(), hipMemcpyHostToDevice, stream));
+  };
+  upload(row_groups, groups);
+  upload(row_fams, list);
+  upload(row_items, items);
+  mi::launch_row_group_reach(row_groups.p, static_cast<int>(groups.size()), row_fams.p, fams.p, pool.p, dims, stream);
+  HIPCHECK(hipGetLastError());
+  HIPCHECK(hipStreamSynchronize(stream));
+  use_rows = true;
 }
 
 void mi_ctx::build_table() {
@@ -2024,9 +2108,8 @@ int mi_obj_log_likelihood(mi_ctx* ctx, int subset, double* value) {
     ctx->check_subset(subset);
     if (!ctx->have_data || !ctx->have_x) throw ApiError(MI_ERR_STATE, "data and estimate must be set first");
     HIPCHECK(hipSetDevice(ctx->device));
-    const int tb = ctx->task_off[ctx->subset_begin(subset)], te = ctx->task_off[ctx->subset_end(subset)];
     ctx->fp(ctx->lm ? mi::FP_LM_VALUE : mi::FP_LOGLIK, ctx->x.p, ctx->ratio.p, subset, ctx->fp_data(), ctx->stream);
-    std::vector<double> h(te - tb);
+    std::vector<double> h(ctx->num_partials(subset));
     HIPCHECK(hipMemcpyAsync(h.data(), ctx->partial.p, h.size() * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
     HIPCHECK(hipStreamSynchronize(ctx->stream));
     double acc = 0;
@@ -2052,10 +2135,7 @@ int mi_obj_value_and_gradient_dev(mi_ctx* ctx, const float* d_image, int subset,
     else if (!d_value) mode = add_sensitivity ? mi::FP_RATIO : mi::FP_GRADIENT;
     else mode = add_sensitivity ? mi::FP_RATIO_LOGLIK : mi::FP_GRADIENT_LOGLIK;
     ctx->fp(mode, ctx->img.p, ctx->ratio.p, subset, ctx->fp_data(), st);
-    if (d_value) {
-      const int tb = ctx->task_off[ctx->subset_begin(subset)], te = ctx->task_off[ctx->subset_end(subset)];
-      mi::launch_sum_partials(ctx->partial.p, te - tb, 1.0, d_value, st);
-    }
+    if (d_value) mi::launch_sum_partials(ctx->partial.p, ctx->num_partials(subset), 1.0, d_value, st);
     if (d_gradient) {
       ctx->bp(mi::BP_PLAIN, ctx->ratio.p, ctx->img2.p, subset, mi::BpData{}, st);
       ctx->image_from_device(ctx->img2.p, d_gradient, st);

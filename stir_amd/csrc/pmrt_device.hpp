@@ -124,6 +124,26 @@ void launch_forward_project(FpMode mode, const FpTask* d_tasks, int ntasks, cons
 // copies of the basic rows per in-plane operation for launch_forward_project
 // (d_ops: 8 * n elements)
 void launch_expand_rows(const int2* d_pool, int64_t n, const ImageDims& dims, int2* d_ops, hipStream_t stream);
+// ---- forward projection by row groups (pmrt_rows.hip): the non-TOF families
+// that share one basic row, `nax` axial positions each
+constexpr int kRowSlack = 16;      // elements after the last row (read-ahead of the forward row loops)
+constexpr int kRowsXcdChunk = 16;  // workgroups of one XCD's turn
+struct RowGroup {
+  int32_t row_start, row_len;
+  int32_t first, nfam;  // fam_list[first .. first + nfam)
+  int32_t nax;
+  int32_t inside;  // no element reaches past the zeros that pad the image columns
+  int32_t pad[2];
+};
+static_assert(sizeof(RowGroup) == 32, "RowGroup layout");
+void launch_row_group_reach(RowGroup* d_groups, int ngroups, const int32_t* d_fam_list, const Family* d_fams,
+                            const int2* d_pool, const ImageDims& dims, hipStream_t stream);
+// items: (group, first bin of the group), 64 bins each
+void launch_forward_project_rows(FpMode mode, const int2* d_items, int nitems, const RowGroup* d_groups,
+                                 const int32_t* d_fam_list, const Family* d_fams, const int2* d_pool,
+                                 const float* d_img, float* d_out, const ImageDims& dims, const FpData& data,
+                                 hipStream_t stream);
+
 // Launch shape of the back projection: image columns are visited in
 // tile_x x tile_y tiles (1 x 1 = raster order), optionally remapped so each XCD
 // gets a contiguous range of tiles, optionally skipping z slots an entry cannot reach.

@@ -29,7 +29,6 @@ namespace {
 using namespace dev;
 
 constexpr int kUnroll = 8;      // matrix elements whose gathers are in flight together
-constexpr int kRowSlack = 16;   // elements after the last row copy (read-ahead of the forward row loop)
 
 // Sum of img * w over one row in row order for every bin of the lane
 // (ProjMatrixElemsForOneBin.cxx:354-371), from the row's copy for the family's
