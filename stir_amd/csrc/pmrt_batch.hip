@@ -155,7 +155,7 @@ __global__ void __launch_bounds__(kWave* kWavesPerBlock) bp_group_kernel(const P
     }
 #pragma unroll
     for (int j = 0; j < kGroupUnroll; ++j)
-      if (ok[j]) acc = acc + w[j] * p[j];
+      if (ok[j]) acc = __builtin_fmaf(w[j], p[j], acc);
   }
   if (!item || zl >= d.nzp) return;
   const int64_t idx = static_cast<int64_t>(W.index) * d.nzp + zl;

@@ -17,7 +17,7 @@
 // come last (and whose relative z is the largest unsigned value). Each column
 // therefore sums exactly its column-table entries in column-table order: the
 // block back projection equals the column back projection bit for bit. A
-// merged entry in which a column has no element adds mul_legacy(0, p) = +0.
+// merged entry in which a column has no element adds fma(0, 0, x) = x.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -31,9 +31,9 @@ namespace {
 
 using namespace dev;
 
-// a * b, except that a zero operand gives +0 whatever the other one is
-// (v_mul_legacy_f32)
-__device__ float mul_legacy(float a, float b) __asm("llvm.amdgcn.fmul.legacy");
+// acc + w * p in one rounding; a zero (wave-uniform) weight adds nothing
+// whatever p is
+__device__ inline float add_term(float w, float p, float acc) { return __builtin_fmaf(w, w != 0.F ? p : 0.F, acc); }
 
 __device__ inline int basic_z(int c) { return static_cast<int>(static_cast<unsigned>(c) >> 20) - 2048; }
 
@@ -192,7 +192,7 @@ __global__ void __launch_bounds__(kWave* kWavesPerBlock) bp_quad_kernel(const in
 #pragma unroll
         for (int c = 0; c < 4; ++c)
 #pragma unroll
-          for (int q = 0; q < NSLOT; ++q) acc[c][q] = acc[c][q] + mul_legacy(Es[j].w[c], p[j][q]);
+          for (int q = 0; q < NSLOT; ++q) acc[c][q] = add_term(Es[j].w[c], p[j][q], acc[c][q]);
     }
     for (; e < end; ++e) {
       const QuadEntry E = ent[e];
@@ -205,7 +205,7 @@ __global__ void __launch_bounds__(kWave* kWavesPerBlock) bp_quad_kernel(const in
 #pragma unroll
       for (int c = 0; c < 4; ++c)
 #pragma unroll
-        for (int q = 0; q < NSLOT; ++q) acc[c][q] = acc[c][q] + mul_legacy(E.w[c], p[q]);
+        for (int q = 0; q < NSLOT; ++q) acc[c][q] = add_term(E.w[c], p[q], acc[c][q]);
     }
   }
 #pragma unroll

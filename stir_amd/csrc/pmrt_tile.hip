@@ -36,9 +36,9 @@
 // Entries: per (phase, column) a list padded to groups of 4 with entries that
 // read the leading zeros with weight 0. Offsets and weights are two arrays;
 // each row of 16 lanes loads the same 16 consecutive entries and a group
-// takes its four by DPP broadcast inside the add and the multiply, so an entry
-// costs one address add, one two-slot LDS read, and a multiply and an add per
-// slot: 5 vector instructions for 128 planes, no scalar ones.
+// takes its four by DPP broadcast inside the add and the multiply-add, so an
+// entry costs one address add, one two-slot LDS read and a multiply-add per
+// slot: 3 vector instructions for 128 planes, no scalar ones.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -264,22 +264,21 @@ __device__ inline int row_bcast(int v) {
 // lane (i + 4) % 16 of the row of 16 lanes
 __device__ inline int row_next4(int v) { return __builtin_amdgcn_update_dpp(0, v, 0x120 + 12, 0xf, 0xf, true); }
 
-// p times lane J's w of the row. The multiply takes the broadcast itself (the
-// compiler moves it to a register first when two slots share the weight). A
-// DPP read needs two wait states after a VALU write of w, which the compiler
-// does not count across asm: the first multiply of a group brings them.
+// acc + lane J's w of the row times p, in one rounding; the instruction takes
+// the broadcast itself (the compiler moves it to a register first when two
+// slots share the weight). A DPP read needs two wait states after a VALU write
+// of w, which the compiler does not count across asm: the first of a group
+// brings them.
 template <int J>
-__device__ inline float mul_bcast(int w, float p) {
-  float r;
+__device__ inline void add_bcast(float& acc, int w, float p) {
   if constexpr (J == 0)
-    asm("s_nop 1\n\tv_mul_f32_dpp %0, %1, %2 row_newbcast:0 row_mask:0xf bank_mask:0xf" : "=v"(r) : "v"(w), "v"(p));
+    asm("s_nop 1\n\tv_fmac_f32_dpp %0, %1, %2 row_newbcast:0 row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(w), "v"(p));
   else if constexpr (J == 1)
-    asm("v_mul_f32_dpp %0, %1, %2 row_newbcast:1 row_mask:0xf bank_mask:0xf" : "=v"(r) : "v"(w), "v"(p));
+    asm("v_fmac_f32_dpp %0, %1, %2 row_newbcast:1 row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(w), "v"(p));
   else if constexpr (J == 2)
-    asm("v_mul_f32_dpp %0, %1, %2 row_newbcast:2 row_mask:0xf bank_mask:0xf" : "=v"(r) : "v"(w), "v"(p));
+    asm("v_fmac_f32_dpp %0, %1, %2 row_newbcast:2 row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(w), "v"(p));
   else
-    asm("v_mul_f32_dpp %0, %1, %2 row_newbcast:3 row_mask:0xf bank_mask:0xf" : "=v"(r) : "v"(w), "v"(p));
-  return r;
+    asm("v_fmac_f32_dpp %0, %1, %2 row_newbcast:3 row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(w), "v"(p));
 }
 
 // an ordered (not invariant) load: it stays behind the copy of the registers it overwrites
@@ -297,13 +296,13 @@ __device__ inline void tile_group(int off, int w, const char* lds, int lane4, fl
 #pragma unroll
     for (int q = 0; q < NSLOT; ++q) v[j][q] = *reinterpret_cast<const float*>(lds + (lane4 + o[j]) + 256 * q);
 #pragma unroll
-  for (int q = 0; q < NSLOT; ++q) acc[q] = acc[q] + mul_bcast<0>(w, v[0][q]);
+  for (int q = 0; q < NSLOT; ++q) add_bcast<0>(acc[q], w, v[0][q]);
 #pragma unroll
-  for (int q = 0; q < NSLOT; ++q) acc[q] = acc[q] + mul_bcast<1>(w, v[1][q]);
+  for (int q = 0; q < NSLOT; ++q) add_bcast<1>(acc[q], w, v[1][q]);
 #pragma unroll
-  for (int q = 0; q < NSLOT; ++q) acc[q] = acc[q] + mul_bcast<2>(w, v[2][q]);
+  for (int q = 0; q < NSLOT; ++q) add_bcast<2>(acc[q], w, v[2][q]);
 #pragma unroll
-  for (int q = 0; q < NSLOT; ++q) acc[q] = acc[q] + mul_bcast<3>(w, v[3][q]);
+  for (int q = 0; q < NSLOT; ++q) add_bcast<3>(acc[q], w, v[3][q]);
 }
 
 template <int MODE, int NSLOT>
