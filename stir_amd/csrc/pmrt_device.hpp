@@ -334,10 +334,10 @@ void launch_back_project_slab(BpMode mode, const SlabArgs& A, int subset_begin, 
 // ---- back projection by image tiles with the runs in LDS (pmrt_tile.hip):
 // non-TOF tables whose families cover whole runs (z-shift symmetry)
 constexpr int kTileSide = 8;          // a tile is 8 x 8 image columns
-constexpr int kTileLdsBytes = 80640;  // LDS of a workgroup: two share the CU's 160 KB
+constexpr int kTileLdsBytes = 53760;  // LDS of a workgroup: three share the CU's 160 KB
 constexpr int kTileXcdChunk = 1;      // tiles of one XCD's turn
 constexpr int kTileCols = kTileSide * kTileSide;
-constexpr int kTileWaves = 16;
+constexpr int kTileWaves = 8;
 constexpr int kTileHdrSlack = 3;   // phases that the kernel's header read-ahead may touch past the last
 constexpr int kTileEntSlack = 64;  // entries that its chunk read-ahead may touch past the last
 constexpr int kTileRowSlack = 64 * kTileWaves;  // rows that its read-ahead may touch past the last

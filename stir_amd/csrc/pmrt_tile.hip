@@ -10,20 +10,19 @@
 // there (each staged run is used by about nine entries at mMR size).
 //
 // Measured at mMR size (4.2e8 entries, 837 x 252 x 344 bins, 344 x 344 x 127
-// voxels): 10.8 ms with the column kernel, 6.4 ms with this one, which then
-// issues vector instructions in 76 % of the cycles (2.8e9 of them, 2.55e9 in
-// the entry loop), reads LDS in 47 % and fetches 17 GB from beyond L2. With
-// the copies left out it takes 4.8 ms, with the entries left out 2.4 ms: the
-// two overlap only in part. Half the waves per workgroup: 7.2 ms; three
-// workgroups of 8 waves and 53 KB per CU: 6.3 ms, four of 40 KB: 6.8 ms
-// (shorter lists, more padding).
+// voxels): 10.8 ms with the column kernel, 5.74 ms with this one: three
+// workgroups of 8 waves and 53 KB of LDS per CU. Two of 16 waves and 80 KB:
+// 6.15 ms (5.97 with the reads of a group kept together); of 8 waves and
+// 80 KB: 6.7; four of 8 waves and 40 KB: 6.3 (shorter lists, more padding);
+// tiles of 12 x 8 columns: 5.75, of 16 x 8: 6.2. With the copies left out it
+// takes 4.1 ms, without copies and barriers 3.6 (the LDS reads alone 3.2).
 //
 // Work: phases. The (segment, view) viewgrams of a subset are taken in family
 // order; consecutive ones form a phase as long as the tangential positions
 // that cross the tile fill no more than `rows` LDS rows. Per phase the
 // workgroup copies the rows (loads that write LDS directly, all in flight at
-// once), then every wave walks its columns' entries. Two workgroups share a
-// CU, so one computes while the other waits for its rows.
+// once), then every wave walks its columns' entries. Three workgroups share a
+// CU, so two compute while one waits for its rows.
 //
 // LDS rows: `stride` floats per run, the run spread to one value per image
 // plane (ppa planes per axial position: zeros between) and followed by zeros.
@@ -295,6 +294,7 @@ __device__ inline void tile_group(int off, int w, const char* lds, int lane4, fl
   for (int j = 0; j < 4; ++j)
 #pragma unroll
     for (int q = 0; q < NSLOT; ++q) v[j][q] = *reinterpret_cast<const float*>(lds + (lane4 + o[j]) + 256 * q);
+  __builtin_amdgcn_sched_barrier(0);  // all reads of the group in flight before the first is waited for
 #pragma unroll
   for (int q = 0; q < NSLOT; ++q) add_bcast<0>(acc[q], w, v[0][q]);
 #pragma unroll
