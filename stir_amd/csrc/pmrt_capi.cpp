@@ -154,16 +154,16 @@ struct mi_ctx {
   // default where build_tile_table accepts the geometry
   bool use_tile = false;
   int64_t tile_entries = 0;
-  DBuf<uint32_t> tile_phase_off, tile_row;
+  DBuf<uint32_t> tile_phase_off;
   DBuf<uint4> tile_hdr;
   DBuf<int32_t> tile_off, tile_order;
   DBuf<float> tile_w;
-  DBuf<int2> tile_rng, tile_segs;
+  DBuf<int2> tile_rng, tile_row;
   mi::TileArgs tile{};
   void release_tile() {
     use_tile = false;
     tile_entries = 0;
-    tile_phase_off.release(); tile_hdr.release(); tile_row.release(); tile_segs.release(); tile_off.release(); tile_order.release();
+    tile_phase_off.release(); tile_hdr.release(); tile_row.release(); tile_off.release(); tile_order.release();
     tile_w.release(); tile_rng.release();
     tile = mi::TileArgs{};
   }
@@ -171,7 +171,7 @@ struct mi_ctx {
     return static_cast<int64_t>(tile_phase_off.bytes() + tile_hdr.bytes() + tile_row.bytes() + tile_off.bytes() +
                                 tile_order.bytes() + tile_w.bytes());
   }
-  bool build_tile_table();
+  bool build_tile_table(int span);
   std::vector<mi::Family> h_fams;
   std::unordered_map<int64_t, int> fam_lookup;  // (seg,view,tang,a0) -> family
   int64_t num_basic_elements = 0;
@@ -387,7 +387,10 @@ struct mi_ctx {
           bool nontof = false) {
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (timing) { e0 = take_event(); e1 = take_event(); HIPCHECK(hipEventRecord(e0, st)); }
-    if (ntof > 1 && !nontof && tof_bp_w > 0)
+    if (ntof > 1 && !nontof && use_tile)
+      mi::launch_back_project_tile(mode, tile, subset_begin(subset), subset_end(subset), d_proj, d_img, dims, data,
+                                   st);
+    else if (ntof > 1 && !nontof && tof_bp_rec.n)
       mi::launch_back_project_tof_rows(mode, uniform_ppa, list_off.p, tof_bp_rec.p, tof_bp_w,
                                        static_cast<int64_t>(tof_bp_rec.n / mi::tof_bp_words(tof_bp_w)) - 1,
                                        subset_begin(subset), subset_end(subset), d_proj, d_img, dims, tofc, data,
@@ -398,7 +401,7 @@ struct mi_ctx {
     else if (use_slab)
       mi::launch_back_project_slab(mode, slab, subset_begin(subset), subset_end(subset), d_proj, d_img, dims, data,
                                    st);
-    else if (use_tile)
+    else if (use_tile && ntof == 1)
       mi::launch_back_project_tile(mode, tile, subset_begin(subset), subset_end(subset), d_proj, d_img, dims, data,
                                    st);
     else if (use_quad())
@@ -424,7 +427,9 @@ struct mi_ctx {
                   int64_t(sizeof(mi::FpTask)) + int64_t(sizeof(mi::Family)) * (t.second >= 0 ? 2 : 1) +
                   (ntof > 1 && !fp_rec ? int64_t(sizeof(mi::FamilyLor)) : 0);
     }
-    if (ntof > 1 && tof_bp_w > 0)
+    if (ntof > 1 && use_tile)
+      bp_bytes = img_bytes + proj_bytes + tile_bytes();
+    else if (ntof > 1 && tof_bp_rec.n)
       bp_bytes = img_bytes + proj_bytes + static_cast<int64_t>(tof_bp_rec.bytes() + list_off.bytes());
     else if (use_quad())
       bp_bytes = img_bytes + proj_bytes + static_cast<int64_t>(quad_ent.bytes() + quad_off.bytes());
@@ -757,11 +762,13 @@ void mi_ctx::build_table() {
   }
   release_slab();
   release_tile();
-  if (build_tile_table()) {
-    use_tile = true;
-    return;
+  if (ntof == 1) {
+    if (build_tile_table(1)) {
+      use_tile = true;
+      return;
+    }
+    release_tile();
   }
-  release_tile();
   const int nsub = plan->num_subsets();
   const int ncols = dims.ncols;
   // entry offsets per family (family order == subset order)
@@ -946,14 +953,23 @@ void mi_ctx::build_tof_rows(int64_t n) {
   tof_fp_rec.alloc(pool_end * mi::tof_fp_words(fw));
   mi::launch_tof_fp_records(fams.p, static_cast<int>(h_fams.size()), lors.p, pool.p, dims, tofc, fnt, fw,
                             tof_fp_rec.p, stream);
+  tof_fp_nt = fnt;
+  tof_fp_w = fw;
+  tof_bp_w = bw;
+  // the back projection by image tiles instead of back records (narrow windows
+  // only: mode 2 keeps the records)
+  if (tof_rows_mode == 1 && build_tile_table(s)) {
+    use_tile = true;
+    HIPCHECK(hipStreamSynchronize(stream));
+    entry_d.release();
+    return;
+  }
+  release_tile();
   tof_bp_rec.alloc((n + 1) * mi::tof_bp_words(bw));  // + the all-zero record read past a list's end
   HIPCHECK(hipMemsetAsync(tof_bp_rec.p + n * mi::tof_bp_words(bw), 0, sizeof(int32_t) * mi::tof_bp_words(bw), stream));
   mi::launch_tof_bp_records(entries.p, entry_d.p, n, tofc, bw, tof_bp_rec.p, stream);
   HIPCHECK(hipGetLastError());
   HIPCHECK(hipStreamSynchronize(stream));
-  tof_fp_nt = fnt;
-  tof_fp_w = fw;
-  tof_bp_w = bw;
   entry_d.release();  // read only by the on-the-fly back projection
 }
 
@@ -1172,22 +1188,26 @@ bool mi_ctx::build_slab_table() {
   return true;
 }
 
-// The tile table (pmrt_tile.hip) of a non-TOF matrix whose families cover
-// whole runs; false where the geometry does not qualify (the column table is
-// built instead). Images of up to 32 planes stay with the column kernels,
-// which pack them better than a wave of 64 planes.
-bool mi_ctx::build_tile_table() {
+// The tile table (pmrt_tile.hip) of a matrix whose families cover whole runs;
+// false where the geometry does not qualify (the column kernels are used
+// then). TOF matrices: from the stored forward records, span the most TOF bins
+// of one element. Images of up to 32 planes stay with the column kernels, which
+// pack them better than a wave of 64 planes.
+bool mi_ctx::build_tile_table(int span) {
   const mi_geometry& g = plan->geometry();
-  if (!slab_allowed || slab_enable || quad_enable || ntof > 1 || dims.nz <= 32 || h_fams.empty()) return false;
+  if (!slab_allowed || slab_enable || quad_enable || dims.nz <= 32 || dims.nz > 256 || h_fams.empty()) return false;
+  if (total_bins() >= (int64_t{1} << 31) || (ntof > 1 && tof_fp_w <= 0)) return false;
+  const int32_t* rec = ntof > 1 ? tof_fp_rec.p : nullptr;
   const auto& keys = plan->family_keys();
   const int nsub = plan->num_subsets(), nfam = static_cast<int>(h_fams.size()), ntang = g.num_tangential_poss;
-  // units: the (segment, view) viewgrams, ntang consecutive families each
-  if (nfam % ntang || int64_t{g.num_views} * ntang >= (1 << 24) || plan->nseg() > 255) return false;
-  const int nunits = nfam / ntang;
+  // units: the (segment, view, TOF bin) viewgrams, ntang consecutive families
+  // per (segment, view)
+  if (nfam % ntang) return false;
+  const int nunits = nfam / ntang * ntof, nrng = g.num_views * ntof;
   std::vector<int4> hunits(nunits);
-  std::vector<int2> hpos(nfam), hsegs(256, make_int2(0, 1 << 16));
+  std::vector<int2> hpos(nfam);
   int longest = 0;
-  for (int u = 0; u < nunits; ++u) {
+  for (int u = 0; u < nfam / ntang; ++u) {
     const auto& k0 = keys[static_cast<size_t>(u) * ntang];
     const mi::Family& f0 = h_fams[static_cast<size_t>(u) * ntang];
     const int64_t seg_off = plan->segment_offset(k0.seg);
@@ -1200,20 +1220,38 @@ bool mi_ctx::build_tile_table() {
         return false;
       hpos[fi] = make_int2(k0.view, i);
     }
-    const int slot = k0.seg - g.min_segment_num, len = f0.ppa * (f0.nax - 1) + 1;
-    hsegs[slot] = make_int2(static_cast<int>(seg_off), f0.nax | f0.ppa << 16);
-    hunits[u] = make_int4(slot, len, 0, k0.view);
-    longest = std::max(longest, len);
+    for (int k = 0; k < ntof; ++k)
+      hunits[u * ntof + k] =
+          make_int4(static_cast<int>(f0.sino_base + k * block_bins), f0.nax, f0.ppa, k0.view * ntof + k);
+    longest = std::max(longest, f0.ppa * (f0.nax - 1) + 1);
   }
   const int nslot = (dims.nz + 63) / 64;
   if (longest > 64 * nslot) return false;
   std::vector<int32_t> hunit_off(nsub + 1);
   for (int s = 0; s <= nsub; ++s) {
     if (plan->subset_family_begin(s) % ntang) return false;
-    hunit_off[s] = plan->subset_family_begin(s) / ntang;
+    hunit_off[s] = plan->subset_family_begin(s) / ntang * ntof;
   }
+  // element offsets per family; the sort of one subset's terms at a time
+  std::vector<int64_t> fam_off(nfam + 1, 0);
+  for (int i = 0; i < nfam; ++i) fam_off[i + 1] = fam_off[i] + h_fams[i].row_len;
+  const int64_t n = fam_off.back();
+  if (n >= (int64_t{1} << 31)) throw ApiError(MI_ERR_ARGUMENT, "back-projection table above 2^31 entries");
+  int64_t most = 0;
+  for (int s = 0; s < nsub; ++s)
+    most = std::max(most, fam_off[plan->subset_family_begin(s + 1)] - fam_off[plan->subset_family_begin(s)]);
+  most *= span;
+  if (most <= 0 || most >= (int64_t{1} << 31)) return false;
   const int ntx = (dims.nx + mi::kTileSide - 1) / mi::kTileSide, nty = (dims.ny + mi::kTileSide - 1) / mi::kTileSide;
   const int ntiles = ntx * nty;
+  if (ntof > 1) {
+    // only where the terms (8 bytes each, padded lists), the rows and the sort's
+    // buffers fit beside everything else
+    size_t free_b = 0, total_b = 0;
+    HIPCHECK(hipMemGetInfo(&free_b, &total_b));
+    const int64_t bytes = 10 * n * span + 32 * most + 4 * (static_cast<int64_t>(ntiles) * nunits);
+    if (bytes > static_cast<int64_t>(free_b / 4 * 3)) return false;
+  }
   auto upload = [&](auto& buf, const auto& v) {
     buf.alloc(v.size());
     HIPCHECK(hipMemcpyAsync(buf.p, v.data(), buf.bytes(), hipMemcpyHostToDevice, stream));
@@ -1225,12 +1263,13 @@ bool mi_ctx::build_tile_table() {
   upload(d_pos, hpos);
   upload(d_unit_off, hunit_off);
   // pass 1: tangential ranges and the zeros a row needs
-  tile_rng.alloc(static_cast<size_t>(ntiles) * g.num_views);
+  tile_rng.alloc(static_cast<size_t>(ntiles) * nrng);
   mi::launch_fill_int2(tile_rng.p, static_cast<int64_t>(tile_rng.n), make_int2(0x7fffffff, -1), stream);
   DBuf<int> d_need;  // planes after a run's start, planes up to its end, flag
   d_need.alloc(3);
   HIPCHECK(hipMemsetAsync(d_need.p, 0, d_need.bytes(), stream));
-  mi::launch_tile_range(fams.p, d_pos.p, nfam, pool.p, dims, ntx, g.num_views, tile_rng.p, d_need.p, stream);
+  mi::launch_tile_range(fams.p, d_pos.p, nfam, pool.p, rec, tof_fp_w, dims, ntx, g.num_views, ntof, tile_rng.p, d_need.p,
+                        stream);
   HIPCHECK(hipGetLastError());
   int need[3];
   HIPCHECK(hipMemcpyAsync(need, d_need.p, sizeof(need), hipMemcpyDeviceToHost, stream));
@@ -1241,11 +1280,12 @@ bool mi_ctx::build_tile_table() {
   A.ntiles = ntiles;
   A.nsub = nsub;
   A.nviews = g.num_views;
+  A.tof = ntof > 1;
   A.stride = std::max({need[0], need[1], (longest + 63) / 64 * 64});  // rows are written 64 lanes at a time
   A.lead = std::max(A.stride, 64 * nslot);  // also the zeros that padding entries read
   A.longest = longest;
   const int rows = (mi::kTileLdsBytes / 4 - A.lead - 64 * nslot) / A.stride;
-  if (rows < 32) return false;
+  if (rows < 24) return false;
   A.lds_floats = mi::kTileLdsBytes / 4;
   // pass 2: phases
   const int64_t nst = static_cast<int64_t>(nsub) * ntiles;
@@ -1255,15 +1295,15 @@ bool mi_ctx::build_tile_table() {
   nrow.alloc(nst + 1);
   HIPCHECK(hipMemsetAsync(nphase.p + nst, 0, sizeof(uint32_t), stream));
   HIPCHECK(hipMemsetAsync(nrow.p + nst, 0, sizeof(uint32_t), stream));
-  mi::launch_tile_phases(d_units.p, d_unit_off.p, nsub, ntiles, nunits, ntang, g.num_views, tile_rng.p, rows, slot.p,
-                         nphase.p, nrow.p, d_need.p + 2, stream);
-  auto scan = [&](const DBuf<uint32_t>& in, DBuf<uint32_t>& out, int64_t n) {  // n counts, then the total
-    out.alloc(n);
+  mi::launch_tile_phases(d_units.p, d_unit_off.p, nsub, ntiles, nunits, nrng, tile_rng.p, rows, slot.p, nphase.p, nrow.p,
+                         d_need.p + 2, stream);
+  auto scan = [&](const DBuf<uint32_t>& in, DBuf<uint32_t>& out, int64_t count) {  // counts, then the total
+    out.alloc(count);
     size_t tb = 0;
-    HIPCHECK(mi::exclusive_scan_u32(nullptr, tb, in.p, out.p, static_cast<int>(n), stream));
+    HIPCHECK(mi::exclusive_scan_u32(nullptr, tb, in.p, out.p, static_cast<int>(count), stream));
     DBuf<char> tmp;
     tmp.alloc(std::max<size_t>(tb, 1));
-    HIPCHECK(mi::exclusive_scan_u32(tmp.p, tb, in.p, out.p, static_cast<int>(n), stream));
+    HIPCHECK(mi::exclusive_scan_u32(tmp.p, tb, in.p, out.p, static_cast<int>(count), stream));
     HIPCHECK(hipStreamSynchronize(stream));
   };
   scan(nphase, tile_phase_off, nst + 1);
@@ -1276,73 +1316,70 @@ bool mi_ctx::build_tile_table() {
   const uint32_t total_rows = totals[1];
   const int64_t nph = totals[0], nlists = nph * mi::kTileCols;
   if (nlists >= (int64_t{1} << 31) - 2) return false;
-  upload(tile_segs, hsegs);
   tile_row.alloc(static_cast<size_t>(total_rows) + mi::kTileRowSlack);
-  HIPCHECK(hipMemsetAsync(tile_row.p + total_rows, 0, mi::kTileRowSlack * sizeof(uint32_t), stream));
+  HIPCHECK(hipMemsetAsync(tile_row.p + total_rows, 0, mi::kTileRowSlack * sizeof(int2), stream));
   phase_row.alloc(nph);
-  mi::launch_tile_rows(d_units.p, d_unit_off.p, nsub, ntiles, nunits, ntang, g.num_views, tile_rng.p, rows,
-                       tile_phase_off.p, row_off.p, tile_row.p, phase_row.p, d_need.p + 2, stream);
+  mi::launch_tile_rows(d_units.p, d_unit_off.p, nsub, ntiles, nunits, nrng, tile_rng.p, rows, tile_phase_off.p,
+                       row_off.p, tile_row.p, phase_row.p, d_need.p + 2, stream);
   A.phase_off = tile_phase_off.p;
   A.row = tile_row.p;
-  A.segs = tile_segs.p;
   A.rng = tile_rng.p;
   // pass 3: entries per list, in groups of 4
-  DBuf<uint32_t> counts, groups, list_start, group_off;
+  DBuf<uint32_t> counts, groups, group_off;
   counts.alloc(nlists + 1);
   HIPCHECK(hipMemsetAsync(counts.p, 0, counts.bytes(), stream));
   for (int s = 0; s < nsub; ++s)
     mi::launch_tile_count(fams.p, d_pos.p, plan->subset_family_begin(s), plan->subset_family_begin(s + 1), ntang, pool.p,
-                          s, dims, A, nunits, slot.p, counts.p, stream);
+                          rec, tof_fp_w, ntof, s, dims, A, nunits, slot.p, counts.p, stream);
   groups.alloc(nlists + 1);
   mi::launch_tile_groups(counts.p, nlists + 1, groups.p, d_need.p + 2, stream);
   HIPCHECK(hipGetLastError());
-  scan(counts, list_start, nlists + 1);
   scan(groups, group_off, nlists + 1);
   counts.release();
-  HIPCHECK(hipMemcpy(&totals[0], list_start.p + nlists, sizeof(uint32_t), hipMemcpyDeviceToHost));
   HIPCHECK(hipMemcpy(&totals[1], group_off.p + nlists, sizeof(uint32_t), hipMemcpyDeviceToHost));
   HIPCHECK(hipMemcpy(need, d_need.p, sizeof(need), hipMemcpyDeviceToHost));
-  const int64_t nent = totals[0], nslots = 4 * static_cast<int64_t>(totals[1]);
+  const int64_t nslots = 4 * static_cast<int64_t>(totals[1]);
   if (need[2]) return false;
   tile_hdr.alloc((nph + mi::kTileHdrSlack) * mi::kTileWaves);
   mi::launch_tile_headers(groups.p, group_off.p, phase_row.p, total_rows, nph, tile_hdr.p, stream);
-  // pass 4: every element's list and entry, sorted by list, to its place
-  std::vector<int64_t> fam_off(nfam + 1, 0);
-  for (int i = 0; i < nfam; ++i) fam_off[i + 1] = fam_off[i] + h_fams[i].row_len;
-  const int64_t n = fam_off.back();
-  if (n >= (int64_t{1} << 31)) throw ApiError(MI_ERR_ARGUMENT, "back-projection table above 2^31 entries");
+  // pass 4, subset by subset: every term's list and entry, sorted by list, to
+  // its place
   DBuf<int64_t> d_fam_off;
   upload(d_fam_off, fam_off);
   tile_off.alloc(nslots + mi::kTileEntSlack);
   tile_w.alloc(nslots + mi::kTileEntSlack);
   HIPCHECK(hipMemsetAsync(tile_off.p, 0, tile_off.bytes(), stream));  // padding: weight 0 times the leading zeros
   HIPCHECK(hipMemsetAsync(tile_w.p, 0, tile_w.bytes(), stream));
-  DBuf<uint32_t> keys_in, keys_out, vals_in, vals_out;
-  DBuf<int2> raw;
-  keys_in.alloc(n);
-  raw.alloc(n);
-  for (int s = 0; s < nsub; ++s)
-    mi::launch_tile_make(fams.p, d_pos.p, plan->subset_family_begin(s), plan->subset_family_begin(s + 1), ntang, pool.p,
-                         s, dims, A, nunits, slot.p, static_cast<uint32_t>(nlists), d_fam_off.p, keys_in.p, raw.p,
-                         stream);
-  keys_out.alloc(n);
-  vals_in.alloc(n);
-  vals_out.alloc(n);
-  mi::launch_iota(vals_in.p, n, stream);
-  int end_bit = 1;
-  while ((int64_t{1} << end_bit) <= nlists) ++end_bit;
   {
-    size_t tb = 0;
-    HIPCHECK(mi::radix_sort_pairs(nullptr, tb, keys_in.p, keys_out.p, vals_in.p, vals_out.p, static_cast<int>(n), end_bit,
-                                  stream));
+    DBuf<uint32_t> keys_in, keys_out, vals_in, vals_out;
+    DBuf<int2> raw;
     DBuf<char> tmp;
+    keys_in.alloc(most);
+    keys_out.alloc(most);
+    vals_in.alloc(most);
+    vals_out.alloc(most);
+    raw.alloc(most);
+    mi::launch_iota(vals_in.p, most, stream);
+    const uint32_t none = static_cast<uint32_t>(nlists);
+    int end_bit = 1;
+    while ((int64_t{1} << end_bit) <= nlists) ++end_bit;
+    size_t tb = 0;
+    HIPCHECK(mi::radix_sort_pairs(nullptr, tb, keys_in.p, keys_out.p, vals_in.p, vals_out.p, static_cast<int>(most),
+                                  end_bit, stream));
     tmp.alloc(std::max<size_t>(tb, 1));
-    HIPCHECK(mi::radix_sort_pairs(tmp.p, tb, keys_in.p, keys_out.p, vals_in.p, vals_out.p, static_cast<int>(n), end_bit,
-                                  stream));
+    for (int s = 0; s < nsub; ++s) {
+      const int fb = plan->subset_family_begin(s), fe = plan->subset_family_begin(s + 1);
+      const int64_t m = (fam_off[fe] - fam_off[fb]) * span;
+      if (m <= 0) continue;
+      mi::launch_tile_make(fams.p, d_pos.p, fb, fe, ntang, pool.p, rec, tof_fp_w, ntof, s, dims, A, nunits, slot.p, none,
+                           span, d_fam_off.p, fam_off[fb], keys_in.p, raw.p, stream);
+      HIPCHECK(mi::radix_sort_pairs(tmp.p, tb, keys_in.p, keys_out.p, vals_in.p, vals_out.p, static_cast<int>(m), end_bit,
+                                    stream));
+      mi::launch_tile_place(keys_out.p, vals_out.p, raw.p, group_off.p, none, m, tile_off.p, tile_w.p, stream);
+    }
+    HIPCHECK(hipGetLastError());
     HIPCHECK(hipStreamSynchronize(stream));
   }
-  mi::launch_tile_place(keys_out.p, vals_out.p, raw.p, list_start.p, group_off.p, nent, tile_off.p, tile_w.p, stream);
-  HIPCHECK(hipGetLastError());
   // launch order: the tiles with the most entries first, so that the last
   // workgroups to run are short ones
   DBuf<uint32_t> d_work;
@@ -1356,7 +1393,6 @@ bool mi_ctx::build_tile_table() {
   std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return work[a] > work[b]; });
   upload(tile_order, order);
   HIPCHECK(hipStreamSynchronize(stream));
-  HIPCHECK(mi::tile_allow_lds(mi::kTileLdsBytes));
   A.hdr = tile_hdr.p;
   A.off = tile_off.p;
   A.w = tile_w.p;
@@ -1513,7 +1549,7 @@ int mi_get_info(mi_ctx* ctx, mi_info* out) {
     out->num_basic_elements = ctx->num_basic_elements;
     out->num_families = static_cast<int64_t>(ctx->h_fams.size());
     out->num_matrix_elements = ctx->num_matrix_elements;
-    out->num_table_entries = static_cast<int64_t>(ctx->use_slab ? ctx->slab_ent.n : ctx->use_tile ? ctx->tile_entries : ctx->entries.n);
+    out->num_table_entries = static_cast<int64_t>(ctx->use_slab ? ctx->slab_ent.n : ctx->use_tile && ctx->ntof == 1 ? static_cast<size_t>(ctx->tile_entries) : ctx->entries.n);
     out->num_nonzeros = ctx->num_nonzeros;
     out->device_bytes = static_cast<int64_t>(ctx->pool.bytes() + ctx->pool_ops.bytes() + ctx->fams.bytes() + ctx->tasks.bytes() +
                                              ctx->list_off.bytes() + ctx->entries.bytes() + ctx->img.bytes() +

@@ -332,52 +332,54 @@ void launch_back_project_slab(BpMode mode, const SlabArgs& A, int subset_begin, 
                               float* d_img, const ImageDims& dims, const BpData& data, hipStream_t stream);
 
 // ---- back projection by image tiles with the runs in LDS (pmrt_tile.hip):
-// non-TOF tables whose families cover whole runs (z-shift symmetry)
+// tables whose families cover whole runs (z-shift symmetry)
 constexpr int kTileSide = 8;          // a tile is 8 x 8 image columns
-constexpr int kTileLdsBytes = 53760;  // LDS of a workgroup: three share the CU's 160 KB
-constexpr int kTileXcdChunk = 1;      // tiles of one XCD's turn
 constexpr int kTileCols = kTileSide * kTileSide;
 constexpr int kTileWaves = 8;
-constexpr int kTileHdrSlack = 3;   // phases that the kernel's header read-ahead may touch past the last
-constexpr int kTileEntSlack = 64;  // entries that its chunk read-ahead may touch past the last
+constexpr int kTileLdsBytes = 53760;  // LDS of a workgroup: three share the CU's 160 KB
+static_assert(kTileLdsBytes <= 65536, "more needs the kernels' dynamic LDS limit raised");
+constexpr int kTileXcdChunk = 1;      // tiles of one XCD's turn
+constexpr int kTileHdrSlack = 3;      // phases that the kernel's header read-ahead may touch past the last
+constexpr int kTileEntSlack = 64;     // entries that its chunk read-ahead may touch past the last
 constexpr int kTileRowSlack = 64 * kTileWaves;  // rows that its read-ahead may touch past the last
-constexpr uint32_t kTileZeroRow = 0xff000000U;  // an empty run: segment slot 255 has no axial positions
 struct TileArgs {
   const uint32_t* phase_off;  // first phase of every (tile, subset)
   const uint4* hdr;           // per (phase, wave): first group, groups of its columns (8 bytes), first row
-  const uint32_t* row;        // LDS rows: segment slot << 24 | run within the segment
-  const int2* segs;           // per segment slot (256): device offset, nax | ppa << 16
+  const int2* row;            // LDS rows: the run's device offset, nax | ppa << 16
   const int32_t* off;         // entries: LDS byte offset of plane 0 in the run's row
   const float* w;             // entries: weight
-  const int2* rng;            // per (tile, view): first and last tangential index (x > y: none)
+  const int2* rng;            // per (tile, view, TOF bin): first and last tangential index (x > y: none)
   const int32_t* order;       // tiles in launch order
   int ntx, ntiles, nsub, nviews;
   int lead, stride, longest;  // floats: zeros before the first row, row pitch, longest run in planes
   int lds_floats;
+  bool tof;                   // entries are (element, TOF bin) terms
 };
-hipError_t tile_allow_lds(int bytes);
-void launch_tile_range(const Family* d_fams, const int2* d_fam_pos, int nfam, const int2* d_pool, const ImageDims& dims,
-                       int ntx, int nviews, int2* d_rng, int* d_need, hipStream_t stream);
-void launch_tile_phases(const int4* d_units, const int32_t* d_unit_off, int nsub, int ntiles, int nunits, int ntang,
-                        int nviews, const int2* d_rng, int rows, uint32_t* d_slot, uint32_t* d_nphase, uint32_t* d_nrow,
-                        int* d_bad, hipStream_t stream);
-void launch_tile_rows(const int4* d_units, const int32_t* d_unit_off, int nsub, int ntiles, int nunits, int ntang,
-                      int nviews, const int2* d_rng, int rows, const uint32_t* d_phase_off, const uint32_t* d_row_off,
-                      uint32_t* d_row, uint32_t* d_phase_row, int* d_bad, hipStream_t stream);
+// The table's passes. d_fp_rec: null, or the stored forward TOF records (w
+// weights each): then every TOF bin of a (segment, view) is a unit of its own.
+void launch_tile_range(const Family* d_fams, const int2* d_fam_pos, int nfam, const int2* d_pool,
+                       const int32_t* d_fp_rec, int w, const ImageDims& dims, int ntx, int nviews, int ntof, int2* d_rng,
+                       int* d_need, hipStream_t stream);
+void launch_tile_phases(const int4* d_units, const int32_t* d_unit_off, int nsub, int ntiles, int nunits, int nrng,
+                        const int2* d_rng, int rows, uint32_t* d_slot, uint32_t* d_nphase, uint32_t* d_nrow, int* d_bad,
+                        hipStream_t stream);
+void launch_tile_rows(const int4* d_units, const int32_t* d_unit_off, int nsub, int ntiles, int nunits, int nrng,
+                      const int2* d_rng, int rows, const uint32_t* d_phase_off, const uint32_t* d_row_off, int2* d_row,
+                      uint32_t* d_phase_row, int* d_bad, hipStream_t stream);
 void launch_tile_work(const uint32_t* d_group_off, const uint32_t* d_phase_off, int nsub, int ntiles, uint32_t* d_work,
                       hipStream_t stream);
 void launch_tile_count(const Family* d_fams, const int2* d_fam_pos, int fam_begin, int fam_end, int ntang,
-                       const int2* d_pool, int subset, const ImageDims& dims, const TileArgs& A, int nunits,
-                       const uint32_t* d_slot, uint32_t* d_counts, hipStream_t stream);
+                       const int2* d_pool, const int32_t* d_fp_rec, int w, int ntof, int subset, const ImageDims& dims,
+                       const TileArgs& A, int nunits, const uint32_t* d_slot, uint32_t* d_counts, hipStream_t stream);
 void launch_tile_make(const Family* d_fams, const int2* d_fam_pos, int fam_begin, int fam_end, int ntang,
-                      const int2* d_pool, int subset, const ImageDims& dims, const TileArgs& A, int nunits,
-                      const uint32_t* d_slot, uint32_t none, const int64_t* d_fam_entry_off, uint32_t* d_keys,
-                      int2* d_raw, hipStream_t stream);
+                      const int2* d_pool, const int32_t* d_fp_rec, int w, int ntof, int subset, const ImageDims& dims,
+                      const TileArgs& A, int nunits, const uint32_t* d_slot, uint32_t none, int span,
+                      const int64_t* d_fam_entry_off, int64_t first, uint32_t* d_keys, int2* d_raw, hipStream_t stream);
 void launch_tile_groups(const uint32_t* d_counts, int64_t n, uint32_t* d_groups, int* d_bad, hipStream_t stream);
 void launch_tile_headers(const uint32_t* d_groups, const uint32_t* d_group_off, const uint32_t* d_phase_row,
                          uint32_t total_rows, int64_t nphase, uint4* d_hdr, hipStream_t stream);
-void launch_tile_place(const uint32_t* d_keys, const uint32_t* d_idx, const int2* d_raw, const uint32_t* d_list_start,
-                       const uint32_t* d_group_off, int64_t n, int32_t* d_off, float* d_w, hipStream_t stream);
+void launch_tile_place(const uint32_t* d_keys, const uint32_t* d_idx, const int2* d_raw, const uint32_t* d_group_off,
+                       uint32_t none, int64_t n, int32_t* d_off, float* d_w, hipStream_t stream);
 void launch_back_project_tile(BpMode mode, const TileArgs& A, int subset_begin, int subset_end, const float* d_proj,
                               float* d_img, const ImageDims& dims, const BpData& data, hipStream_t stream);
 

@@ -38,6 +38,13 @@
 // takes its four by DPP broadcast inside the add and the multiply-add, so an
 // entry costs one address add, one two-slot LDS read and a multiply-add per
 // slot: 3 vector instructions for 128 planes, no scalar ones.
+//
+// TOF: every (element, TOF bin it reaches) is an entry of its own, and every
+// TOF bin of a (segment, view) a viewgram with rows of its own: 2.1e9 terms at
+// mMR size with 11 TOF bins (up to 5 per element). 24.4 ms, against 48.2 with
+// the stored back records, whose five gathers per element also went to L2; per
+// term it costs what the non-TOF kernel does. The table is 17 GB beside 27 GB
+// of records and 200 ms more to make.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -71,13 +78,30 @@ __device__ inline bool tile_elem(const Family& f, int coords, const ImageDims& d
   return true;
 }
 
-// pass 1, one wave per family: the tangential positions of every (tile, view)
-// and, over all elements, the most planes a row needs after a run's start
-// (rows[0]: nz - k) and before its end (rows[1]: run length + k)
+// The terms of a family's element e: its weight (non-TOF), or its weight in
+// each TOF bin it reaches, from the stored forward record (fp_rec, W weights
+// from bin c on; TOF families have rows of their own). fn(bin, weight).
+template <class F>
+__device__ inline void element_terms(const int32_t* __restrict__ fp_rec, int W, int64_t pool_index, int weight, F&& fn) {
+  if (!fp_rec) {
+    fn(0, weight);
+    return;
+  }
+  const int32_t* r = fp_rec + pool_index * (2 + W);
+  const int c = r[0] >> 20;
+  for (int j = 0; j < W; ++j)
+    if (__int_as_float(r[2 + j]) != 0.F) fn(c + j, r[2 + j]);
+}
+
+// pass 1, one wave per family: the tangential positions of every (tile, view,
+// TOF bin) and, over all elements, the most planes a row needs after a run's
+// start (need[0]: nz - k) and before its end (need[1]: run length + k)
 __global__ void __launch_bounds__(kWave) tile_range_kernel(const Family* __restrict__ fams,
                                                            const int2* __restrict__ fam_pos, int nfam,
-                                                           const int2* __restrict__ pool, ImageDims d, int ntx,
-                                                           int nviews, int2* __restrict__ rng, int* __restrict__ need) {
+                                                           const int2* __restrict__ pool,
+                                                           const int32_t* __restrict__ fp_rec, int W, ImageDims d,
+                                                           int ntx, int nviews, int ntof, int2* __restrict__ rng,
+                                                           int* __restrict__ need) {
   const int fi = blockIdx.x;
   if (fi >= nfam) return;
   const Family f = fams[fi];
@@ -87,26 +111,35 @@ __global__ void __launch_bounds__(kWave) tile_range_kernel(const Family* __restr
   for (int e0 = 0; e0 < f.row_len; e0 += kWave) {
     const int e = e0 + lane;
     TileElem E;
-    const bool ok = e < f.row_len && tile_elem(f, pool[f.row_start + (e < f.row_len ? e : 0)].x, d, ntx, E);
-    const int t = ok ? E.t : -1;
+    const int64_t pi = static_cast<int64_t>(f.row_start) + (e < f.row_len ? e : 0);
+    const bool ok = e < f.row_len && tile_elem(f, pool[pi].x, d, ntx, E);
+    uint32_t bins = 0;  // the element's TOF bins
     if (ok) {
       after = max(after, d.nz - E.k);
       before = max(before, f.ppa * (f.nax - 1) + 1 + E.k);
+      element_terms(fp_rec, W, pi, 0, [&](int bin, int) { bins |= 1U << bin; });
     }
-    // neighbouring elements of a row lie mostly in one tile: one update per run of them
-    const int prev = __shfl_up(t, 1, kWave);
-    if (ok && (lane == 0 || prev != t)) {
-      int2* r = rng + static_cast<int64_t>(t) * nviews + pos.x;
-      atomicMin(&r->x, pos.y);
-      atomicMax(&r->y, pos.y);
+    // neighbouring elements of a row lie mostly in one tile and the same bins:
+    // one update per run of them
+    const int t = ok ? E.t : -1;
+    const int prev_t = __shfl_up(t, 1, kWave);
+    const uint32_t prev_b = __shfl_up(bins, 1, kWave);
+    if (ok && (lane == 0 || prev_t != t || (bins & ~prev_b))) {
+      for (int k = 0; k < ntof; ++k) {
+        if (!(bins >> k & 1)) continue;
+        int2* r = rng + (static_cast<int64_t>(t) * nviews + pos.x) * ntof + k;
+        // (a stale value read here only costs the atomic)
+        if (pos.y < __hip_atomic_load(&r->x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(&r->x, pos.y);
+        if (pos.y > __hip_atomic_load(&r->y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(&r->y, pos.y);
+      }
     }
   }
   for (int o = kWave / 2; o > 0; o >>= 1) {
     after = max(after, __shfl_xor(after, o, kWave));
     before = max(before, __shfl_xor(before, o, kWave));
   }
-  // most families do not raise the maxima: read them first (a stale value
-  // only costs the atomic), or every wave would queue on one address
+  // most families do not raise the maxima: read them first, or every wave
+  // would queue on one address
   if (lane == 0 && before > 0) {
     if (after > __hip_atomic_load(need, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(need, after);
     if (before > __hip_atomic_load(need + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(need + 1, before);
@@ -120,10 +153,10 @@ __global__ void __launch_bounds__(kWave) tile_range_kernel(const Family* __restr
 // longer run (of another segment) a row of zeros lies between.
 template <bool FILL>
 __global__ void tile_phase_kernel(const int4* __restrict__ units, const int32_t* __restrict__ unit_off, int nsub,
-                                  int ntiles, int nunits, int ntang, int nviews, const int2* __restrict__ rng, int rows,
+                                  int ntiles, int nunits, int nrng, const int2* __restrict__ rng, int rows,
                                   uint32_t* __restrict__ slot, uint32_t* __restrict__ nphase,
                                   uint32_t* __restrict__ nrow, const uint32_t* __restrict__ phase_off,
-                                  const uint32_t* __restrict__ row_off, uint32_t* __restrict__ row,
+                                  const uint32_t* __restrict__ row_off, int2* __restrict__ row,
                                   uint32_t* __restrict__ phase_row, int* __restrict__ bad) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= nsub * ntiles) return;
@@ -131,23 +164,23 @@ __global__ void tile_phase_kernel(const int4* __restrict__ units, const int32_t*
   int ph = -1, used = 0, prev = 0;
   uint32_t n = 0;
   for (int u = unit_off[s]; u < unit_off[s + 1]; ++u) {
-    const int4 U = units[u];  // segment slot, run length in planes, -, view
-    const int2 r = rng[static_cast<int64_t>(t) * nviews + U.w];
+    const int4 U = units[u];  // device offset, nax, ppa, index among the tile's ranges
+    const int2 r = rng[static_cast<int64_t>(t) * nrng + U.w];
     const int T = r.y - r.x + 1;
     if (r.y < r.x) continue;
-    int gap = prev > U.y;
+    const int len = U.z * (U.y - 1) + 1;
+    int gap = prev > len;
     if (T > rows) *bad = 1;
     if (ph < 0 || used + gap + T > rows) {
       ++ph;
       used = gap = 0;
       if (FILL) phase_row[phase_off[i] + ph] = row_off[i] + n;
     }
-    prev = U.y;
+    prev = len;
     if (FILL) {
-      uint32_t* o = row + row_off[i] + n;
-      if (gap) *o++ = kTileZeroRow;
-      const uint32_t first = static_cast<uint32_t>(U.x) << 24 | static_cast<uint32_t>(U.w * ntang + r.x);
-      for (int k = 0; k < T; ++k) o[k] = first + k;
+      int2* o = row + row_off[i] + n;
+      if (gap) *o++ = make_int2(0, 1 << 16);  // an empty run
+      for (int k = 0; k < T; ++k) o[k] = make_int2(U.x + (r.x + k) * U.y, U.y | U.z << 16);
     } else {
       slot[static_cast<int64_t>(t) * nunits + u] = static_cast<uint32_t>(ph) << 16 | (used + gap);
     }
@@ -162,43 +195,47 @@ __global__ void tile_phase_kernel(const int4* __restrict__ units, const int32_t*
 }
 
 // passes 3 and 4, one wave per family of subset s: the number of entries of
-// every (phase, column), then every element's key and entry in family order,
-// element order (elements without an image plane get the last key)
+// every (phase, column), then every term's key and entry at slot
+// (element offset - first) * span + its rank, in family order, element order,
+// bin order (slots without a term get the last key)
 template <bool COUNT>
 __global__ void __launch_bounds__(kWave) tile_entries_kernel(const Family* __restrict__ fams,
                                                              const int2* __restrict__ fam_pos, int fam_begin,
                                                              int fam_end, int ntang, const int2* __restrict__ pool,
+                                                             const int32_t* __restrict__ fp_rec, int W, int ntof,
                                                              int subset, ImageDims d, TileArgs A, int nunits,
                                                              const uint32_t* __restrict__ slot,
-                                                             uint32_t* __restrict__ counts, uint32_t none,
-                                                             const int64_t* __restrict__ fam_entry_off,
+                                                             uint32_t* __restrict__ counts, uint32_t none, int span,
+                                                             const int64_t* __restrict__ fam_entry_off, int64_t first,
                                                              uint32_t* __restrict__ keys, int2* __restrict__ raw) {
   const int fi = fam_begin + blockIdx.x;
   if (fi >= fam_end) return;
   const Family f = fams[fi];
   const int2 pos = fam_pos[fi];
-  const int unit = fi / ntang;
-  const int64_t base = COUNT ? 0 : fam_entry_off[fi];
+  const int unit = fi / ntang * ntof;
+  const int64_t base = COUNT ? 0 : fam_entry_off[fi] - first;
   for (int e = threadIdx.x; e < f.row_len; e += kWave) {
-    const int2 el = pool[f.row_start + e];
+    const int64_t pi = static_cast<int64_t>(f.row_start) + e;
+    const int2 el = pool[pi];
     TileElem E;
-    uint32_t key = none;
-    int off4 = 0;
-    if (tile_elem(f, el.x, d, A.ntx, E)) {
-      const uint32_t sl = slot[static_cast<int64_t>(E.t) * nunits + unit];
-      const uint32_t ph = A.phase_off[static_cast<int64_t>(E.t) * A.nsub + subset] + (sl >> 16);
-      key = ph * kTileCols + E.c;
-      if (COUNT) {
-        atomicAdd(&counts[key], 1U);
-      } else {
-        const int row = static_cast<int>(sl & 0xffff) + pos.y - A.rng[static_cast<int64_t>(E.t) * A.nviews + pos.x].x;
-        off4 = 4 * (A.lead + row * A.stride - E.k);
-      }
-    }
-    if (!COUNT) {
-      keys[base + e] = key;
-      raw[base + e] = make_int2(off4, el.y);
-    }
+    int n = 0;
+    if (tile_elem(f, el.x, d, A.ntx, E))
+      element_terms(fp_rec, W, pi, el.y, [&](int bin, int weight) {
+        const uint32_t sl = slot[static_cast<int64_t>(E.t) * nunits + unit + bin];
+        const uint32_t ph = A.phase_off[static_cast<int64_t>(E.t) * A.nsub + subset] + (sl >> 16);
+        const uint32_t key = ph * kTileCols + E.c;
+        if (COUNT) {
+          atomicAdd(&counts[key], 1U);
+        } else {
+          const int2 r = A.rng[(static_cast<int64_t>(E.t) * A.nviews + pos.x) * ntof + bin];
+          const int row = static_cast<int>(sl & 0xffff) + pos.y - r.x;
+          keys[(base + e) * span + n] = key;
+          raw[(base + e) * span + n] = make_int2(4 * (A.lead + row * A.stride - E.k), weight);
+        }
+        ++n;
+      });
+    if (!COUNT)
+      for (; n < span; ++n) keys[(base + e) * span + n] = none;
   }
 }
 
@@ -240,16 +277,19 @@ __global__ void tile_work_kernel(const uint32_t* __restrict__ group_off, const u
   work[t] = group_off[b * kTileCols] - group_off[a * kTileCols];
 }
 
-// sorted element r -> its place: 4 x its list's first group + its rank in the list
+// sorted term r -> its place: 4 x its list's first group + its rank in the
+// list (a list has a few tens of entries)
 __global__ void tile_place_kernel(const uint32_t* __restrict__ keys, const uint32_t* __restrict__ idx,
-                                  const int2* __restrict__ raw, const uint32_t* __restrict__ list_start,
-                                  const uint32_t* __restrict__ group_off, int64_t n, int32_t* __restrict__ off,
-                                  float* __restrict__ w) {
+                                  const int2* __restrict__ raw, const uint32_t* __restrict__ group_off, uint32_t none,
+                                  int64_t n, int32_t* __restrict__ off, float* __restrict__ w) {
   for (int64_t r = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; r < n;
        r += static_cast<int64_t>(gridDim.x) * blockDim.x) {
     const uint32_t key = keys[r];
+    if (key == none) continue;
+    int64_t rank = 0;
+    while (rank < r && keys[r - rank - 1] == key) ++rank;
     const int2 E = raw[idx[r]];
-    const int64_t at = 4 * static_cast<int64_t>(group_off[key]) + (r - list_start[key]);
+    const int64_t at = 4 * static_cast<int64_t>(group_off[key]) + rank;
     off[at] = E.x;
     w[at] = __int_as_float(E.y);
   }
@@ -305,7 +345,13 @@ __device__ inline void tile_group(int off, int w, const char* lds, int lane4, fl
   for (int q = 0; q < NSLOT; ++q) add_bcast<3>(acc[q], w, v[3][q]);
 }
 
-template <int MODE, int NSLOT>
+// TOF: the sums of kTileSumPhases phases are added to the voxel's sum
+// together. An element has a term per TOF bin here, so that one chain of
+// additions would be as many times longer than the elements' (and its rounding
+// error larger) as an element reaches bins.
+constexpr uint32_t kTileSumPhases = 8;
+
+template <int MODE, int NSLOT, bool TOF>
 __global__ void __launch_bounds__(kWave* kTileWaves) bp_tile_kernel(TileArgs A, int sb, int se,
                                                                     const float* __restrict__ proj,
                                                                     float* __restrict__ img, ImageDims d, BpData data,
@@ -318,11 +364,11 @@ __global__ void __launch_bounds__(kWave* kTileWaves) bp_tile_kernel(TileArgs A, 
   const int lane = static_cast<int>(threadIdx.x % kWave);
   const int lane4 = 4 * lane;
   for (int i = threadIdx.x; i < A.lds_floats; i += kWave * kTileWaves) tile_lds[i] = 0.F;
-  float acc[kTileCpw][NSLOT];
+  float acc[kTileCpw][NSLOT], sum[kTileCpw][NSLOT];
 #pragma unroll
   for (int c = 0; c < kTileCpw; ++c)
 #pragma unroll
-    for (int q = 0; q < NSLOT; ++q) acc[c][q] = 0.F;
+    for (int q = 0; q < NSLOT; ++q) acc[c][q] = sum[c][q] = 0.F;
 #if defined(__HIP_DEVICE_COMPILE__)
   const char* lds = reinterpret_cast<const char*>(tile_lds);
   const int l16 = lane % 16;
@@ -335,23 +381,22 @@ __global__ void __launch_bounds__(kWave* kTileWaves) bp_tile_kernel(TileArgs A, 
   asm volatile("" : "+v"(zero));
   const uint4* hp = A.hdr + static_cast<int64_t>(p0) * kTileWaves + wave + zero;
   uint4 h = hp[0], h1 = hp[kTileWaves];
-  uint32_t rw = A.row[h.w + wave + kTileWaves * lane];
+  int2 rw = A.row[h.w + wave + kTileWaves * lane];
   for (uint32_t p = p0; p < p1; ++p) {
     const uint32_t group0 = __builtin_amdgcn_readfirstlane(h.x);
     const uint32_t cnt[2] = {static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(h.y)),
                              static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(h.z))};
     const int nrow = static_cast<int>(__builtin_amdgcn_readfirstlane(h1.w) - __builtin_amdgcn_readfirstlane(h.w));
-    const int2 sg = A.segs[rw >> 24];  // device offset, nax | ppa << 16
-    const int base = sg.x + static_cast<int>(rw & 0xffffff) * (sg.y & 0xffff);
+    const int2 cur = rw;
     const char* po = reinterpret_cast<const char*>(A.off + 4 * static_cast<int64_t>(group0));
     const char* pw = reinterpret_cast<const char*>(A.w + 4 * static_cast<int64_t>(group0));
     unsigned at = 4 * l16;  // byte offset of this lane's entry
     __syncthreads();        // the previous phase's rows have been read
     float* dst = tile_lds + A.lead + wave * A.stride;
     for (int l = 0, r = wave; r < nrow; ++l, r += kTileWaves, dst += kTileWaves * A.stride) {
-      const int np = __builtin_amdgcn_readlane(sg.y, l);
+      const int np = __builtin_amdgcn_readlane(cur.y, l);
       const __amdgpu_buffer_rsrc_t run =
-          run_buffer(as_const(proj), static_cast<unsigned>(__builtin_amdgcn_readlane(base, l)), np & 0xffff);
+          run_buffer(as_const(proj), static_cast<unsigned>(__builtin_amdgcn_readlane(cur.x, l)), np & 0xffff);
 #pragma unroll
       for (int q = 0; q < NSLOT; ++q) {
         // this lane's plane in the run; outside [0, 4 nax) the buffer reads 0
@@ -396,6 +441,23 @@ __global__ void __launch_bounds__(kWave* kTileWaves) bp_tile_kernel(TileArgs A, 
         }
       }
     }
+    if constexpr (TOF) {
+      if ((p - p0) % kTileSumPhases == kTileSumPhases - 1) {
+#pragma unroll
+        for (int c = 0; c < kTileCpw; ++c)
+#pragma unroll
+          for (int q = 0; q < NSLOT; ++q) {
+            sum[c][q] += acc[c][q];
+            acc[c][q] = 0.F;
+          }
+      }
+    }
+  }
+  if constexpr (TOF) {
+#pragma unroll
+    for (int c = 0; c < kTileCpw; ++c)
+#pragma unroll
+      for (int q = 0; q < NSLOT; ++q) acc[c][q] += sum[c][q];
   }
 #endif
   const int x0 = (t % A.ntx) * kTileSide, y0 = (t / A.ntx) * kTileSide;
@@ -432,46 +494,47 @@ unsigned grid_of(int64_t n) {
 
 }  // namespace
 
-void launch_tile_range(const Family* d_fams, const int2* d_fam_pos, int nfam, const int2* d_pool, const ImageDims& dims,
-                       int ntx, int nviews, int2* d_rng, int* d_need, hipStream_t stream) {
+void launch_tile_range(const Family* d_fams, const int2* d_fam_pos, int nfam, const int2* d_pool,
+                       const int32_t* d_fp_rec, int w, const ImageDims& dims, int ntx, int nviews, int ntof, int2* d_rng,
+                       int* d_need, hipStream_t stream) {
   if (nfam <= 0) return;
-  hipLaunchKernelGGL(tile_range_kernel, dim3(nfam), dim3(kWave), 0, stream, d_fams, d_fam_pos, nfam, d_pool, dims, ntx,
-                     nviews, d_rng, d_need);
+  hipLaunchKernelGGL(tile_range_kernel, dim3(nfam), dim3(kWave), 0, stream, d_fams, d_fam_pos, nfam, d_pool, d_fp_rec, w,
+                     dims, ntx, nviews, ntof, d_rng, d_need);
 }
 
-void launch_tile_phases(const int4* d_units, const int32_t* d_unit_off, int nsub, int ntiles, int nunits, int ntang,
-                        int nviews, const int2* d_rng, int rows, uint32_t* d_slot, uint32_t* d_nphase, uint32_t* d_nrow,
+void launch_tile_phases(const int4* d_units, const int32_t* d_unit_off, int nsub, int ntiles, int nunits, int nrng,
+                        const int2* d_rng, int rows, uint32_t* d_slot, uint32_t* d_nphase, uint32_t* d_nrow,
                         int* d_bad, hipStream_t stream) {
   hipLaunchKernelGGL(tile_phase_kernel<false>, dim3((nsub * ntiles + 63) / 64), dim3(64), 0, stream, d_units, d_unit_off,
-                     nsub, ntiles, nunits, ntang, nviews, d_rng, rows, d_slot, d_nphase, d_nrow, nullptr, nullptr,
+                     nsub, ntiles, nunits, nrng, d_rng, rows, d_slot, d_nphase, d_nrow, nullptr, nullptr,
                      nullptr, nullptr, d_bad);
 }
 
-void launch_tile_rows(const int4* d_units, const int32_t* d_unit_off, int nsub, int ntiles, int nunits, int ntang,
-                      int nviews, const int2* d_rng, int rows, const uint32_t* d_phase_off, const uint32_t* d_row_off,
-                      uint32_t* d_row, uint32_t* d_phase_row, int* d_bad, hipStream_t stream) {
+void launch_tile_rows(const int4* d_units, const int32_t* d_unit_off, int nsub, int ntiles, int nunits, int nrng,
+                      const int2* d_rng, int rows, const uint32_t* d_phase_off, const uint32_t* d_row_off,
+                      int2* d_row, uint32_t* d_phase_row, int* d_bad, hipStream_t stream) {
   hipLaunchKernelGGL(tile_phase_kernel<true>, dim3((nsub * ntiles + 63) / 64), dim3(64), 0, stream, d_units, d_unit_off,
-                     nsub, ntiles, nunits, ntang, nviews, d_rng, rows, nullptr, nullptr, nullptr, d_phase_off, d_row_off,
+                     nsub, ntiles, nunits, nrng, d_rng, rows, nullptr, nullptr, nullptr, d_phase_off, d_row_off,
                      d_row, d_phase_row, d_bad);
 }
 
 void launch_tile_count(const Family* d_fams, const int2* d_fam_pos, int fam_begin, int fam_end, int ntang,
-                       const int2* d_pool, int subset, const ImageDims& dims, const TileArgs& A, int nunits,
-                       const uint32_t* d_slot, uint32_t* d_counts, hipStream_t stream) {
+                       const int2* d_pool, const int32_t* d_fp_rec, int w, int ntof, int subset, const ImageDims& dims,
+                       const TileArgs& A, int nunits, const uint32_t* d_slot, uint32_t* d_counts, hipStream_t stream) {
   if (fam_end <= fam_begin) return;
   hipLaunchKernelGGL(tile_entries_kernel<true>, dim3(fam_end - fam_begin), dim3(kWave), 0, stream, d_fams, d_fam_pos,
-                     fam_begin, fam_end, ntang, d_pool, subset, dims, A, nunits, d_slot, d_counts, 0U, nullptr, nullptr,
-                     nullptr);
+                     fam_begin, fam_end, ntang, d_pool, d_fp_rec, w, ntof, subset, dims, A, nunits, d_slot, d_counts, 0U,
+                     0, nullptr, int64_t{0}, nullptr, nullptr);
 }
 
 void launch_tile_make(const Family* d_fams, const int2* d_fam_pos, int fam_begin, int fam_end, int ntang,
-                      const int2* d_pool, int subset, const ImageDims& dims, const TileArgs& A, int nunits,
-                      const uint32_t* d_slot, uint32_t none, const int64_t* d_fam_entry_off, uint32_t* d_keys,
-                      int2* d_raw, hipStream_t stream) {
+                      const int2* d_pool, const int32_t* d_fp_rec, int w, int ntof, int subset, const ImageDims& dims,
+                      const TileArgs& A, int nunits, const uint32_t* d_slot, uint32_t none, int span,
+                      const int64_t* d_fam_entry_off, int64_t first, uint32_t* d_keys, int2* d_raw, hipStream_t stream) {
   if (fam_end <= fam_begin) return;
   hipLaunchKernelGGL(tile_entries_kernel<false>, dim3(fam_end - fam_begin), dim3(kWave), 0, stream, d_fams, d_fam_pos,
-                     fam_begin, fam_end, ntang, d_pool, subset, dims, A, nunits, d_slot, nullptr, none, d_fam_entry_off,
-                     d_keys, d_raw);
+                     fam_begin, fam_end, ntang, d_pool, d_fp_rec, w, ntof, subset, dims, A, nunits, d_slot, nullptr, none,
+                     span, d_fam_entry_off, first, d_keys, d_raw);
 }
 
 void launch_tile_groups(const uint32_t* d_counts, int64_t n, uint32_t* d_groups, int* d_bad, hipStream_t stream) {
@@ -491,11 +554,11 @@ void launch_tile_work(const uint32_t* d_group_off, const uint32_t* d_phase_off, 
                      ntiles, d_work);
 }
 
-void launch_tile_place(const uint32_t* d_keys, const uint32_t* d_idx, const int2* d_raw, const uint32_t* d_list_start,
-                       const uint32_t* d_group_off, int64_t n, int32_t* d_off, float* d_w, hipStream_t stream) {
+void launch_tile_place(const uint32_t* d_keys, const uint32_t* d_idx, const int2* d_raw, const uint32_t* d_group_off,
+                       uint32_t none, int64_t n, int32_t* d_off, float* d_w, hipStream_t stream) {
   if (n <= 0) return;
-  hipLaunchKernelGGL(tile_place_kernel, dim3(grid_of(n)), dim3(256), 0, stream, d_keys, d_idx, d_raw, d_list_start,
-                     d_group_off, n, d_off, d_w);
+  hipLaunchKernelGGL(tile_place_kernel, dim3(grid_of(n)), dim3(256), 0, stream, d_keys, d_idx, d_raw, d_group_off, none,
+                     n, d_off, d_w);
 }
 
 void launch_back_project_tile(BpMode mode, const TileArgs& A, int subset_begin, int subset_end, const float* d_proj,
@@ -504,38 +567,25 @@ void launch_back_project_tile(BpMode mode, const TileArgs& A, int subset_begin, 
   const int chunk = kTileXcdChunk, round = kNumXcd * chunk;
   const dim3 grid((A.ntiles + round - 1) / round * round), block(kWave * kTileWaves);
   const size_t lds = static_cast<size_t>(A.lds_floats) * sizeof(float);
-#define MI_TILE(M, S)                                                                                                 \
-  hipLaunchKernelGGL((bp_tile_kernel<M, S>), grid, block, lds, stream, A, subset_begin, subset_end, d_proj, d_img, dims, \
-                     data, chunk)
-#define MI_TILE_S(M)             \
-  switch (nslot) {               \
-    case 1: MI_TILE(M, 1); break; \
-    case 2: MI_TILE(M, 2); break; \
-    case 3: MI_TILE(M, 3); break; \
-    default: MI_TILE(M, 4); break; \
+#define MI_TILE(M, S, T)                                                                                          \
+  hipLaunchKernelGGL((bp_tile_kernel<M, S, T>), grid, block, lds, stream, A, subset_begin, subset_end, d_proj, d_img, \
+                     dims, data, chunk)
+#define MI_TILE_S(M, T)              \
+  switch (nslot) {                  \
+    case 1: MI_TILE(M, 1, T); break; \
+    case 2: MI_TILE(M, 2, T); break; \
+    case 3: MI_TILE(M, 3, T); break; \
+    default: MI_TILE(M, 4, T); break; \
   }
-  if (mode == BP_PLAIN) { MI_TILE_S(BP_PLAIN) }
-  else { MI_TILE_S(BP_OSEM_UPDATE) }
+  if (A.tof) {
+    if (mode == BP_PLAIN) { MI_TILE_S(BP_PLAIN, true) }
+    else { MI_TILE_S(BP_OSEM_UPDATE, true) }
+  } else {
+    if (mode == BP_PLAIN) { MI_TILE_S(BP_PLAIN, false) }
+    else { MI_TILE_S(BP_OSEM_UPDATE, false) }
+  }
 #undef MI_TILE_S
 #undef MI_TILE
-}
-
-// LDS above 64 KB per workgroup needs the kernels' dynamic limit raised on
-// every device they run on
-hipError_t tile_allow_lds(int bytes) {
-  const void* k[] = {reinterpret_cast<const void*>(&bp_tile_kernel<BP_PLAIN, 1>),
-                     reinterpret_cast<const void*>(&bp_tile_kernel<BP_PLAIN, 2>),
-                     reinterpret_cast<const void*>(&bp_tile_kernel<BP_PLAIN, 3>),
-                     reinterpret_cast<const void*>(&bp_tile_kernel<BP_PLAIN, 4>),
-                     reinterpret_cast<const void*>(&bp_tile_kernel<BP_OSEM_UPDATE, 1>),
-                     reinterpret_cast<const void*>(&bp_tile_kernel<BP_OSEM_UPDATE, 2>),
-                     reinterpret_cast<const void*>(&bp_tile_kernel<BP_OSEM_UPDATE, 3>),
-                     reinterpret_cast<const void*>(&bp_tile_kernel<BP_OSEM_UPDATE, 4>)};
-  for (const void* f : k) {
-    const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    if (e != hipSuccess) return e;
-  }
-  return hipSuccess;
 }
 
 }  // namespace mi
