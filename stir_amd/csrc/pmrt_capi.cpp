@@ -181,6 +181,8 @@ struct mi_ctx {
   // time of flight: ntof blocks of block_bins bins each
   int ntof = 1;
   int64_t block_bins = 0;
+  DBuf<mi::LayoutBlock> lay_blocks;  // the segments, then the image
+  int num_segs = 0, max_axial = 0;
   DBuf<mi::FamilyLor> lors;
   DBuf<float> entry_d;   // TOF distance of every back-projection table entry
   // stored TOF rows (records with each element's TOF weights, pmrt_tof.hip):
@@ -281,32 +283,22 @@ struct mi_ctx {
   static hipStream_t pick(void* s) { return static_cast<hipStream_t>(s); }
 
   // ---- layout conversions
+  // lay_blocks: the segments, then the image
   void image_to_device(const float* src_stir, float* dst, hipStream_t st) const {
-    mi::launch_transpose(src_stir, dst, dims.nz, dims.ncols, dims.ncols, dims.nzp, st);
+    mi::launch_layout(true, lay_blocks.p + num_segs, 1, dims.nz, dims.ncols, 1, 0, src_stir, dst, st);
   }
   void image_from_device(const float* src, float* dst_stir, hipStream_t st) const {
-    mi::launch_transpose(src, dst_stir, dims.ncols, dims.nz, dims.nzp, dims.ncols, st);
+    mi::launch_layout(false, lay_blocks.p + num_segs, 1, dims.nz, dims.ncols, 1, 0, src, dst_stir, st);
   }
-  // projection data: each TOF block (one block without TOF) is converted on its own
   void proj_to_device(const float* src_stir, float* dst, hipStream_t st) const {
     const mi_geometry& g = plan->geometry();
-    const int cols = g.num_views * g.num_tangential_poss;
-    for (int k = 0; k < ntof; ++k)
-      for (int seg : plan->segment_sequence()) {
-        const int64_t off = plan->segment_offset(seg) + k * block_bins;
-        const int nax = plan->num_axial(seg);
-        mi::launch_transpose(src_stir + off, dst + off, nax, cols, cols, nax, st);
-      }
+    mi::launch_layout(true, lay_blocks.p, num_segs, max_axial, g.num_views * g.num_tangential_poss, ntof, block_bins,
+                      src_stir, dst, st);
   }
   void proj_from_device(const float* src, float* dst_stir, hipStream_t st) const {
     const mi_geometry& g = plan->geometry();
-    const int cols = g.num_views * g.num_tangential_poss;
-    for (int k = 0; k < ntof; ++k)
-      for (int seg : plan->segment_sequence()) {
-        const int64_t off = plan->segment_offset(seg) + k * block_bins;
-        const int nax = plan->num_axial(seg);
-        mi::launch_transpose(src + off, dst_stir + off, cols, nax, nax, cols, st);
-      }
+    mi::launch_layout(false, lay_blocks.p, num_segs, max_axial, g.num_views * g.num_tangential_poss, ntof, block_bins, src,
+                      dst_stir, st);
   }
 
   // ---- projections on device-layout buffers
@@ -1438,6 +1430,17 @@ void mi_ctx::set_up(const mi_geometry& g, int nsub) {
   dims.ncols = plan->num_columns();
   ntof = plan->num_tof_bins();
   block_bins = plan->num_bins();
+  std::vector<mi::LayoutBlock> lay;
+  max_axial = 0;
+  for (int seg : plan->segment_sequence()) {
+    const int nax = plan->num_axial(seg);
+    lay.push_back({plan->segment_offset(seg), nax, nax});
+    max_axial = std::max(max_axial, nax);
+  }
+  num_segs = static_cast<int>(lay.size());
+  lay.push_back({0, dims.nz, dims.nzp});
+  lay_blocks.alloc(lay.size());
+  HIPCHECK(hipMemcpy(lay_blocks.p, lay.data(), lay_blocks.bytes(), hipMemcpyHostToDevice));
   if (ntof > 1) {
     for (const mi::Family& f : plan->families()) {
       if (f.inplane != mi::IP_ID || f.zsign != 1) throw ApiError(MI_ERR_INTERNAL, "TOF family with an in-plane symmetry");

@@ -167,7 +167,16 @@ struct BpTuning {
 void launch_back_project(BpMode mode, int ppa, const int64_t* d_list_off, const BpEntry* d_entries, int subset_begin,
                          int subset_end, const float* d_proj, float* d_img, const ImageDims& dims, const BpData& data,
                          const BpTuning& tune, hipStream_t stream, int64_t proj_values = 0);
-// 2-D transpose used for the STIR <-> device layout conversions:
+// STIR <-> device layout of whole images and projection data sets: `nblocks`
+// blocks of `rows` x cols values at the same offset on both sides, [row][col]
+// on STIR's and [col][row] with pitch ld on the device's; ntof sets of them.
+struct LayoutBlock {
+  int64_t off;
+  int rows, ld;
+};
+void launch_layout(bool to_device, const LayoutBlock* d_blocks, int nblocks, int max_rows, int cols, int ntof,
+                   int64_t tof_stride, const float* src, float* dst, hipStream_t stream);
+// 2-D transpose, for single viewgrams:
 // dst[c * dst_ld + r] = src[r * src_ld + c] for r < rows, c < cols.
 void launch_transpose(const float* src, float* dst, int rows, int cols, int src_ld, int dst_ld, hipStream_t stream);
 
