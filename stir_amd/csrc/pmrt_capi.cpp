@@ -1183,11 +1183,10 @@ bool mi_ctx::build_slab_table() {
 // The tile table (pmrt_tile.hip) of a matrix whose families cover whole runs;
 // false where the geometry does not qualify (the column kernels are used
 // then). TOF matrices: from the stored forward records, span the most TOF bins
-// of one element. Images of up to 32 planes stay with the column kernels, which
-// pack them better than a wave of 64 planes.
+// of one element.
 bool mi_ctx::build_tile_table(int span) {
   const mi_geometry& g = plan->geometry();
-  if (!slab_allowed || slab_enable || quad_enable || dims.nz <= 32 || dims.nz > 256 || h_fams.empty()) return false;
+  if (!slab_allowed || slab_enable || quad_enable || dims.nz > 256 || h_fams.empty()) return false;
   if (total_bins() >= (int64_t{1} << 31) || (ntof > 1 && tof_fp_w <= 0)) return false;
   const int32_t* rec = ntof > 1 ? tof_fp_rec.p : nullptr;
   const auto& keys = plan->family_keys();
@@ -1196,6 +1195,15 @@ bool mi_ctx::build_tile_table(int span) {
   // per (segment, view)
   if (nfam % ntang) return false;
   const int nunits = nfam / ntang * ntof, nrng = g.num_views * ntof;
+  mi::TileShape S{8, 8, 1, 0, 64};
+  const bool short_img = dims.nz <= mi::kTileShortPlanes;
+  if (short_img) {
+    if (total_bins() >= (int64_t{1} << 30)) return false;
+    S.par = uniform_ppa == 2 ? 2 : 1;
+    S.lanes = (dims.nz <= mi::kTileShortPlanes / 2 ? 16 : 32) / S.par;
+    S.ty = 4;
+  }
+  S.ntx = (dims.nx + S.tx - 1) / S.tx;
   std::vector<int4> hunits(nunits);
   std::vector<int2> hpos(nfam);
   int longest = 0;
@@ -1214,11 +1222,11 @@ bool mi_ctx::build_tile_table(int span) {
     }
     for (int k = 0; k < ntof; ++k)
       hunits[u * ntof + k] =
-          make_int4(static_cast<int>(f0.sino_base + k * block_bins), f0.nax, f0.ppa, k0.view * ntof + k);
-    longest = std::max(longest, f0.ppa * (f0.nax - 1) + 1);
+          make_int4(static_cast<int>(f0.sino_base + k * block_bins), f0.nax, f0.ppa / S.par, k0.view * ntof + k);
+    longest = std::max(longest, f0.ppa / S.par * (f0.nax - 1) + 1);
   }
   const int nslot = (dims.nz + 63) / 64;
-  if (longest > 64 * nslot) return false;
+  if (!short_img && longest > 64 * nslot) return false;
   std::vector<int32_t> hunit_off(nsub + 1);
   for (int s = 0; s <= nsub; ++s) {
     if (plan->subset_family_begin(s) % ntang) return false;
@@ -1234,8 +1242,7 @@ bool mi_ctx::build_tile_table(int span) {
     most = std::max(most, fam_off[plan->subset_family_begin(s + 1)] - fam_off[plan->subset_family_begin(s)]);
   most *= span;
   if (most <= 0 || most >= (int64_t{1} << 31)) return false;
-  const int ntx = (dims.nx + mi::kTileSide - 1) / mi::kTileSide, nty = (dims.ny + mi::kTileSide - 1) / mi::kTileSide;
-  const int ntiles = ntx * nty;
+  const int ntiles = S.ntx * ((dims.ny + S.ty - 1) / S.ty);
   if (ntof > 1) {
     // only where the terms (8 bytes each, padded lists), the rows and the sort's
     // buffers fit beside everything else
@@ -1260,7 +1267,7 @@ bool mi_ctx::build_tile_table(int span) {
   DBuf<int> d_need;  // planes after a run's start, planes up to its end, flag
   d_need.alloc(3);
   HIPCHECK(hipMemsetAsync(d_need.p, 0, d_need.bytes(), stream));
-  mi::launch_tile_range(fams.p, d_pos.p, nfam, pool.p, rec, tof_fp_w, dims, ntx, g.num_views, ntof, tile_rng.p, d_need.p,
+  mi::launch_tile_range(fams.p, d_pos.p, nfam, pool.p, rec, tof_fp_w, dims, S, g.num_views, ntof, tile_rng.p, d_need.p,
                         stream);
   HIPCHECK(hipGetLastError());
   int need[3];
@@ -1268,17 +1275,30 @@ bool mi_ctx::build_tile_table(int span) {
   HIPCHECK(hipStreamSynchronize(stream));
   if (need[1] <= 0) return false;  // no element reaches the image
   mi::TileArgs A{};
-  A.ntx = ntx;
+  A.shape = S;
   A.ntiles = ntiles;
   A.nsub = nsub;
   A.nviews = g.num_views;
   A.tof = ntof > 1;
-  A.stride = std::max({need[0], need[1], (longest + 63) / 64 * 64});  // rows are written 64 lanes at a time
-  A.lead = std::max(A.stride, 64 * nslot);  // also the zeros that padding entries read
   A.longest = longest;
-  const int rows = (mi::kTileLdsBytes / 4 - A.lead - 64 * nslot) / A.stride;
+  int rows;
+  if (short_img) {
+    // rows end to end; a copy writes up to 63 floats past the last, and lanes
+    // beyond a line's planes read up to as many more
+    A.stride = std::max({need[0], need[1], 2});
+    A.lead = std::max(A.stride, 64);
+    A.buffer = mi::kShortLdsBytes / 8;
+    A.div_stride = static_cast<uint32_t>(((uint64_t{1} << 32) + A.stride - 1) / A.stride);
+    A.proj_bytes = static_cast<uint32_t>(4 * total_bins());
+    rows = (A.buffer - A.lead - 128) / A.stride;
+    A.lds_floats = 2 * A.buffer;
+  } else {
+    A.stride = std::max({need[0], need[1], (longest + 63) / 64 * 64});  // rows are written 64 lanes at a time
+    A.lead = std::max(A.stride, 64 * nslot);  // also the zeros that padding entries read
+    rows = (mi::kTileLdsBytes / 4 - A.lead - 64 * nslot) / A.stride;
+    A.lds_floats = mi::kTileLdsBytes / 4;
+  }
   if (rows < 24) return false;
-  A.lds_floats = mi::kTileLdsBytes / 4;
   // pass 2: phases
   const int64_t nst = static_cast<int64_t>(nsub) * ntiles;
   DBuf<uint32_t> slot, nphase, nrow, row_off, phase_row;
@@ -1306,7 +1326,7 @@ bool mi_ctx::build_tile_table(int span) {
   HIPCHECK(hipMemcpy(need, d_need.p, sizeof(need), hipMemcpyDeviceToHost));
   if (need[2]) return false;
   const uint32_t total_rows = totals[1];
-  const int64_t nph = totals[0], nlists = nph * mi::kTileCols;
+  const int64_t nph = totals[0], nlists = nph * S.lines();
   if (nlists >= (int64_t{1} << 31) - 2) return false;
   tile_row.alloc(static_cast<size_t>(total_rows) + mi::kTileRowSlack);
   HIPCHECK(hipMemsetAsync(tile_row.p + total_rows, 0, mi::kTileRowSlack * sizeof(int2), stream));
@@ -1324,7 +1344,7 @@ bool mi_ctx::build_tile_table(int span) {
     mi::launch_tile_count(fams.p, d_pos.p, plan->subset_family_begin(s), plan->subset_family_begin(s + 1), ntang, pool.p,
                           rec, tof_fp_w, ntof, s, dims, A, nunits, slot.p, counts.p, stream);
   groups.alloc(nlists + 1);
-  mi::launch_tile_groups(counts.p, nlists + 1, groups.p, d_need.p + 2, stream);
+  mi::launch_tile_groups(counts.p, nlists + 1, S.lockstep(), groups.p, d_need.p + 2, stream);
   HIPCHECK(hipGetLastError());
   scan(groups, group_off, nlists + 1);
   counts.release();
@@ -1333,7 +1353,7 @@ bool mi_ctx::build_tile_table(int span) {
   const int64_t nslots = 4 * static_cast<int64_t>(totals[1]);
   if (need[2]) return false;
   tile_hdr.alloc((nph + mi::kTileHdrSlack) * mi::kTileWaves);
-  mi::launch_tile_headers(groups.p, group_off.p, phase_row.p, total_rows, nph, tile_hdr.p, stream);
+  mi::launch_tile_headers(groups.p, group_off.p, phase_row.p, total_rows, nph, S, tile_hdr.p, stream);
   // pass 4, subset by subset: every term's list and entry, sorted by list, to
   // its place
   DBuf<int64_t> d_fam_off;
@@ -1367,7 +1387,7 @@ bool mi_ctx::build_tile_table(int span) {
                            span, d_fam_off.p, fam_off[fb], keys_in.p, raw.p, stream);
       HIPCHECK(mi::radix_sort_pairs(tmp.p, tb, keys_in.p, keys_out.p, vals_in.p, vals_out.p, static_cast<int>(m), end_bit,
                                     stream));
-      mi::launch_tile_place(keys_out.p, vals_out.p, raw.p, group_off.p, none, m, tile_off.p, tile_w.p, stream);
+      mi::launch_tile_place(keys_out.p, vals_out.p, raw.p, group_off.p, none, S.lockstep(), m, tile_off.p, tile_w.p, stream);
     }
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipStreamSynchronize(stream));
@@ -1376,7 +1396,7 @@ bool mi_ctx::build_tile_table(int span) {
   // workgroups to run are short ones
   DBuf<uint32_t> d_work;
   d_work.alloc(ntiles);
-  mi::launch_tile_work(group_off.p, tile_phase_off.p, nsub, ntiles, d_work.p, stream);
+  mi::launch_tile_work(group_off.p, tile_phase_off.p, nsub, ntiles, S.lines(), d_work.p, stream);
   std::vector<uint32_t> work(ntiles);
   HIPCHECK(hipMemcpyAsync(work.data(), d_work.p, d_work.bytes(), hipMemcpyDeviceToHost, stream));
   HIPCHECK(hipStreamSynchronize(stream));

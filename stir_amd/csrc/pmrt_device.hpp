@@ -342,41 +342,58 @@ void launch_back_project_slab(BpMode mode, const SlabArgs& A, int subset_begin, 
 
 // ---- back projection by image tiles with the runs in LDS (pmrt_tile.hip):
 // tables whose families cover whole runs (z-shift symmetry)
-constexpr int kTileSide = 8;          // a tile is 8 x 8 image columns
-constexpr int kTileCols = kTileSide * kTileSide;
-constexpr int kTileWaves = 8;
+constexpr int kTileWaves = 8;         // waves that add entries, of either kernel
+// images of more than kTileShortPlanes planes: tiles of 64 columns
+constexpr int kTileCols = 64;
 constexpr int kTileLdsBytes = 53760;  // LDS of a workgroup: three share the CU's 160 KB
-static_assert(kTileLdsBytes <= 65536, "more needs the kernels' dynamic LDS limit raised");
+// shorter images: several lines share a wave
+constexpr int kTileShortPlanes = 32;
+constexpr int kShortCopyWaves = 4;     // waves of a workgroup that copy rows
+constexpr int kShortLdsBytes = 65536;  // two buffers
+static_assert(kTileLdsBytes <= 65536 && kShortLdsBytes <= 65536, "more needs the kernels' dynamic LDS limit raised");
+// A line is the planes of a column that one list of entries reaches: all, or
+// (par 2) those of one parity.
+struct TileShape {
+  int tx, ty, par, ntx;  // columns of a tile, lines per column, tiles in x
+  int lanes;             // of a line: 64, or less in the kernel for short images
+  __host__ __device__ int lines() const { return tx * ty * par; }
+  __host__ __device__ int lines_of_wave() const { return lines() / kTileWaves; }
+  __host__ __device__ int lockstep() const { return lanes < 64 ? lines_of_wave() : 1; }  // lines whose lists are as long
+};
 constexpr int kTileXcdChunk = 1;      // tiles of one XCD's turn
 constexpr int kTileHdrSlack = 3;      // phases that the kernel's header read-ahead may touch past the last
-constexpr int kTileEntSlack = 64;     // entries that its chunk read-ahead may touch past the last
+constexpr int kTileEntSlack = 512;    // entries that its chunk read-ahead may touch past the last
 constexpr int kTileRowSlack = 64 * kTileWaves;  // rows that its read-ahead may touch past the last
 struct TileArgs {
   const uint32_t* phase_off;  // first phase of every (tile, subset)
-  const uint4* hdr;           // per (phase, wave): first group, groups of its columns (8 bytes), first row
-  const int2* row;            // LDS rows: the run's device offset, nax | ppa << 16
+  const uint4* hdr;           // per (phase, wave): first group, groups of its 8 columns (a byte each) or, in
+                              // lockstep, of each of its lines, first row
+  const int2* row;            // LDS rows: the run's device offset, nax | ppa << 16 (ppa: of a line)
   const int32_t* off;         // entries: LDS byte offset of plane 0 in the run's row
   const float* w;             // entries: weight
   const int2* rng;            // per (tile, view, TOF bin): first and last tangential index (x > y: none)
   const int32_t* order;       // tiles in launch order
-  int ntx, ntiles, nsub, nviews;
+  TileShape shape;
+  int ntiles, nsub, nviews;
   int lead, stride, longest;  // floats: zeros before the first row, row pitch, longest run in planes
-  int lds_floats;
+  int lds_floats, buffer;     // floats: of the workgroup, of one buffer (short images)
+  uint32_t div_stride;        // ceil(2^32 / stride)
+  uint32_t proj_bytes;        // of the projection data (short images)
   bool tof;                   // entries are (element, TOF bin) terms
 };
 // The table's passes. d_fp_rec: null, or the stored forward TOF records (w
 // weights each): then every TOF bin of a (segment, view) is a unit of its own.
 void launch_tile_range(const Family* d_fams, const int2* d_fam_pos, int nfam, const int2* d_pool,
-                       const int32_t* d_fp_rec, int w, const ImageDims& dims, int ntx, int nviews, int ntof, int2* d_rng,
-                       int* d_need, hipStream_t stream);
+                       const int32_t* d_fp_rec, int w, const ImageDims& dims, const TileShape& shape, int nviews, int ntof,
+                       int2* d_rng, int* d_need, hipStream_t stream);
 void launch_tile_phases(const int4* d_units, const int32_t* d_unit_off, int nsub, int ntiles, int nunits, int nrng,
                         const int2* d_rng, int rows, uint32_t* d_slot, uint32_t* d_nphase, uint32_t* d_nrow, int* d_bad,
                         hipStream_t stream);
 void launch_tile_rows(const int4* d_units, const int32_t* d_unit_off, int nsub, int ntiles, int nunits, int nrng,
                       const int2* d_rng, int rows, const uint32_t* d_phase_off, const uint32_t* d_row_off, int2* d_row,
                       uint32_t* d_phase_row, int* d_bad, hipStream_t stream);
-void launch_tile_work(const uint32_t* d_group_off, const uint32_t* d_phase_off, int nsub, int ntiles, uint32_t* d_work,
-                      hipStream_t stream);
+void launch_tile_work(const uint32_t* d_group_off, const uint32_t* d_phase_off, int nsub, int ntiles, int lines,
+                      uint32_t* d_work, hipStream_t stream);
 void launch_tile_count(const Family* d_fams, const int2* d_fam_pos, int fam_begin, int fam_end, int ntang,
                        const int2* d_pool, const int32_t* d_fp_rec, int w, int ntof, int subset, const ImageDims& dims,
                        const TileArgs& A, int nunits, const uint32_t* d_slot, uint32_t* d_counts, hipStream_t stream);
@@ -384,11 +401,12 @@ void launch_tile_make(const Family* d_fams, const int2* d_fam_pos, int fam_begin
                       const int2* d_pool, const int32_t* d_fp_rec, int w, int ntof, int subset, const ImageDims& dims,
                       const TileArgs& A, int nunits, const uint32_t* d_slot, uint32_t none, int span,
                       const int64_t* d_fam_entry_off, int64_t first, uint32_t* d_keys, int2* d_raw, hipStream_t stream);
-void launch_tile_groups(const uint32_t* d_counts, int64_t n, uint32_t* d_groups, int* d_bad, hipStream_t stream);
+void launch_tile_groups(const uint32_t* d_counts, int64_t n, int lockstep, uint32_t* d_groups, int* d_bad,
+                        hipStream_t stream);
 void launch_tile_headers(const uint32_t* d_groups, const uint32_t* d_group_off, const uint32_t* d_phase_row,
-                         uint32_t total_rows, int64_t nphase, uint4* d_hdr, hipStream_t stream);
+                         uint32_t total_rows, int64_t nphase, const TileShape& shape, uint4* d_hdr, hipStream_t stream);
 void launch_tile_place(const uint32_t* d_keys, const uint32_t* d_idx, const int2* d_raw, const uint32_t* d_group_off,
-                       uint32_t none, int64_t n, int32_t* d_off, float* d_w, hipStream_t stream);
+                       uint32_t none, int lockstep, int64_t n, int32_t* d_off, float* d_w, hipStream_t stream);
 void launch_back_project_tile(BpMode mode, const TileArgs& A, int subset_begin, int subset_end, const float* d_proj,
                               float* d_img, const ImageDims& dims, const BpData& data, hipStream_t stream);
 

@@ -60,12 +60,13 @@ using namespace dev;
 
 constexpr int kTileCpw = kTileCols / kTileWaves;  // columns per wave
 
-// The matrix element of a family as the tile table sees it: tile, column of
-// the tile, plane of axial position 0; false when it reaches no image plane.
+// The matrix element of a family as the tile table sees it: tile, line of the
+// tile, the line's plane of axial position 0; false when it reaches no image
+// plane.
 struct TileElem {
   int t, c, k;
 };
-__device__ inline bool tile_elem(const Family& f, int coords, const ImageDims& d, int ntx, TileElem& E) {
+__device__ inline bool tile_elem(const Family& f, int coords, const ImageDims& d, const TileShape& S, TileElem& E) {
   int x, y, z, xo, yo;
   decode(coords, x, y, z);
   inplane_any_op(f.inplane, x, y, xo, yo);
@@ -73,8 +74,12 @@ __device__ inline bool tile_elem(const Family& f, int coords, const ImageDims& d
   E.k = f.zsign * z + f.zadd0 - d.min_z;
   const int last = E.k + f.ppa * (f.nax - 1);
   if (cx < 0 || cx >= d.nx || cy < 0 || cy >= d.ny || last < 0 || E.k >= d.nz) return false;
-  E.t = (cy / kTileSide) * ntx + cx / kTileSide;
-  E.c = (cy % kTileSide) * kTileSide + cx % kTileSide;
+  E.t = (cy / S.ty) * S.ntx + cx / S.tx;
+  E.c = (cy % S.ty) * S.tx + cx % S.tx;
+  if (S.par == 2) {
+    E.c = 2 * E.c + (E.k & 1);
+    E.k >>= 1;
+  }
   return true;
 }
 
@@ -100,7 +105,7 @@ __global__ void __launch_bounds__(kWave) tile_range_kernel(const Family* __restr
                                                            const int2* __restrict__ fam_pos, int nfam,
                                                            const int2* __restrict__ pool,
                                                            const int32_t* __restrict__ fp_rec, int W, ImageDims d,
-                                                           int ntx, int nviews, int ntof, int2* __restrict__ rng,
+                                                           TileShape S, int nviews, int ntof, int2* __restrict__ rng,
                                                            int* __restrict__ need) {
   const int fi = blockIdx.x;
   if (fi >= nfam) return;
@@ -112,11 +117,11 @@ __global__ void __launch_bounds__(kWave) tile_range_kernel(const Family* __restr
     const int e = e0 + lane;
     TileElem E;
     const int64_t pi = static_cast<int64_t>(f.row_start) + (e < f.row_len ? e : 0);
-    const bool ok = e < f.row_len && tile_elem(f, pool[pi].x, d, ntx, E);
+    const bool ok = e < f.row_len && tile_elem(f, pool[pi].x, d, S, E);
     uint32_t bins = 0;  // the element's TOF bins
     if (ok) {
-      after = max(after, d.nz - E.k);
-      before = max(before, f.ppa * (f.nax - 1) + 1 + E.k);
+      after = max(after, (d.nz + S.par - 1) / S.par - E.k);
+      before = max(before, f.ppa / S.par * (f.nax - 1) + 1 + E.k);
       element_terms(fp_rec, W, pi, 0, [&](int bin, int) { bins |= 1U << bin; });
     }
     // neighbouring elements of a row lie mostly in one tile and the same bins:
@@ -164,7 +169,7 @@ __global__ void tile_phase_kernel(const int4* __restrict__ units, const int32_t*
   int ph = -1, used = 0, prev = 0;
   uint32_t n = 0;
   for (int u = unit_off[s]; u < unit_off[s + 1]; ++u) {
-    const int4 U = units[u];  // device offset, nax, ppa, index among the tile's ranges
+    const int4 U = units[u];  // device offset, nax, ppa (of a line), index among the tile's ranges
     const int2 r = rng[static_cast<int64_t>(t) * nrng + U.w];
     const int T = r.y - r.x + 1;
     if (r.y < r.x) continue;
@@ -219,11 +224,11 @@ __global__ void __launch_bounds__(kWave) tile_entries_kernel(const Family* __res
     const int2 el = pool[pi];
     TileElem E;
     int n = 0;
-    if (tile_elem(f, el.x, d, A.ntx, E))
+    if (tile_elem(f, el.x, d, A.shape, E))
       element_terms(fp_rec, W, pi, el.y, [&](int bin, int weight) {
         const uint32_t sl = slot[static_cast<int64_t>(E.t) * nunits + unit + bin];
         const uint32_t ph = A.phase_off[static_cast<int64_t>(E.t) * A.nsub + subset] + (sl >> 16);
-        const uint32_t key = ph * kTileCols + E.c;
+        const uint32_t key = ph * A.shape.lines() + E.c;
         if (COUNT) {
           atomicAdd(&counts[key], 1U);
         } else {
@@ -239,22 +244,28 @@ __global__ void __launch_bounds__(kWave) tile_entries_kernel(const Family* __res
   }
 }
 
-// groups of 4 entries of every list
-__global__ void tile_groups_kernel(const uint32_t* __restrict__ counts, int64_t n, uint32_t* __restrict__ groups,
-                                   int* __restrict__ bad) {
+// groups of 4 entries of every list: of lists in lockstep the most of them
+__global__ void tile_groups_kernel(const uint32_t* __restrict__ counts, int64_t n, int lockstep,
+                                   uint32_t* __restrict__ groups, int* __restrict__ bad) {
   for (int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; i < n;
        i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-    groups[i] = (counts[i] + 3) / 4;
-    if (groups[i] > 255) *bad = 1;
+    uint32_t g = (counts[i] + 3) / 4;
+    if (lockstep > 1) {
+      const int64_t first = i / lockstep * lockstep;
+      for (int64_t j = first; j < first + lockstep && j < n; ++j) g = max(g, (counts[j] + 3) / 4);
+    }
+    groups[i] = g;
+    if (g > 255 && lockstep == 1) *bad = 1;
   }
 }
 
 // per (phase, wave): first group, the group counts of its columns (one byte
-// each) and the phase's first row; `slack` more phases without groups close
-// the list
+// each) or of its lines in lockstep, and the phase's first row; `slack` more
+// phases without groups close the list
 __global__ void tile_headers_kernel(const uint32_t* __restrict__ groups, const uint32_t* __restrict__ group_off,
                                     const uint32_t* __restrict__ phase_row, uint32_t total_rows, int64_t nphase,
-                                    int64_t slack, uint4* __restrict__ hdr) {
+                                    int64_t slack, TileShape S, uint4* __restrict__ hdr) {
+  const int lw = S.lines_of_wave();
   for (int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; i < (nphase + slack) * kTileWaves;
        i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
     const int64_t p = i / kTileWaves;
@@ -263,25 +274,27 @@ __global__ void tile_headers_kernel(const uint32_t* __restrict__ groups, const u
       continue;
     }
     uint32_t c[2] = {0, 0};
-    for (int j = 0; j < kTileCpw; ++j) c[j / 4] |= groups[i * kTileCpw + j] << (8 * (j % 4));
-    hdr[i] = make_uint4(group_off[i * kTileCpw], c[0], c[1], phase_row[p]);
+    if (S.lockstep() > 1) c[0] = groups[i * lw];
+    else
+      for (int j = 0; j < kTileCpw; ++j) c[j / 4] |= groups[i * lw + j] << (8 * (j % 4));
+    hdr[i] = make_uint4(group_off[i * lw], c[0], c[1], phase_row[p]);
   }
 }
 
 // groups of every tile (its work)
 __global__ void tile_work_kernel(const uint32_t* __restrict__ group_off, const uint32_t* __restrict__ phase_off, int nsub,
-                                 int ntiles, uint32_t* __restrict__ work) {
+                                 int ntiles, int lines, uint32_t* __restrict__ work) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= ntiles) return;
   const int64_t a = phase_off[static_cast<int64_t>(t) * nsub], b = phase_off[static_cast<int64_t>(t + 1) * nsub];
-  work[t] = group_off[b * kTileCols] - group_off[a * kTileCols];
+  work[t] = group_off[b * lines] - group_off[a * lines];
 }
 
-// sorted term r -> its place: 4 x its list's first group + its rank in the
-// list (a list has a few tens of entries)
+// sorted term r -> its place: the groups of a list follow one another, those
+// of lists in lockstep alternate (a list has a few tens of entries)
 __global__ void tile_place_kernel(const uint32_t* __restrict__ keys, const uint32_t* __restrict__ idx,
                                   const int2* __restrict__ raw, const uint32_t* __restrict__ group_off, uint32_t none,
-                                  int64_t n, int32_t* __restrict__ off, float* __restrict__ w) {
+                                  int lockstep, int64_t n, int32_t* __restrict__ off, float* __restrict__ w) {
   for (int64_t r = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; r < n;
        r += static_cast<int64_t>(gridDim.x) * blockDim.x) {
     const uint32_t key = keys[r];
@@ -289,7 +302,8 @@ __global__ void tile_place_kernel(const uint32_t* __restrict__ keys, const uint3
     int64_t rank = 0;
     while (rank < r && keys[r - rank - 1] == key) ++rank;
     const int2 E = raw[idx[r]];
-    const int64_t at = 4 * static_cast<int64_t>(group_off[key]) + rank;
+    const uint32_t line = key % lockstep;
+    const int64_t at = 4 * (group_off[key - line] + rank / 4 * lockstep + line) + rank % 4;
     off[at] = E.x;
     w[at] = __int_as_float(E.y);
   }
@@ -460,11 +474,12 @@ __global__ void __launch_bounds__(kWave* kTileWaves) bp_tile_kernel(TileArgs A, 
       for (int q = 0; q < NSLOT; ++q) acc[c][q] += sum[c][q];
   }
 #endif
-  const int x0 = (t % A.ntx) * kTileSide, y0 = (t / A.ntx) * kTileSide;
+  const TileShape& S = A.shape;
+  const int x0 = (t % S.ntx) * S.tx, y0 = (t / S.ntx) * S.ty;
 #pragma unroll
   for (int c = 0; c < kTileCpw; ++c) {
     const int cc = wave * kTileCpw + c;
-    const int cx = x0 + cc % kTileSide, cy = y0 + cc / kTileSide;
+    const int cx = x0 + cc % S.tx, cy = y0 + cc / S.tx;
     if (cx >= d.nx || cy >= d.ny) continue;
     const int col = cy * d.nx + cx;
 #pragma unroll
@@ -485,6 +500,289 @@ __global__ void __launch_bounds__(kWave* kTileWaves) bp_tile_kernel(TileArgs A, 
   }
 }
 
+// ---- short images
+//
+// A wave holds 64 / LPC lines of LPC lanes, LPC >= the planes of a line: an
+// image of up to 16 or 32 planes. With two planes per axial position (span 1)
+// an entry reaches the planes of one parity, so each parity is a line of its
+// own, its planes l of [0, LPC) the image's PAR l + parity, and the rows need
+// no zeros between. One wave has one set of lines, whose lists are padded to
+// the same length.
+//
+// What bounds it: with short lines the rows are short too (8 floats for 8
+// rings) and a phase has hundreds of them, so that copying them takes about as
+// long as adding the entries. Copy waves fill one buffer while the others read
+// the other; a copy wave's lanes cover the rows end to end (64 lanes write 64
+// consecutive floats), each with its own address from the row list.
+//
+// Measured, all subsets, against the column kernels: 8 rings, span 1, 128^2
+// columns 182 -> 34 us, 256^2 and all ring differences 2670 -> 475; 8 rings,
+// span 3, 69 -> 28; 16 rings, span 1, 1755 -> 460; span 3, 734 -> 443; 4 rings,
+// 64^2, 48 -> 17 us. Without the additions it takes as long: requests to memory
+// bound it (copies by 4-byte lanes, entries of 8 bytes). Lists of lines in
+// lockstep alternate by groups, so that one load covers 128 bytes of entries
+// and not pieces of 16 (8 rings, 256^2: 585 -> 507 us); the steps from copy to
+// copy by a carry instead of a division: 507 -> 475. 8 copy waves: the same.
+
+template <int CTRL>
+__device__ inline int dpp_all(int v) { return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true); }
+
+// acc + lane J's w of the quad times p (see add_bcast)
+template <int J>
+__device__ inline void add_quad(float& acc, int w, float p) {
+  if constexpr (J == 0)
+    asm("s_nop 1\n\tv_fmac_f32_dpp %0, %1, %2 quad_perm:[0,0,0,0] row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(w), "v"(p));
+  else if constexpr (J == 1)
+    asm("v_fmac_f32_dpp %0, %1, %2 quad_perm:[1,1,1,1] row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(w), "v"(p));
+  else if constexpr (J == 2)
+    asm("v_fmac_f32_dpp %0, %1, %2 quad_perm:[2,2,2,2] row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(w), "v"(p));
+  else
+    asm("v_fmac_f32_dpp %0, %1, %2 quad_perm:[3,3,3,3] row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(w), "v"(p));
+}
+
+// N groups of four entries of every line of the wave (each quad of lanes holds
+// its line's), all reads in flight before the first is waited for
+template <int N>
+__device__ inline void short_groups(const int* off, const int* w, const char* lds, int lane4, float& acc) {
+  float v[N][4];
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    v[j][0] = *reinterpret_cast<const float*>(lds + (lane4 + dpp_all<0x00>(off[j])));
+    v[j][1] = *reinterpret_cast<const float*>(lds + (lane4 + dpp_all<0x55>(off[j])));
+    v[j][2] = *reinterpret_cast<const float*>(lds + (lane4 + dpp_all<0xaa>(off[j])));
+    v[j][3] = *reinterpret_cast<const float*>(lds + (lane4 + dpp_all<0xff>(off[j])));
+  }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    add_quad<0>(acc, w[j], v[j][0]);
+    add_quad<1>(acc, w[j], v[j][1]);
+    add_quad<2>(acc, w[j], v[j][2]);
+    add_quad<3>(acc, w[j], v[j][3]);
+  }
+}
+
+constexpr int kShortThreads = kWave * (kTileWaves + kShortCopyWaves);
+constexpr int kShortBatch = 8;  // row list entries of a copy wave requested together
+
+// SUM2: the sum of a phase is added to the voxel's sum as a whole (shorter
+// chains of additions); otherwise all terms one by one, as the column kernel
+// for one plane per axial position.
+template <int MODE, int LPC, int PAR, bool SUM2>
+__global__ void __launch_bounds__(kShortThreads, 6) bp_tile_short_kernel(TileArgs A, int sb, int se,
+                                                                      const float* __restrict__ proj,
+                                                                      float* __restrict__ img, ImageDims d, BpData data,
+                                                                      int chunk) {
+  extern __shared__ float tile_lds[];
+  const int b = xcd_chunk_remap(static_cast<int>(blockIdx.x), chunk);
+  if (b >= A.ntiles) return;
+  const int t = as_const(A.order)[b];
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
+  const int lane = static_cast<int>(threadIdx.x % kWave);
+  for (int i = threadIdx.x; i < 2 * A.lead; i += kShortThreads)
+    tile_lds[i < A.lead ? i : A.buffer + i - A.lead] = 0.F;
+  constexpr int NSET = 32 * PAR * LPC / (kTileWaves * kWave);  // sets of lines of a wave
+  float acc[NSET], sum[NSET];
+#pragma unroll
+  for (int s = 0; s < NSET; ++s) acc[s] = sum[s] = 0.F;
+#if defined(__HIP_DEVICE_COMPILE__)
+  const uint32_t p0 = as_const(A.phase_off)[static_cast<int64_t>(t) * A.nsub + sb];
+  const uint32_t p1 = as_const(A.phase_off)[static_cast<int64_t>(t) * A.nsub + se];
+  int zero = 0;
+  asm volatile("" : "+v"(zero));
+  const int cw = wave - kTileWaves;
+  const uint4* hp = A.hdr + static_cast<int64_t>(p0) * kTileWaves + zero;
+  if (cw >= 0) {
+    const __amdgpu_buffer_rsrc_t all =
+        __builtin_amdgcn_make_buffer_rsrc((void*)proj, static_cast<short>(0), static_cast<int>(A.proj_bytes), 0x00020000);
+    // Copy i of the wave takes the phase's floats (cw + kShortCopyWaves i) 64 to
+    // + 63; this lane's row and place in it go from copy to copy by a step and
+    // a carry. (Past the phase's last row a copy writes the next phase's floats
+    // into the buffer's slack.)
+    const int f0 = cw * kWave + lane;
+    const int row_first = static_cast<int>(__umulhi(static_cast<uint32_t>(f0), A.div_stride));
+    const int at_first = f0 - row_first * A.stride;
+    constexpr int kAdvance = kShortCopyWaves * kWave;
+    const int row_step = static_cast<int>(__umulhi(static_cast<uint32_t>(kAdvance), A.div_stride));
+    const int at_step = kAdvance - row_step * A.stride;
+    auto carry = [&](int& at) {  // at in [0, stride) again; whether it passed the end
+      at += at_step;
+      const bool over = at >= A.stride;
+      at -= over ? A.stride : 0;
+      return over;
+    };
+    int2 ra[kShortBatch], rb[kShortBatch];
+    int row = 0, row_at = 0, at = 0;  // of the next request, of the next copy
+    auto request = [&](int2 (&r)[kShortBatch], uint32_t base) {
+      const int2* list = A.row + base;
+#pragma unroll
+      for (int j = 0; j < kShortBatch; ++j) {
+        r[j] = list[row];
+        row += row_step + carry(row_at);
+      }
+    };
+    auto copy = [&](const int2 (&r)[kShortBatch], int first, int n, float* buf) {
+#pragma unroll
+      for (int j = 0; j < kShortBatch; ++j) {
+        const int f = (cw + kShortCopyWaves * (first + j)) * kWave;
+        if (f < n) {
+          const int nax = r[j].y & 0xffff, ppa = r[j].y >> 16;
+          int a = at;
+          bool ok = true;
+          if (PAR == 1 && ppa > 1) {
+            a = at / ppa;
+            ok = a * ppa == at;
+          }
+          ok = ok && a < nax;
+          const int v = ok ? static_cast<int>(4U * static_cast<unsigned>(r[j].x + a)) : -4;  // -4: reads 0
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(all, (__attribute__((address_space(3))) void*)(buf + f), 4,
+                                                   whole_offset(v), 0, 0, 0);
+          carry(at);
+        }
+      }
+    };
+    uint32_t row0 = hp[0].w, row1 = hp[kTileWaves].w;
+    int nrow = static_cast<int>(__builtin_amdgcn_readfirstlane(row1) - __builtin_amdgcn_readfirstlane(row0));
+    row = row_first;
+    row_at = at_first;
+    request(ra, row0);
+    int which = 0;
+    for (uint32_t p = p0; p <= p1; ++p) {
+      if (p < p1) {
+        float* buf = tile_lds + A.lead + which * A.buffer;
+        which ^= 1;
+        const int n = nrow * A.stride;
+        auto any = [&](int first) { return (cw + kShortCopyWaves * first) * kWave < n; };
+        at = at_first;
+        for (int first = 0; any(first); first += 2 * kShortBatch) {
+          const bool second = any(first + kShortBatch);
+          if (second) request(rb, row0);
+          copy(ra, first, n, buf);
+          if (any(first + 2 * kShortBatch)) request(ra, row0);
+          if (second) copy(rb, first + kShortBatch, n, buf);
+        }
+        // the next phase's first batch
+        hp += kTileWaves;
+        row0 = row1;
+        row1 = hp[kTileWaves].w;
+        nrow = static_cast<int>(__builtin_amdgcn_readfirstlane(row1) - __builtin_amdgcn_readfirstlane(row0));
+        row = row_first;
+        row_at = at_first;
+        request(ra, row0);
+        __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's rows are in LDS
+      }
+      __syncthreads();
+    }
+    return;
+  }
+  const char* lds = reinterpret_cast<const char*>(tile_lds);
+  const int lane4 = 4 * (lane % LPC);
+  // The wave's entries are one stream over the phases, requested kRing chunks
+  // of four groups ahead (they come from memory, and a phase has only a few
+  // chunks). Lane i holds the header of phase q0 + i. The loop below has no
+  // load behind a branch: the compiler counts the loads in flight, and would
+  // wait for all of them where it cannot.
+  constexpr int kRing = 2, kLast = 8, kEnd = 16;
+  constexpr int kStep = 16 * NSET * kWave / LPC;  // bytes of a group of all the wave's lines
+  struct Chunk {
+    int o[NSET][4], w[NSET][4], info;  // info: groups, last of its phase, end of the stream
+  } ring[kRing];
+  int which = 0;
+  bool first_block = true;
+  for (uint32_t q0 = p0; q0 < p1; q0 += kWave) {
+    const uint32_t q1 = min(q0 + kWave, p1);
+    // (the header of phase p1 exists, of the next tile or the table's slack)
+    const uint4 hq = A.hdr[static_cast<int64_t>(min(q0 + lane, q1)) * kTileWaves + wave + zero];
+    uint32_t fp = q0;
+    int fleft = 0;
+    const char *po = nullptr, *pw = nullptr;
+    unsigned at[NSET];
+    auto phase = [&] {  // the phase fp: its first group and groups left
+      const uint32_t first = __builtin_amdgcn_readlane(hq.x, fp - q0);
+      fleft = __builtin_amdgcn_readlane(hq.y, fp - q0);
+      po = reinterpret_cast<const char*>(A.off + 4 * static_cast<int64_t>(first));
+      pw = reinterpret_cast<const char*>(A.w + 4 * static_cast<int64_t>(first));
+#pragma unroll
+      for (int s = 0; s < NSET; ++s) at[s] = 16 * (s * (kWave / LPC) + lane / LPC) + 4 * (lane % 4);
+    };
+    auto fetch = [&](Chunk& c) {
+      c.info = fp >= q1 ? kEnd : min(fleft, 4);
+#pragma unroll
+      for (int s = 0; s < NSET; ++s)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {  // past the stream's end its last chunk again
+          c.o[s][j] = entry_word(po, at[s] + kStep * j);
+          c.w[s][j] = entry_word(pw, at[s] + kStep * j);
+        }
+      if (fp < q1) {
+        fleft -= 4;
+        if (fleft <= 0) {
+          c.info |= kLast;
+          if (++fp < q1) phase();
+        } else {
+#pragma unroll
+          for (int s = 0; s < NSET; ++s) at[s] += 4 * kStep;
+        }
+      }
+    };
+    phase();
+#pragma unroll
+    for (int r = 0; r < kRing; ++r) fetch(ring[r]);
+    if (first_block) __syncthreads();  // the first phase's rows are there (and the leading zeros)
+    first_block = false;
+    while (ring[0].info != kEnd) {  // (chunks past the end: no groups)
+#pragma unroll
+      for (int r = 0; r < kRing; ++r) {
+        Chunk& c = ring[r];
+        const int n = c.info & 7;
+        if (n == 4) {
+#pragma unroll
+          for (int s = 0; s < NSET; ++s) short_groups<4>(c.o[s], c.w[s], lds, lane4, acc[s]);
+        } else {
+#pragma unroll
+          for (int j = 0; j < 3; ++j)
+            if (n > j) {
+#pragma unroll
+              for (int s = 0; s < NSET; ++s) short_groups<1>(c.o[s] + j, c.w[s] + j, lds, lane4, acc[s]);
+            }
+        }
+        if (c.info & kLast) {
+          if constexpr (SUM2) {
+#pragma unroll
+            for (int s = 0; s < NSET; ++s) {
+              sum[s] += acc[s];
+              acc[s] = 0.F;
+            }
+          }
+          which ^= 1;
+          lds = reinterpret_cast<const char*>(tile_lds + which * A.buffer);
+          __syncthreads();
+        }
+        fetch(c);
+      }
+    }
+  }
+  if (first_block) __syncthreads();
+#endif
+  const TileShape& S = A.shape;
+#pragma unroll
+  for (int s = 0; s < NSET; ++s) {
+    const int ln = (wave * NSET + s) * (kWave / LPC) + lane / LPC;
+    const int cc = ln / PAR, z = PAR * (lane % LPC) + ln % PAR;
+    const int cx = (t % S.ntx) * S.tx + cc % S.tx, cy = (t / S.ntx) * S.ty + cc / S.tx;
+    if (cx >= d.nx || cy >= d.ny || z >= d.nzp) continue;
+    const int64_t idx = static_cast<int64_t>(cy * d.nx + cx) * d.nzp + z;
+    const float v = SUM2 ? sum[s] : acc[s];
+    if constexpr (MODE == BP_PLAIN) {
+      as_global(img)[idx] = z < d.nz ? v : 0.F;
+    } else if (z < d.nz) {
+      const float u = osem_factor(v, as_const(data.sens)[idx], data.threshold, data.thr_lo, data.thr_hi);
+      as_global(data.estimate)[idx] = as_global(data.estimate)[idx] * u;
+      if (data.update) as_global(data.update)[idx] = u;
+    }
+  }
+}
+
 unsigned grid_of(int64_t n) {
   int64_t b = (n + 255) / 256;
   if (b > 65536) b = 65536;
@@ -495,11 +793,11 @@ unsigned grid_of(int64_t n) {
 }  // namespace
 
 void launch_tile_range(const Family* d_fams, const int2* d_fam_pos, int nfam, const int2* d_pool,
-                       const int32_t* d_fp_rec, int w, const ImageDims& dims, int ntx, int nviews, int ntof, int2* d_rng,
-                       int* d_need, hipStream_t stream) {
+                       const int32_t* d_fp_rec, int w, const ImageDims& dims, const TileShape& shape, int nviews, int ntof,
+                       int2* d_rng, int* d_need, hipStream_t stream) {
   if (nfam <= 0) return;
   hipLaunchKernelGGL(tile_range_kernel, dim3(nfam), dim3(kWave), 0, stream, d_fams, d_fam_pos, nfam, d_pool, d_fp_rec, w,
-                     dims, ntx, nviews, ntof, d_rng, d_need);
+                     dims, shape, nviews, ntof, d_rng, d_need);
 }
 
 void launch_tile_phases(const int4* d_units, const int32_t* d_unit_off, int nsub, int ntiles, int nunits, int nrng,
@@ -537,28 +835,29 @@ void launch_tile_make(const Family* d_fams, const int2* d_fam_pos, int fam_begin
                      span, d_fam_entry_off, first, d_keys, d_raw);
 }
 
-void launch_tile_groups(const uint32_t* d_counts, int64_t n, uint32_t* d_groups, int* d_bad, hipStream_t stream) {
-  hipLaunchKernelGGL(tile_groups_kernel, dim3(grid_of(n)), dim3(256), 0, stream, d_counts, n, d_groups, d_bad);
+void launch_tile_groups(const uint32_t* d_counts, int64_t n, int lockstep, uint32_t* d_groups, int* d_bad,
+                        hipStream_t stream) {
+  hipLaunchKernelGGL(tile_groups_kernel, dim3(grid_of(n)), dim3(256), 0, stream, d_counts, n, lockstep, d_groups, d_bad);
 }
 
 void launch_tile_headers(const uint32_t* d_groups, const uint32_t* d_group_off, const uint32_t* d_phase_row,
-                         uint32_t total_rows, int64_t nphase, uint4* d_hdr, hipStream_t stream) {
+                         uint32_t total_rows, int64_t nphase, const TileShape& shape, uint4* d_hdr, hipStream_t stream) {
   const int64_t n = (nphase + kTileHdrSlack) * kTileWaves;
   hipLaunchKernelGGL(tile_headers_kernel, dim3(grid_of(n)), dim3(256), 0, stream, d_groups, d_group_off, d_phase_row,
-                     total_rows, nphase, int64_t{kTileHdrSlack}, d_hdr);
+                     total_rows, nphase, int64_t{kTileHdrSlack}, shape, d_hdr);
 }
 
-void launch_tile_work(const uint32_t* d_group_off, const uint32_t* d_phase_off, int nsub, int ntiles, uint32_t* d_work,
-                      hipStream_t stream) {
+void launch_tile_work(const uint32_t* d_group_off, const uint32_t* d_phase_off, int nsub, int ntiles, int lines,
+                      uint32_t* d_work, hipStream_t stream) {
   hipLaunchKernelGGL(tile_work_kernel, dim3((ntiles + 255) / 256), dim3(256), 0, stream, d_group_off, d_phase_off, nsub,
-                     ntiles, d_work);
+                     ntiles, lines, d_work);
 }
 
 void launch_tile_place(const uint32_t* d_keys, const uint32_t* d_idx, const int2* d_raw, const uint32_t* d_group_off,
-                       uint32_t none, int64_t n, int32_t* d_off, float* d_w, hipStream_t stream) {
+                       uint32_t none, int lockstep, int64_t n, int32_t* d_off, float* d_w, hipStream_t stream) {
   if (n <= 0) return;
   hipLaunchKernelGGL(tile_place_kernel, dim3(grid_of(n)), dim3(256), 0, stream, d_keys, d_idx, d_raw, d_group_off, none,
-                     n, d_off, d_w);
+                     lockstep, n, d_off, d_w);
 }
 
 void launch_back_project_tile(BpMode mode, const TileArgs& A, int subset_begin, int subset_end, const float* d_proj,
@@ -567,6 +866,29 @@ void launch_back_project_tile(BpMode mode, const TileArgs& A, int subset_begin, 
   const int chunk = kTileXcdChunk, round = kNumXcd * chunk;
   const dim3 grid((A.ntiles + round - 1) / round * round), block(kWave * kTileWaves);
   const size_t lds = static_cast<size_t>(A.lds_floats) * sizeof(float);
+  if (A.shape.lanes < kWave) {
+    // one plane per axial position (and mixed ones): the column kernel's order
+    // of additions, bit for bit
+#define MI_SHORT(M, L, P, S2)                                                                                          \
+  hipLaunchKernelGGL((bp_tile_short_kernel<M, L, P, S2>), grid, dim3(kShortThreads), lds, stream, A, subset_begin,     \
+                     subset_end, d_proj, d_img, dims, data, chunk)
+#define MI_SHORT_S(M)                                        \
+  if (A.shape.par == 2) {                                    \
+    if (A.shape.lanes == 8) MI_SHORT(M, 8, 2, true);         \
+    else MI_SHORT(M, 16, 2, true);                           \
+  } else if (A.tof) {                                        \
+    if (A.shape.lanes == 16) MI_SHORT(M, 16, 1, true);       \
+    else MI_SHORT(M, 32, 1, true);                           \
+  } else {                                                   \
+    if (A.shape.lanes == 16) MI_SHORT(M, 16, 1, false);      \
+    else MI_SHORT(M, 32, 1, false);                          \
+  }
+    if (mode == BP_PLAIN) { MI_SHORT_S(BP_PLAIN) }
+    else { MI_SHORT_S(BP_OSEM_UPDATE) }
+#undef MI_SHORT_S
+#undef MI_SHORT
+    return;
+  }
 #define MI_TILE(M, S, T)                                                                                          \
   hipLaunchKernelGGL((bp_tile_kernel<M, S, T>), grid, block, lds, stream, A, subset_begin, subset_end, d_proj, d_img, \
                      dims, data, chunk)
