@@ -11,6 +11,7 @@
 #include <stdexcept>
 #include <string>
 #include <unordered_map>
+#include <deque>
 #include <vector>
 
 #include "pmrt_device.hpp"
@@ -89,6 +90,24 @@ struct DBuf {
     n = count;
   }
   size_t bytes() const { return n * sizeof(T); }
+};
+// Device memory for the steps of a set-up, in blocks freed together at its
+// end: an allocation and a free cost 0.1 ms, and a table takes twenty of them.
+struct Arena {
+  std::deque<DBuf<char>> blocks;
+  size_t used = 0;
+  template <class T>
+  T* get(size_t count) {
+    const size_t bytes = (count * sizeof(T) + 255) / 256 * 256;
+    if (blocks.empty() || used + bytes > blocks.back().n) {
+      blocks.emplace_back();
+      blocks.back().alloc(std::max(bytes, size_t{32} << 20));
+      used = 0;
+    }
+    T* p = reinterpret_cast<T*>(blocks.back().p + used);
+    used += bytes;
+    return p;
+  }
 };
 
 }  // namespace
@@ -1251,27 +1270,25 @@ bool mi_ctx::build_tile_table(int span) {
     const int64_t bytes = 10 * n * span + 32 * most + 4 * (static_cast<int64_t>(ntiles) * nunits);
     if (bytes > static_cast<int64_t>(free_b / 4 * 3)) return false;
   }
-  auto upload = [&](auto& buf, const auto& v) {
-    buf.alloc(v.size());
-    HIPCHECK(hipMemcpyAsync(buf.p, v.data(), buf.bytes(), hipMemcpyHostToDevice, stream));
+  Arena mem;
+  auto upload = [&](const auto& v) {
+    auto* d = mem.get<typename std::decay_t<decltype(v)>::value_type>(v.size());
+    HIPCHECK(hipMemcpyAsync(d, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice, stream));
+    return d;
   };
-  DBuf<int4> d_units;
-  DBuf<int2> d_pos;
-  DBuf<int32_t> d_unit_off;
-  upload(d_units, hunits);
-  upload(d_pos, hpos);
-  upload(d_unit_off, hunit_off);
+  const int4* d_units = upload(hunits);
+  const int2* d_pos = upload(hpos);
+  const int32_t* d_unit_off = upload(hunit_off);
   // pass 1: tangential ranges and the zeros a row needs
   tile_rng.alloc(static_cast<size_t>(ntiles) * nrng);
   mi::launch_fill_int2(tile_rng.p, static_cast<int64_t>(tile_rng.n), make_int2(0x7fffffff, -1), stream);
-  DBuf<int> d_need;  // planes after a run's start, planes up to its end, flag
-  d_need.alloc(3);
-  HIPCHECK(hipMemsetAsync(d_need.p, 0, d_need.bytes(), stream));
-  mi::launch_tile_range(fams.p, d_pos.p, nfam, pool.p, rec, tof_fp_w, dims, S, g.num_views, ntof, tile_rng.p, d_need.p,
+  int need[3];
+  int* d_need = mem.get<int>(3);  // planes after a run's start, planes up to its end, flag
+  HIPCHECK(hipMemsetAsync(d_need, 0, sizeof(need), stream));
+  mi::launch_tile_range(fams.p, d_pos, nfam, pool.p, rec, tof_fp_w, dims, S, g.num_views, ntof, tile_rng.p, d_need,
                         stream);
   HIPCHECK(hipGetLastError());
-  int need[3];
-  HIPCHECK(hipMemcpyAsync(need, d_need.p, sizeof(need), hipMemcpyDeviceToHost, stream));
+  HIPCHECK(hipMemcpyAsync(need, d_need, sizeof(need), hipMemcpyDeviceToHost, stream));
   HIPCHECK(hipStreamSynchronize(stream));
   if (need[1] <= 0) return false;  // no element reaches the image
   mi::TileArgs A{};
@@ -1301,109 +1318,99 @@ bool mi_ctx::build_tile_table(int span) {
   if (rows < 24) return false;
   // pass 2: phases
   const int64_t nst = static_cast<int64_t>(nsub) * ntiles;
-  DBuf<uint32_t> slot, nphase, nrow, row_off, phase_row;
-  slot.alloc(static_cast<size_t>(ntiles) * nunits);
-  nphase.alloc(nst + 1);
-  nrow.alloc(nst + 1);
-  HIPCHECK(hipMemsetAsync(nphase.p + nst, 0, sizeof(uint32_t), stream));
-  HIPCHECK(hipMemsetAsync(nrow.p + nst, 0, sizeof(uint32_t), stream));
-  mi::launch_tile_phases(d_units.p, d_unit_off.p, nsub, ntiles, nunits, nrng, tile_rng.p, rows, slot.p, nphase.p, nrow.p,
-                         d_need.p + 2, stream);
-  auto scan = [&](const DBuf<uint32_t>& in, DBuf<uint32_t>& out, int64_t count) {  // counts, then the total
-    out.alloc(count);
+  uint32_t* slot = mem.get<uint32_t>(static_cast<size_t>(ntiles) * nunits);
+  uint32_t *nphase = mem.get<uint32_t>(nst + 1), *nrow = mem.get<uint32_t>(nst + 1);
+  uint32_t* row_off = mem.get<uint32_t>(nst + 1);
+  tile_phase_off.alloc(nst + 1);
+  HIPCHECK(hipMemsetAsync(nphase + nst, 0, sizeof(uint32_t), stream));
+  HIPCHECK(hipMemsetAsync(nrow + nst, 0, sizeof(uint32_t), stream));
+  mi::launch_tile_phases(d_units, d_unit_off, nsub, ntiles, nunits, nrng, tile_rng.p, rows, slot, nphase, nrow,
+                         d_need + 2, stream);
+  auto scan = [&](const uint32_t* in, uint32_t* out, int64_t count) {  // counts, then the total
     size_t tb = 0;
-    HIPCHECK(mi::exclusive_scan_u32(nullptr, tb, in.p, out.p, static_cast<int>(count), stream));
-    DBuf<char> tmp;
-    tmp.alloc(std::max<size_t>(tb, 1));
-    HIPCHECK(mi::exclusive_scan_u32(tmp.p, tb, in.p, out.p, static_cast<int>(count), stream));
+    HIPCHECK(mi::exclusive_scan_u32(nullptr, tb, in, out, static_cast<int>(count), stream));
+    char* tmp = mem.get<char>(std::max<size_t>(tb, 1));
+    HIPCHECK(mi::exclusive_scan_u32(tmp, tb, in, out, static_cast<int>(count), stream));
     HIPCHECK(hipStreamSynchronize(stream));
   };
-  scan(nphase, tile_phase_off, nst + 1);
+  scan(nphase, tile_phase_off.p, nst + 1);
   scan(nrow, row_off, nst + 1);
   uint32_t totals[2];
   HIPCHECK(hipMemcpy(&totals[0], tile_phase_off.p + nst, sizeof(uint32_t), hipMemcpyDeviceToHost));
-  HIPCHECK(hipMemcpy(&totals[1], row_off.p + nst, sizeof(uint32_t), hipMemcpyDeviceToHost));
-  HIPCHECK(hipMemcpy(need, d_need.p, sizeof(need), hipMemcpyDeviceToHost));
+  HIPCHECK(hipMemcpy(&totals[1], row_off + nst, sizeof(uint32_t), hipMemcpyDeviceToHost));
+  HIPCHECK(hipMemcpy(need, d_need, sizeof(need), hipMemcpyDeviceToHost));
   if (need[2]) return false;
   const uint32_t total_rows = totals[1];
   const int64_t nph = totals[0], nlists = nph * S.lines();
   if (nlists >= (int64_t{1} << 31) - 2) return false;
   tile_row.alloc(static_cast<size_t>(total_rows) + mi::kTileRowSlack);
   HIPCHECK(hipMemsetAsync(tile_row.p + total_rows, 0, mi::kTileRowSlack * sizeof(int2), stream));
-  phase_row.alloc(nph);
-  mi::launch_tile_rows(d_units.p, d_unit_off.p, nsub, ntiles, nunits, nrng, tile_rng.p, rows, tile_phase_off.p,
-                       row_off.p, tile_row.p, phase_row.p, d_need.p + 2, stream);
+  uint32_t* phase_row = mem.get<uint32_t>(nph);
+  mi::launch_tile_rows(d_units, d_unit_off, nsub, ntiles, nunits, nrng, tile_rng.p, rows, tile_phase_off.p,
+                       row_off, tile_row.p, phase_row, d_need + 2, stream);
   A.phase_off = tile_phase_off.p;
   A.row = tile_row.p;
   A.rng = tile_rng.p;
   // pass 3: entries per list, in groups of 4
-  DBuf<uint32_t> counts, groups, group_off;
-  counts.alloc(nlists + 1);
-  HIPCHECK(hipMemsetAsync(counts.p, 0, counts.bytes(), stream));
+  uint32_t *counts = mem.get<uint32_t>(nlists + 1), *groups = mem.get<uint32_t>(nlists + 1);
+  uint32_t* group_off = mem.get<uint32_t>(nlists + 1);
+  HIPCHECK(hipMemsetAsync(counts, 0, (nlists + 1) * sizeof(uint32_t), stream));
   for (int s = 0; s < nsub; ++s)
-    mi::launch_tile_count(fams.p, d_pos.p, plan->subset_family_begin(s), plan->subset_family_begin(s + 1), ntang, pool.p,
-                          rec, tof_fp_w, ntof, s, dims, A, nunits, slot.p, counts.p, stream);
-  groups.alloc(nlists + 1);
-  mi::launch_tile_groups(counts.p, nlists + 1, S.lockstep(), groups.p, d_need.p + 2, stream);
+    mi::launch_tile_count(fams.p, d_pos, plan->subset_family_begin(s), plan->subset_family_begin(s + 1), ntang, pool.p,
+                          rec, tof_fp_w, ntof, s, dims, A, nunits, slot, counts, stream);
+  mi::launch_tile_groups(counts, nlists + 1, S.lockstep(), groups, d_need + 2, stream);
   HIPCHECK(hipGetLastError());
   scan(groups, group_off, nlists + 1);
-  counts.release();
-  HIPCHECK(hipMemcpy(&totals[1], group_off.p + nlists, sizeof(uint32_t), hipMemcpyDeviceToHost));
-  HIPCHECK(hipMemcpy(need, d_need.p, sizeof(need), hipMemcpyDeviceToHost));
+  HIPCHECK(hipMemcpy(&totals[1], group_off + nlists, sizeof(uint32_t), hipMemcpyDeviceToHost));
+  HIPCHECK(hipMemcpy(need, d_need, sizeof(need), hipMemcpyDeviceToHost));
   const int64_t nslots = 4 * static_cast<int64_t>(totals[1]);
   if (need[2]) return false;
   tile_hdr.alloc((nph + mi::kTileHdrSlack) * mi::kTileWaves);
-  mi::launch_tile_headers(groups.p, group_off.p, phase_row.p, total_rows, nph, S, tile_hdr.p, stream);
+  mi::launch_tile_headers(groups, group_off, phase_row, total_rows, nph, S, tile_hdr.p, stream);
   // pass 4, subset by subset: every term's list and entry, sorted by list, to
   // its place
-  DBuf<int64_t> d_fam_off;
-  upload(d_fam_off, fam_off);
+  const int64_t* d_fam_off = upload(fam_off);
   tile_off.alloc(nslots + mi::kTileEntSlack);
   tile_w.alloc(nslots + mi::kTileEntSlack);
   HIPCHECK(hipMemsetAsync(tile_off.p, 0, tile_off.bytes(), stream));  // padding: weight 0 times the leading zeros
   HIPCHECK(hipMemsetAsync(tile_w.p, 0, tile_w.bytes(), stream));
   {
-    DBuf<uint32_t> keys_in, keys_out, vals_in, vals_out;
-    DBuf<int2> raw;
-    DBuf<char> tmp;
-    keys_in.alloc(most);
-    keys_out.alloc(most);
-    vals_in.alloc(most);
-    vals_out.alloc(most);
-    raw.alloc(most);
-    mi::launch_iota(vals_in.p, most, stream);
+    uint32_t *keys_in = mem.get<uint32_t>(most), *keys_out = mem.get<uint32_t>(most);
+    uint32_t *vals_in = mem.get<uint32_t>(most), *vals_out = mem.get<uint32_t>(most);
+    int2* raw = mem.get<int2>(most);
+    mi::launch_iota(vals_in, most, stream);
     const uint32_t none = static_cast<uint32_t>(nlists);
     int end_bit = 1;
     while ((int64_t{1} << end_bit) <= nlists) ++end_bit;
     size_t tb = 0;
-    HIPCHECK(mi::radix_sort_pairs(nullptr, tb, keys_in.p, keys_out.p, vals_in.p, vals_out.p, static_cast<int>(most),
+    HIPCHECK(mi::radix_sort_pairs(nullptr, tb, keys_in, keys_out, vals_in, vals_out, static_cast<int>(most),
                                   end_bit, stream));
-    tmp.alloc(std::max<size_t>(tb, 1));
+    char* tmp = mem.get<char>(std::max<size_t>(tb, 1));
     for (int s = 0; s < nsub; ++s) {
       const int fb = plan->subset_family_begin(s), fe = plan->subset_family_begin(s + 1);
       const int64_t m = (fam_off[fe] - fam_off[fb]) * span;
       if (m <= 0) continue;
-      mi::launch_tile_make(fams.p, d_pos.p, fb, fe, ntang, pool.p, rec, tof_fp_w, ntof, s, dims, A, nunits, slot.p, none,
-                           span, d_fam_off.p, fam_off[fb], keys_in.p, raw.p, stream);
-      HIPCHECK(mi::radix_sort_pairs(tmp.p, tb, keys_in.p, keys_out.p, vals_in.p, vals_out.p, static_cast<int>(m), end_bit,
+      mi::launch_tile_make(fams.p, d_pos, fb, fe, ntang, pool.p, rec, tof_fp_w, ntof, s, dims, A, nunits, slot, none,
+                           span, d_fam_off, fam_off[fb], keys_in, raw, stream);
+      HIPCHECK(mi::radix_sort_pairs(tmp, tb, keys_in, keys_out, vals_in, vals_out, static_cast<int>(m), end_bit,
                                     stream));
-      mi::launch_tile_place(keys_out.p, vals_out.p, raw.p, group_off.p, none, S.lockstep(), m, tile_off.p, tile_w.p, stream);
+      mi::launch_tile_place(keys_out, vals_out, raw, group_off, none, S.lockstep(), m, tile_off.p, tile_w.p, stream);
     }
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipStreamSynchronize(stream));
   }
   // launch order: the tiles with the most entries first, so that the last
   // workgroups to run are short ones
-  DBuf<uint32_t> d_work;
-  d_work.alloc(ntiles);
-  mi::launch_tile_work(group_off.p, tile_phase_off.p, nsub, ntiles, S.lines(), d_work.p, stream);
+  uint32_t* d_work = mem.get<uint32_t>(ntiles);
+  mi::launch_tile_work(group_off, tile_phase_off.p, nsub, ntiles, S.lines(), d_work, stream);
   std::vector<uint32_t> work(ntiles);
-  HIPCHECK(hipMemcpyAsync(work.data(), d_work.p, d_work.bytes(), hipMemcpyDeviceToHost, stream));
+  HIPCHECK(hipMemcpyAsync(work.data(), d_work, ntiles * sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
   HIPCHECK(hipStreamSynchronize(stream));
   std::vector<int32_t> order(ntiles);
   for (int t = 0; t < ntiles; ++t) order[t] = t;
   std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return work[a] > work[b]; });
-  upload(tile_order, order);
+  tile_order.alloc(ntiles);
+  HIPCHECK(hipMemcpyAsync(tile_order.p, order.data(), tile_order.bytes(), hipMemcpyHostToDevice, stream));
   HIPCHECK(hipStreamSynchronize(stream));
   A.hdr = tile_hdr.p;
   A.off = tile_off.p;

@@ -299,8 +299,27 @@ __global__ void tile_place_kernel(const uint32_t* __restrict__ keys, const uint3
        r += static_cast<int64_t>(gridDim.x) * blockDim.x) {
     const uint32_t key = keys[r];
     if (key == none) continue;
-    int64_t rank = 0;
-    while (rank < r && keys[r - rank - 1] == key) ++rank;
+    // the list's first term among the wave's, or else by bisection before them
+    const int lane = static_cast<int>(threadIdx.x % kWave);
+    const bool head = r == 0 || keys[r - 1] != key;
+    const uint64_t heads = __ballot(head) & (~0ull >> (kWave - 1 - lane));
+    int64_t rank;
+    if (heads) {
+      rank = lane - (63 - __builtin_clzll(heads));
+    } else {
+      int64_t lo = 0, hi = r - lane - 1;  // keys[hi] == key
+      for (int64_t step = 64; hi > 0; step *= 2) {
+        const int64_t at = hi > step ? hi - step : 0;
+        if (keys[at] != key) { lo = at + 1; break; }
+        hi = at;
+      }
+      while (lo < hi) {
+        const int64_t mid = (lo + hi) / 2;
+        if (keys[mid] == key) hi = mid;
+        else lo = mid + 1;
+      }
+      rank = r - hi;
+    }
     const int2 E = raw[idx[r]];
     const uint32_t line = key % lockstep;
     const int64_t at = 4 * (group_off[key - line] + rank / 4 * lockstep + line) + rank % 4;
