@@ -144,7 +144,7 @@ struct mi_ctx {
   DBuf<mi::BpEntry> entries;
   // back projection through LDS slabs (build_slab_table), or by image
   // column over the column table (list_off) otherwise
-  bool slab_allowed = true;  // batches read the column table
+  bool in_batch = false;  // the batch kernels read the column table of images of up to kTileShortPlanes planes
   int slab_enable = 0;       // MI_TUNE_BP_SLAB
   int slab_tx = 8, slab_ty = 8, slab_cpw = 4, slab_lds_kb = 80;
   bool use_slab = false;
@@ -173,6 +173,7 @@ struct mi_ctx {
   // default where build_tile_table accepts the geometry
   bool use_tile = false;
   int64_t tile_entries = 0;
+  std::vector<uint32_t> tile_work;  // groups of entries of every tile
   DBuf<uint32_t> tile_phase_off;
   DBuf<uint4> tile_hdr;
   DBuf<int32_t> tile_off, tile_order;
@@ -990,7 +991,7 @@ void mi_ctx::build_tof_rows(int64_t n) {
 // table is built instead).
 bool mi_ctx::build_slab_table() {
   const mi_geometry& g = plan->geometry();
-  if (!slab_allowed || !slab_enable || ntof > 1 || uniform_ppa != 1 || dims.nzp > 2 * 64 || h_fams.empty())
+  if (in_batch || !slab_enable || ntof > 1 || uniform_ppa != 1 || dims.nzp > 2 * 64 || h_fams.empty())
     return false;
   const auto& keys = plan->family_keys();
   for (size_t i = 0; i < h_fams.size(); ++i)
@@ -1205,7 +1206,7 @@ bool mi_ctx::build_slab_table() {
 // of one element.
 bool mi_ctx::build_tile_table(int span) {
   const mi_geometry& g = plan->geometry();
-  if (!slab_allowed || slab_enable || quad_enable || dims.nz > 256 || h_fams.empty()) return false;
+  if ((in_batch && dims.nz <= mi::kTileShortPlanes) || slab_enable || quad_enable || dims.nz > 256 || h_fams.empty()) return false;
   if (total_bins() >= (int64_t{1} << 31) || (ntof > 1 && tof_fp_w <= 0)) return false;
   const int32_t* rec = ntof > 1 ? tof_fp_rec.p : nullptr;
   const auto& keys = plan->family_keys();
@@ -1403,7 +1404,8 @@ bool mi_ctx::build_tile_table(int span) {
   // workgroups to run are short ones
   uint32_t* d_work = mem.get<uint32_t>(ntiles);
   mi::launch_tile_work(group_off, tile_phase_off.p, nsub, ntiles, S.lines(), d_work, stream);
-  std::vector<uint32_t> work(ntiles);
+  std::vector<uint32_t>& work = tile_work;
+  work.resize(ntiles);
   HIPCHECK(hipMemcpyAsync(work.data(), d_work, ntiles * sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
   HIPCHECK(hipStreamSynchronize(stream));
   std::vector<int32_t> order(ntiles);
@@ -2735,6 +2737,10 @@ struct mi_batch {
   // [ppa class * 6 + variant], variants: 4 parts, 2 parts, 1..4 slots
   std::array<int, 18> bpw_n{};
   std::array<std::unique_ptr<DBuf<mi::WorkItem>>, 18> bpw_work;
+  // back projection by image tiles, per slot count: (problem, tile)
+  DBuf<mi::TileArgs> tile_args;
+  std::array<int, 4> tile_n{};
+  std::array<std::unique_ptr<DBuf<mi::WorkItem>>, 4> tile_work;
   // forward row groups per subset: items and their family lists
   std::vector<int> rg_n;
   std::vector<std::unique_ptr<DBuf<mi::RowGroupItem>>> rg_items;
@@ -2916,8 +2922,15 @@ void batch_prepare(mi_batch* b) {
   // of at most 32 planes in lane groups (when packing), the others one column per wave
   std::array<std::vector<mi::WorkItem>, 4> lists;
   std::array<std::vector<mi::WorkItem>, 18> wide;
+  std::array<std::vector<mi::WorkItem>, 4> tiles;
+  std::vector<mi::TileArgs> targs(np);
   for (int p = 0; p < np; ++p) {
     const mi::ImageDims& d = b->probs[p]->dims;
+    if (b->probs[p]->use_tile) {
+      targs[p] = b->probs[p]->tile;
+      for (int t = 0; t < targs[p].ntiles; ++t) tiles[(d.nz - 1) / 64].push_back({p, t});
+      continue;
+    }
     const int gi = group_index_at_least(d.nzp);
     const bool grouped = b->bp_pack == 1 && gi >= 0 && gi <= 2;
     const int ppa = b->probs[p]->uniform_ppa;
@@ -2940,6 +2953,15 @@ void batch_prepare(mi_batch* b) {
     b->bp_n[gi] = static_cast<int>(lists[gi].size());
     b->bp_work[gi] = upload(lists[gi]);
   }
+  b->tile_args.alloc(np);
+  HIPCHECK(hipMemcpy(b->tile_args.p, targs.data(), b->tile_args.bytes(), hipMemcpyHostToDevice));
+  for (int k = 0; k < 4; ++k) {  // the tiles with the most entries first
+    std::stable_sort(tiles[k].begin(), tiles[k].end(), [&](const mi::WorkItem& a, const mi::WorkItem& c) {
+      return b->probs[a.problem]->tile_work[a.index] > b->probs[c.problem]->tile_work[c.index];
+    });
+    b->tile_n[k] = static_cast<int>(tiles[k].size());
+    b->tile_work[k] = upload(tiles[k]);
+  }
   for (int k = 0; k < 18; ++k) {
     b->bpw_n[k] = static_cast<int>(wide[k].size());
     b->bpw_work[k] = upload(wide[k]);
@@ -2956,6 +2978,9 @@ void batch_fp(mi_batch* b, mi::FpMode mode, int s) {
 }
 void batch_bp(mi_batch* b, mi::BpMode mode, int s, int threshold) {
   static const int kVariantSlots[6] = {-4, -2, 1, 2, 3, 4};
+  for (int k = 0; k < 4; ++k)
+    mi::launch_back_project_tile_batch(mode, k + 1, b->descs.p, b->tile_args.p, b->tile_work[k]->p, b->tile_n[k], s,
+                                       threshold, b->stream);
   for (int k = 0; k < 18; ++k)
     mi::launch_bp_batch(mode, k / 6, kVariantSlots[k % 6], b->descs.p, b->bpw_work[k]->p, b->bpw_n[k], s, threshold,
                         b->stream);
@@ -2991,7 +3016,7 @@ int mi_batch_create(int device, int n, const mi_geometry* geometries, int num_su
       mi_ctx* c = nullptr;
       if (mi_ctx_create(device, &c) != MI_OK) throw ApiError(MI_ERR_DEVICE, g_last_error);
       b->probs.push_back(c);
-      c->slab_allowed = false;  // the batch kernels read the column table
+      c->in_batch = true;
       if (mi_set_up(c, &geometries[i], num_subsets) != MI_OK)
         throw ApiError(MI_ERR_ARGUMENT, "problem " + std::to_string(i) + ": " + g_last_error);
     }

@@ -409,6 +409,10 @@ void launch_tile_place(const uint32_t* d_keys, const uint32_t* d_idx, const int2
                        uint32_t none, int lockstep, int64_t n, int32_t* d_off, float* d_w, hipStream_t stream);
 void launch_back_project_tile(BpMode mode, const TileArgs& A, int subset_begin, int subset_end, const float* d_proj,
                               float* d_img, const ImageDims& dims, const BpData& data, hipStream_t stream);
+// one subset of several problems (images of more than kTileShortPlanes planes,
+// 64 nslot at most): work items are (problem, tile)
+void launch_back_project_tile_batch(BpMode mode, int nslot, const ProblemDesc* d_descs, const TileArgs* d_tiles,
+                                    const WorkItem* d_work, int nwork, int subset, int threshold, hipStream_t stream);
 
 // ---- BP table build (pmrt_table.hip)
 void launch_count_entries(const Family* d_fams, int fam_begin, int fam_end, const int2* d_pool, int subset,

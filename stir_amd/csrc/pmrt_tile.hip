@@ -385,14 +385,9 @@ __device__ inline void tile_group(int off, int w, const char* lds, int lane4, fl
 constexpr uint32_t kTileSumPhases = 8;
 
 template <int MODE, int NSLOT, bool TOF>
-__global__ void __launch_bounds__(kWave* kTileWaves) bp_tile_kernel(TileArgs A, int sb, int se,
-                                                                    const float* __restrict__ proj,
-                                                                    float* __restrict__ img, ImageDims d, BpData data,
-                                                                    int chunk) {
+__device__ __forceinline__ void tile_sums(const TileArgs& A, int t, int sb, int se, const float* __restrict__ proj,
+                                          float* __restrict__ img, const ImageDims& d, const BpData& data) {
   extern __shared__ float tile_lds[];
-  const int b = xcd_chunk_remap(static_cast<int>(blockIdx.x), chunk);
-  if (b >= A.ntiles) return;
-  const int t = as_const(A.order)[b];
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
   const int lane = static_cast<int>(threadIdx.x % kWave);
   const int lane4 = 4 * lane;
@@ -517,6 +512,38 @@ __global__ void __launch_bounds__(kWave* kTileWaves) bp_tile_kernel(TileArgs A, 
       }
     }
   }
+}
+
+template <int MODE, int NSLOT, bool TOF>
+__global__ void __launch_bounds__(kWave* kTileWaves) bp_tile_kernel(TileArgs A, int sb, int se,
+                                                                    const float* __restrict__ proj,
+                                                                    float* __restrict__ img, ImageDims d, BpData data,
+                                                                    int chunk) {
+  const int b = xcd_chunk_remap(static_cast<int>(blockIdx.x), chunk);
+  if (b >= A.ntiles) return;
+  tile_sums<MODE, NSLOT, TOF>(A, as_const(A.order)[b], sb, se, proj, img, d, data);
+}
+
+// tiles of several problems, heaviest first, one subset
+template <int MODE, int NSLOT>
+__global__ void __launch_bounds__(kWave* kTileWaves) bp_tile_batch_kernel(const ProblemDesc* __restrict__ descs,
+                                                                          const TileArgs* __restrict__ tiles,
+                                                                          const WorkItem* __restrict__ work, int nwork,
+                                                                          int subset, int threshold) {
+  const int b = xcd_chunk_remap(static_cast<int>(blockIdx.x), kTileXcdChunk);
+  if (b >= nwork) return;
+  const int p = __builtin_amdgcn_readfirstlane(work[b].problem);
+  const int t = __builtin_amdgcn_readfirstlane(work[b].index);
+  const ProblemDesc& P = descs[p];
+  BpData bd{};
+  bd.sens = P.sens ? as_const(P.sens)[subset] : nullptr;
+  bd.estimate = P.estimate;
+  bd.update = nullptr;
+  bd.threshold = threshold;
+  bd.thr_lo = P.thr_lo;
+  bd.thr_hi = P.thr_hi;
+  const TileArgs A = tiles[p];
+  tile_sums<MODE, NSLOT, false>(A, t, subset, subset + 1, P.bp_in, P.bp_out, P.d, bd);
 }
 
 // ---- short images
@@ -925,6 +952,27 @@ void launch_back_project_tile(BpMode mode, const TileArgs& A, int subset_begin, 
     if (mode == BP_PLAIN) { MI_TILE_S(BP_PLAIN, false) }
     else { MI_TILE_S(BP_OSEM_UPDATE, false) }
   }
+#undef MI_TILE_S
+#undef MI_TILE
+}
+
+void launch_back_project_tile_batch(BpMode mode, int nslot, const ProblemDesc* d_descs, const TileArgs* d_tiles,
+                                    const WorkItem* d_work, int nwork, int subset, int threshold, hipStream_t stream) {
+  if (nwork <= 0) return;
+  const int round = kNumXcd * kTileXcdChunk;
+  const dim3 grid((nwork + round - 1) / round * round), block(kWave * kTileWaves);
+#define MI_TILE(M, S) \
+  hipLaunchKernelGGL((bp_tile_batch_kernel<M, S>), grid, block, kTileLdsBytes, stream, d_descs, d_tiles, d_work, nwork, \
+                     subset, threshold)
+#define MI_TILE_S(M)               \
+  switch (nslot) {                 \
+    case 1: MI_TILE(M, 1); break;  \
+    case 2: MI_TILE(M, 2); break;  \
+    case 3: MI_TILE(M, 3); break;  \
+    default: MI_TILE(M, 4); break; \
+  }
+  if (mode == BP_OSEM_UPDATE) { MI_TILE_S(BP_OSEM_UPDATE) }
+  else { MI_TILE_S(BP_PLAIN) }
 #undef MI_TILE_S
 #undef MI_TILE
 }
