@@ -279,7 +279,7 @@ struct mi_ctx {
   float prior_beta = 0.F, prior_gamma = 2.F, prior_eps = 0.F;
   int prior_only_2D = 0;
   mi::PriorWeights prior_w{};
-  DBuf<float> prior_kappa, prior_grad, small_part, small_val;
+  DBuf<float> prior_kappa, prior_grad, small_part;
   bool prior_active() const { return prior_kind != 0 && prior_beta != 0.F; }
   mi::PriorImage device_prior_image() const {
     const mi_geometry& g = plan->geometry();
@@ -2106,9 +2106,8 @@ static void osem_step(mi_ctx* ctx, int subset, int subiteration_num) {
   ctx->bp(mi::BP_PLAIN, ctx->ratio.p, ctx->img2.p, subset, mi::BpData{}, ctx->stream);
   mi::launch_prior(ctx->prior_kind, ctx->x.p, ctx->prior_kappa.p, ctx->device_prior_image(), ctx->prior_w,
                    ctx->prior_only_2D, ctx->prior_beta, ctx->prior_gamma, ctx->prior_eps, ctx->prior_grad.p,
-                   ctx->prior_partial.p, ctx->stream);
-  mi::launch_small_value(ctx->img2.p, ctx->img2.n, 0.000001F, ctx->small_part.p, ctx->small_val.p, ctx->stream);
-  mi::launch_osl_update(ctx->x.p, ctx->img2.p, ctx->prior_grad.p, ctx->sens[subset]->p, ctx->small_val.p,
+                   nullptr, ctx->stream);
+  mi::launch_osl_update(ctx->x.p, ctx->img2.p, ctx->prior_grad.p, ctx->sens[subset]->p, 0.000001F, ctx->small_part.p,
                         ctx->plan->num_subsets(), ctx->map_multiplicative, subiteration_num != 1, ctx->min_rel,
                         ctx->max_rel, ctx->dims.nz, ctx->dims.nzp, ctx->img.n, ctx->stream);
 }
@@ -2229,7 +2228,7 @@ int mi_quadratic_prior_dev(mi_ctx* ctx, const float* d_image, const float* d_kap
       if (weights) std::memcpy(W.w, weights, sizeof(W.w));
       else default_prior_weights(g, W.w);
       mi::launch_prior(1, d_image, d_kappa, ctx->stir_prior_image(), W, only_2D, beta, 0.F, 0.F, d_gradient,
-                       ctx->prior_partial.p, st);
+                       d_value ? ctx->prior_partial.p : nullptr, st);
       if (d_value)
         mi::launch_sum_partials(ctx->prior_partial.p, mi::prior_num_partials(ctx->stir_prior_image()),
                                 static_cast<double>(beta), d_value, st);
@@ -2262,7 +2261,7 @@ int mi_quadratic_prior_noalloc_dev(int device, int nz, int ny, int nx, float vox
       mi::PriorWeights W;
       if (weights) std::memcpy(W.w, weights, sizeof(W.w));
       else default_prior_weights(vox_z, vox_y, vox_x, W.w);
-      mi::launch_prior(1, d_image, d_kappa, im, W, only_2D, beta, 0.F, 0.F, d_gradient, partials, st);
+      mi::launch_prior(1, d_image, d_kappa, im, W, only_2D, beta, 0.F, 0.F, d_gradient, d_value ? partials : nullptr, st);
       if (d_value) mi::launch_sum_partials(partials, nparts, static_cast<double>(beta), d_value, st);
     }
     HIPCHECK(hipGetLastError());
@@ -2483,7 +2482,6 @@ int mi_obj_set_prior(mi_ctx* ctx, const mi_prior* prior) {
     ctx->prior_grad.alloc(ctx->img.n);
     HIPCHECK(hipMemsetAsync(ctx->prior_grad.p, 0, ctx->prior_grad.bytes(), st));
     ctx->small_part.alloc(mi::max_num_partials());
-    ctx->small_val.alloc(1);
     HIPCHECK(hipStreamSynchronize(st));
   });
 }
@@ -2506,7 +2504,7 @@ int mi_relative_difference_prior_dev(mi_ctx* ctx, const float* d_image, const fl
       if (weights) std::memcpy(W.w, weights, sizeof(W.w));
       else default_prior_weights(g, W.w);
       mi::launch_prior(2, d_image, d_kappa, ctx->stir_prior_image(), W, only_2D, beta, gamma, epsilon, d_gradient,
-                       ctx->prior_partial.p, st);
+                       d_value ? ctx->prior_partial.p : nullptr, st);
       if (d_value)
         mi::launch_sum_partials(ctx->prior_partial.p, mi::prior_num_partials(ctx->stir_prior_image()),
                                 static_cast<double>(beta), d_value, st);

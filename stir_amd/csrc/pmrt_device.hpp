@@ -469,8 +469,8 @@ struct PriorImage {
   int nz, ny, nx, nzp;
   int zfast;
 };
-// Value partials without beta (one double per workgroup, count returned by
-// prior_num_partials) and beta * gradient (if d_grad) of a neighbourhood
+// Value partials without beta (if d_partial; one double per workgroup, count
+// returned by prior_num_partials) and beta * gradient (if d_grad) of a neighbourhood
 // prior: kind 1 quadratic, 2 relative difference (gamma, eps); kappa may be null.
 int prior_num_partials(const PriorImage& im);
 void launch_prior(int kind, const float* d_img, const float* d_kappa, const PriorImage& im, const PriorWeights& w,
@@ -488,19 +488,18 @@ void launch_prior_hessian(int kind, const float* d_x, const float* d_in, const f
 constexpr int kNoAllocPartials = 65536;
 constexpr int kMaxDevices = 64;
 double* noalloc_partials(int device);
-// *d_small = max(max(v) * small_num, 0) over n floats (d_part: max_num_partials() floats)
+// One-step-late OSMAPOSL update on the device layout (n = ncols * nzp elements);
+// d_part: max_num_partials() floats
 int max_num_partials();
-void launch_small_value(const float* d_v, int64_t n, float small_num, float* d_part, float* d_small, hipStream_t stream);
-// One-step-late OSMAPOSL update on the device layout (n = ncols * nzp elements)
-void launch_osl_update(float* d_x, const float* d_upd, const float* d_pgrad, const float* d_sens, const float* d_small,
-                       int nsub, int multiplicative, int threshold, float lo, float hi, int nz, int nzp, int64_t n,
-                       hipStream_t stream);
+void launch_osl_update(float* d_x, const float* d_upd, const float* d_pgrad, const float* d_sens, float small_num,
+                       float* d_part, int nsub, int multiplicative, int threshold, float lo, float hi, int nz, int nzp,
+                       int64_t n, hipStream_t stream);
 // dst += src; dst /= d (element-wise, n elements)
 void launch_accumulate(float* d_dst, const float* d_src, int64_t n, hipStream_t stream);
 void launch_divide_scalar(float* d_dst, float d, int64_t n, hipStream_t stream);
 void launch_subtract(float* d_dst, const float* d_src, int64_t n, hipStream_t stream);  // dst -= src
-// *d_out = sum of n doubles in a fixed order (one workgroup); d_out may be null-checked by the caller.
-void launch_sum_partials(const double* d_partial, int n, double scale, double* d_out, hipStream_t stream);
+// *d_out = scale * the sum of n doubles in a fixed order; more than a few thousand are overwritten.
+void launch_sum_partials(double* d_partial, int n, double scale, double* d_out, hipStream_t stream);
 // v = g * x / sens (0 where sens == 0), device image layout, n elements; v may alias g or x
 void launch_osem_vjp_scale(const float* d_g, const float* d_x, const float* d_sens, float* d_v, int64_t n,
                            hipStream_t stream);
