@@ -134,6 +134,7 @@ struct mi_ctx {
   // forward projection by row groups (pmrt_rows.hip), for short families
   bool use_rows = false;
   std::vector<int> item_off;  // per subset, size nsub+1
+  std::vector<int2> h_row_items;  // of a batch's problem
   DBuf<mi::RowGroup> row_groups;
   DBuf<int32_t> row_fams;
   DBuf<int2> row_items;
@@ -760,6 +761,7 @@ void mi_ctx::build_row_groups() {
   upload(row_groups, groups);
   upload(row_fams, list);
   upload(row_items, items);
+  if (in_batch) h_row_items = items;
   mi::launch_row_group_reach(row_groups.p, static_cast<int>(groups.size()), row_fams.p, fams.p, pool.p, dims, stream);
   HIPCHECK(hipGetLastError());
   HIPCHECK(hipStreamSynchronize(stream));
@@ -2743,6 +2745,9 @@ struct mi_batch {
   std::vector<int> rg_n;
   std::vector<std::unique_ptr<DBuf<mi::RowGroupItem>>> rg_items;
   std::vector<std::unique_ptr<DBuf<int32_t>>> rg_fams;
+  // problems with row groups of their own: (problem, item) per subset
+  DBuf<mi::RowProblem> rows;
+  std::vector<std::unique_ptr<DBuf<int4>>> row_work;
   bool lists_ready = false;
   hipGraphExec_t graph_exec = nullptr;
   int graph_key[3] = {0, 0, 0};  // start subiteration, count, start subset of the captured graph
@@ -2840,13 +2845,26 @@ void batch_prepare(mi_batch* b) {
   b->rg_n.assign(b->nsub, 0);
   b->rg_items.clear();
   b->rg_fams.clear();
+  b->row_work.clear();
+  std::vector<mi::RowProblem> rows(np, mi::RowProblem{});
+  for (int p = 0; p < np; ++p)
+    if (b->probs[p]->use_rows)
+      rows[p] = {b->probs[p]->row_groups.p, b->probs[p]->row_fams.p};
+  b->rows.alloc(np);
+  HIPCHECK(hipMemcpy(b->rows.p, rows.data(), b->rows.bytes(), hipMemcpyHostToDevice));
   for (int s = 0; s < b->nsub; ++s) {
+    std::vector<int4> row_work;
     std::array<std::vector<mi::WorkItem>, 4> lists;
     std::array<std::vector<mi::WorkItem>, 4> wide;
     std::vector<mi::RowGroupItem> rg;
     std::vector<int32_t> rg_fam;
     for (int p = 0; p < np; ++p) {
       const mi_ctx* c = b->probs[p];
+      if (c->use_rows && b->fp_rowgroup_max > 0) {  // the groups its own forward projection uses
+        for (int i = c->item_off[s]; i < c->item_off[s + 1]; ++i)
+          row_work.push_back(make_int4(p, c->h_row_items[i].x, c->h_row_items[i].y, 0));
+        continue;
+      }
       std::vector<mi::FpTask> ht(c->task_off[s + 1] - c->task_off[s]);
       if (!ht.empty())
         HIPCHECK(hipMemcpy(ht.data(), c->tasks.p + c->task_off[s], ht.size() * sizeof(mi::FpTask), hipMemcpyDeviceToHost));
@@ -2904,6 +2922,12 @@ void batch_prepare(mi_batch* b) {
       b->fpw_n[s][k] = static_cast<int>(wide[k].size());
       b->fpw_work[s][k] = upload(wide[k]);
     }
+    auto rw = std::make_unique<DBuf<int4>>();
+    if (!row_work.empty()) {
+      rw->alloc(row_work.size());
+      HIPCHECK(hipMemcpy(rw->p, row_work.data(), rw->bytes(), hipMemcpyHostToDevice));
+    }
+    b->row_work.push_back(std::move(rw));
     b->rg_n[s] = static_cast<int>(rg.size());
     auto di = std::make_unique<DBuf<mi::RowGroupItem>>();
     auto df = std::make_unique<DBuf<int32_t>>();
@@ -2968,6 +2992,8 @@ void batch_prepare(mi_batch* b) {
 }
 
 void batch_fp(mi_batch* b, mi::FpMode mode, int s) {
+  mi::launch_forward_project_rows_batch(mode, b->descs.p, b->rows.p, b->row_work[s]->p,
+                                        static_cast<int>(b->row_work[s]->n), b->stream);
   mi::launch_fp_rowgroup(mode, b->descs.p, b->rg_items[s]->p, b->rg_fams[s]->p, b->rg_n[s], b->stream);
   for (int k = 0; k < 4; ++k)
     mi::launch_fp_batch(mode, k + 1, b->descs.p, b->task_lists.p, b->fpw_work[s][k]->p, b->fpw_n[s][k], b->stream);

@@ -262,6 +262,14 @@ struct WorkItem {
   int32_t problem;
   int32_t index;
 };
+// a problem's own row groups, for the batched forward projection; work items
+// are (problem, group, first bin)
+struct RowProblem {
+  const RowGroup* groups;
+  const int32_t* fam_list;
+};
+void launch_forward_project_rows_batch(FpMode mode, const ProblemDesc* d_descs, const RowProblem* d_rows,
+                                       const int4* d_work, int nwork, hipStream_t stream);
 // a row group of a batched forward projection: item_fams[first .. first+count)
 // are families of one problem sharing one basic row, at most 64 axial
 // positions in total

@@ -80,20 +80,13 @@ __global__ void __launch_bounds__(kWave) row_group_reach_kernel(RowGroup* __rest
   groups[g].inside = inside;
 }
 
+// item it (group, first bin): 64 bins of a group; log-likelihood sum to place w
 template <int MODE>
-__global__ void __launch_bounds__(kWave* kWavesPerBlock) fp_rows_kernel(const int2* __restrict__ items, int nitems,
-                                                                        const RowGroup* __restrict__ groups,
-                                                                        const int32_t* __restrict__ fam_list,
-                                                                        const Family* __restrict__ fams,
-                                                                        const int2* __restrict__ pool,
-                                                                        const float* __restrict__ img,
-                                                                        float* __restrict__ out, ImageDims d,
-                                                                        FpData data) {
-  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
-  const int w = xcd_chunk_remap(static_cast<int>(blockIdx.x), kRowsXcdChunk) * kWavesPerBlock + wave;
-  if (w >= nitems) return;
+__device__ __forceinline__ void rows_item(int w, const int2 it, const RowGroup* __restrict__ groups,
+                                          const int32_t* __restrict__ fam_list, const Family* __restrict__ fams,
+                                          const int2* __restrict__ pool, const float* __restrict__ img,
+                                          float* __restrict__ out, const ImageDims& d, const FpData& data) {
   const int lane = static_cast<int>(threadIdx.x % kWave);
-  const int2 it = as_const(items)[w];  // group, first bin
   const RowGroup G = as_const(groups)[it.x];
   const int j = it.y + lane, last = G.nfam * G.nax - 1;
   const bool valid = j <= last;
@@ -158,6 +151,36 @@ __global__ void __launch_bounds__(kWave* kWavesPerBlock) fp_rows_kernel(const in
   }
 }
 
+template <int MODE>
+__global__ void __launch_bounds__(kWave* kWavesPerBlock) fp_rows_kernel(const int2* __restrict__ items, int nitems,
+                                                                        const RowGroup* __restrict__ groups,
+                                                                        const int32_t* __restrict__ fam_list,
+                                                                        const Family* __restrict__ fams,
+                                                                        const int2* __restrict__ pool,
+                                                                        const float* __restrict__ img,
+                                                                        float* __restrict__ out, ImageDims d,
+                                                                        FpData data) {
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
+  const int w = xcd_chunk_remap(static_cast<int>(blockIdx.x), kRowsXcdChunk) * kWavesPerBlock + wave;
+  if (w >= nitems) return;
+  rows_item<MODE>(w, as_const(items)[w], groups, fam_list, fams, pool, img, out, d, data);
+}
+
+// work: (problem, group, first bin)
+template <int MODE>
+__global__ void __launch_bounds__(kWave* kWavesPerBlock) fp_rows_batch_kernel(const ProblemDesc* __restrict__ descs,
+                                                                              const RowProblem* __restrict__ rows,
+                                                                              const int4* __restrict__ work,
+                                                                              int nwork) {
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
+  const int w = xcd_chunk_remap(static_cast<int>(blockIdx.x), kRowsXcdChunk) * kWavesPerBlock + wave;
+  if (w >= nwork) return;
+  const int4 it = as_const(work)[w];
+  const ProblemDesc P = as_const(descs)[it.x];
+  const RowProblem R = as_const(rows)[it.x];
+  rows_item<MODE>(w, make_int2(it.y, it.z), R.groups, R.fam_list, P.fams, P.pool, P.fp_in, P.fp_out, P.d, P.fd);
+}
+
 }  // namespace
 
 void launch_row_group_reach(RowGroup* d_groups, int ngroups, const int32_t* d_fam_list, const Family* d_fams,
@@ -192,6 +215,17 @@ void launch_forward_project_rows(FpMode mode, const int2* d_items, int nitems, c
     MI_ROWS(FP_LM_VALUE)
 #undef MI_ROWS
   }
+}
+
+void launch_forward_project_rows_batch(FpMode mode, const ProblemDesc* d_descs, const RowProblem* d_rows,
+                                       const int4* d_work, int nwork, hipStream_t stream) {
+  if (nwork <= 0) return;
+  const int blocks = (nwork + kWavesPerBlock - 1) / kWavesPerBlock, round = kNumXcd * kRowsXcdChunk;
+  const dim3 grid((blocks + round - 1) / round * round), block(kWave * kWavesPerBlock);
+  if (mode == FP_RATIO)
+    hipLaunchKernelGGL(fp_rows_batch_kernel<FP_RATIO>, grid, block, 0, stream, d_descs, d_rows, d_work, nwork);
+  else
+    hipLaunchKernelGGL(fp_rows_batch_kernel<FP_PLAIN>, grid, block, 0, stream, d_descs, d_rows, d_work, nwork);
 }
 
 }  // namespace mi
