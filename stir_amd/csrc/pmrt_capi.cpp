@@ -914,7 +914,9 @@ void mi_ctx::build_quad_table(const uint32_t* d_perm, int64_t n, const int64_t* 
   quad_entries = total;
 }
 
-// Stored TOF rows when every family has a row of its own, the planes per
+// Stored TOF rows (forward records, and for the back projection the tile
+// table's terms or, where that is not built, records) when every family has a
+// row of its own, the planes per
 // axial position fit the record's 4 bits, the TOF data hold fewer than 2^31
 // bins, the widest live range fits a
 // window and the records fit in three quarters of the free device memory;
@@ -1224,6 +1226,12 @@ bool mi_ctx::build_tile_table(int span) {
     S.par = uniform_ppa == 2 ? 2 : 1;
     S.lanes = (dims.nz <= mi::kTileShortPlanes / 2 ? 16 : 32) / S.par;
     S.ty = 4;
+    // Lines of 16 (parity) or 32 lanes: tiles of 8 x 4 columns give a wave two
+    // sets of them and share the copied rows among more columns, but with fewer
+    // tiles than two workgroups per CU the chip is not filled: 4 x 4 columns
+    // then. All subsets, 16 rings, span 1: 60 x 60 columns 58 -> 37 us, 96 x 96
+    // 148 -> 130; 128 x 128 (512 tiles) 459 against 482 us with 4 x 4.
+    if (S.lanes * S.par == 32 && ((dims.nx + 7) / 8) * ((dims.ny + 3) / 4) < 2 * mi::kNumCu) S.tx = 4;
   }
   S.ntx = (dims.nx + S.tx - 1) / S.tx;
   std::vector<int4> hunits(nunits);

@@ -350,6 +350,7 @@ void launch_back_project_slab(BpMode mode, const SlabArgs& A, int subset_begin, 
 
 // ---- back projection by image tiles with the runs in LDS (pmrt_tile.hip):
 // tables whose families cover whole runs (z-shift symmetry)
+constexpr int kNumCu = 256;
 constexpr int kTileWaves = 8;         // waves that add entries, of either kernel
 // images of more than kTileShortPlanes planes: tiles of 64 columns
 constexpr int kTileCols = 64;

@@ -10,12 +10,15 @@
 // there (each staged run is used by about nine entries at mMR size).
 //
 // Measured at mMR size (4.2e8 entries, 837 x 252 x 344 bins, 344 x 344 x 127
-// voxels): 10.8 ms with the column kernel, 5.74 ms with this one: three
+// voxels): 10.8 ms with the column kernel, 5.65 ms with this one: three
 // workgroups of 8 waves and 53 KB of LDS per CU. Two of 16 waves and 80 KB:
 // 6.15 ms (5.97 with the reads of a group kept together); of 8 waves and
 // 80 KB: 6.7; four of 8 waves and 40 KB: 6.3 (shorter lists, more padding);
 // tiles of 12 x 8 columns: 5.75, of 16 x 8: 6.2. With the copies left out it
 // takes 4.1 ms, without copies and barriers 3.6 (the LDS reads alone 3.2).
+//
+// In OSEM a subset's pass takes 0.32 ms, 21 of them 6.8: of that, 0.05 go to
+// reading sensitivities and the estimate and writing it.
 //
 // Work: phases. The (segment, view) viewgrams of a subset are taken in family
 // order; consecutive ones form a phase as long as the tangential positions
@@ -614,7 +617,7 @@ constexpr int kShortBatch = 8;  // row list entries of a copy wave requested tog
 // SUM2: the sum of a phase is added to the voxel's sum as a whole (shorter
 // chains of additions); otherwise all terms one by one, as the column kernel
 // for one plane per axial position.
-template <int MODE, int LPC, int PAR, bool SUM2>
+template <int MODE, int LPC, int PAR, bool SUM2, int NSET>  // NSET: sets of lines of a wave
 __global__ void __launch_bounds__(kShortThreads, 6) bp_tile_short_kernel(TileArgs A, int sb, int se,
                                                                       const float* __restrict__ proj,
                                                                       float* __restrict__ img, ImageDims d, BpData data,
@@ -627,7 +630,6 @@ __global__ void __launch_bounds__(kShortThreads, 6) bp_tile_short_kernel(TileArg
   const int lane = static_cast<int>(threadIdx.x % kWave);
   for (int i = threadIdx.x; i < 2 * A.lead; i += kShortThreads)
     tile_lds[i < A.lead ? i : A.buffer + i - A.lead] = 0.F;
-  constexpr int NSET = 32 * PAR * LPC / (kTileWaves * kWave);  // sets of lines of a wave
   float acc[NSET], sum[NSET];
 #pragma unroll
   for (int s = 0; s < NSET; ++s) acc[s] = sum[s] = 0.F;
@@ -915,23 +917,27 @@ void launch_back_project_tile(BpMode mode, const TileArgs& A, int subset_begin, 
   if (A.shape.lanes < kWave) {
     // one plane per axial position (and mixed ones): the column kernel's order
     // of additions, bit for bit
-#define MI_SHORT(M, L, P, S2)                                                                                          \
-  hipLaunchKernelGGL((bp_tile_short_kernel<M, L, P, S2>), grid, dim3(kShortThreads), lds, stream, A, subset_begin,     \
+#define MI_SHORT(M, L, P, S2, N)                                                                                       \
+  hipLaunchKernelGGL((bp_tile_short_kernel<M, L, P, S2, N>), grid, dim3(kShortThreads), lds, stream, A, subset_begin,  \
                      subset_end, d_proj, d_img, dims, data, chunk)
+#define MI_SHORT_N(M, L, P, S2)               \
+  if (A.shape.tx == 8) MI_SHORT(M, L, P, S2, 2); \
+  else MI_SHORT(M, L, P, S2, 1);
 #define MI_SHORT_S(M)                                        \
   if (A.shape.par == 2) {                                    \
-    if (A.shape.lanes == 8) MI_SHORT(M, 8, 2, true);         \
-    else MI_SHORT(M, 16, 2, true);                           \
+    if (A.shape.lanes == 8) MI_SHORT(M, 8, 2, true, 1);      \
+    else { MI_SHORT_N(M, 16, 2, true) }                      \
   } else if (A.tof) {                                        \
-    if (A.shape.lanes == 16) MI_SHORT(M, 16, 1, true);       \
-    else MI_SHORT(M, 32, 1, true);                           \
+    if (A.shape.lanes == 16) MI_SHORT(M, 16, 1, true, 1);    \
+    else { MI_SHORT_N(M, 32, 1, true) }                      \
   } else {                                                   \
-    if (A.shape.lanes == 16) MI_SHORT(M, 16, 1, false);      \
-    else MI_SHORT(M, 32, 1, false);                          \
+    if (A.shape.lanes == 16) MI_SHORT(M, 16, 1, false, 1);   \
+    else { MI_SHORT_N(M, 32, 1, false) }                     \
   }
     if (mode == BP_PLAIN) { MI_SHORT_S(BP_PLAIN) }
     else { MI_SHORT_S(BP_OSEM_UPDATE) }
 #undef MI_SHORT_S
+#undef MI_SHORT_N
 #undef MI_SHORT
     return;
   }

@@ -11,8 +11,8 @@ within 2 n 2^-24. With one bin in 100 set, a voxel has a few tens of non-zero
 terms, so that a term that is lost or misplaced shows.
 
 Sizes at the edges: 1, 15, 16, 17, 31 and 32 planes (8, 16 and 32 lanes per
-line), image sides that are not multiples of the 8 x 4 tile, four planes per
-axial position, more than 64 phases per tile and fewer rows than one copy.
+line), image sides that are not multiples of the 8 x 4 or 4 x 4 tile, fewer and
+no fewer than 512 tiles (one or two sets of lines per wave), four planes per axial position, more than 64 phases per tile and fewer rows than one copy.
 """
 import numpy as np
 import pytest
@@ -34,6 +34,10 @@ CASES = {
     "31planes_span3": (16, 3, 10, 32, 31, 40, 41, 2.0, 0, True),
     "32planes_mixed": (16, 3, 15, 32, 32, 40, 40, 2.0, 0, True),
     "31planes_many_phases": (16, 1, 15, 96, 31, 30, 30, 2.0, 0, False),
+    "31planes_span1_512tiles": (16, 1, 3, 32, 31, 130, 132, 2.0, 0, False),
+    "32planes_span3_512tiles": (16, 3, 7, 32, 32, 128, 128, 2.0, 0, True),
+    "31planes_tof_512tiles": (16, 1, 3, 32, 31, 130, 132, 2.0, 5, False),
+    "31planes_span3_tof_512tiles": (16, 3, 7, 32, 31, 128, 128, 2.0, 5, False),
     "14planes_zoom2": (4, 1, 3, 32, 14, 40, 40, 1.0, 0, True),
     "15planes_tof": (8, 1, 7, 32, 15, 41, 47, 2.0, 5, False),
     "31planes_span3_tof": (16, 3, 10, 32, 31, 40, 41, 2.0, 9, False),
