@@ -170,7 +170,7 @@ def main():
     nvox = int(img.num_voxels)
     dominant = "bp" if bp_avg >= fp_avg else "fp"
     dom_ms = bp_avg if dominant == "bp" else fp_avg
-    kernel = ("bp_quad_kernel" if args.bp_quad else "bp_kernel") if dominant == "bp" else "fp_kernel"
+    kernel = ("bp_quad_kernel" if args.bp_quad else "bp_tile_kernel") if dominant == "bp" else "fp_kernel"
     # HBM bytes per launch under this design: the matrix data the kernel
     # streams (back: table + offsets; forward: rows per task + records) plus
     # one read of the input and one write of the output (mi_info)
@@ -400,7 +400,7 @@ def tof_bench(dev, x, steps, nsub, radius):
     out = {"pairs_per_s": round(1.0 / dt, 4), "ms_per_pair": round(dt * 1000, 3),
            "fp_kernel_ms": round(fp_ms / max(nfp, 1), 3), "bp_kernel_ms": round(bp_ms / max(nbp, 1), 3),
            "num_bins": int(pdi.num_bins), "tof_bins": int(pdi.num_tof_bins), "setup_s": round(setup_s, 3),
-           "weights": ("stored windows of %d (forward) and %d (back) TOF bins" % (info.tof_fp_window, info.tof_bp_window)
+           "weights": ("stored: forward in windows of %d TOF bins, back per TOF bin (image tiles)" % info.tof_fp_window
                        if info.tof_fp_window else "computed on the fly"),
            "live_span": int(info.tof_live_span)}
     log(f"TOF pair {dt * 1000:.2f} ms (fp {out['fp_kernel_ms']} ms, bp {out['bp_kernel_ms']} ms)")

@@ -115,14 +115,15 @@ typedef struct {
    * input and one write of the output. */
   int64_t fp_design_bytes;
   int64_t bp_design_bytes;
-  /* back projection: 1 through LDS slabs of image tiles, 0 by image column
-   * over the column table; the slab tile and its segment groups per view */
+  /* back projection: 1 through LDS slabs of image tiles (MI_TUNE_BP_SLAB), 0
+   * otherwise; the slab tile and its segment groups per view */
   int32_t slab_back_projection;
   int32_t slab_tile_x, slab_tile_y, slab_segment_groups;
   int32_t slab_lds_bytes; /* LDS of one slab workgroup */
-  /* TOF: window widths of the stored forward and back records (TOF bins per
-   * element; 0 when the weights are computed on the fly) and the widest
-   * range of TOF bins with a non-zero weight of one element */
+  /* TOF: window widths of the stored weights, forward and back (TOF bins per
+   * element; 0 when they are computed on the fly; the default back projection
+   * keeps its weights per TOF bin instead of in windows) and the widest range
+   * of TOF bins with a non-zero weight of one element */
   int32_t tof_fp_window;
   int32_t tof_bp_window;
   int32_t tof_live_span;
@@ -455,7 +456,8 @@ int mi_batch_get_estimate(mi_batch* batch, int problem, float* image);
  * fp_widen 1 doubles those groups; columns of images of at most 32 planes run
  * one per full wave (bp_pack 0), packed in lane groups (1), or one per wave
  * split into 2 or 4 parts that sum different table entries (2); tile_x x
- * tile_y orders the columns. Defaults 32, 0, 2, 32, 8. */
+ * tile_y orders the columns (taller images run by image tiles). Defaults 32, 0,
+ * 2, 32, 8. */
 int mi_batch_set_launch(mi_batch* batch, int fp_group_max, int fp_widen, int bp_pack, int tile_x, int tile_y);
 /* Forward projection in row groups: the families of one basic row with at
  * most max_axial axial positions (0: none) run up to 64 axial positions per
@@ -478,14 +480,16 @@ int mi_batch_synchronize(mi_batch* batch);
  * workgroups to XCDs: 0 in hardware order, 1 in one contiguous range per XCD,
  * k > 1 in chunks of k workgroups (4 columns each) dealt to the XCDs in turn
  * (default 64: half an 8 x 64 tile per chunk); MI_TUNE_BP_SLOT_SKIP skips z slots
- * an entry cannot reach (default off). Results do not depend on these
- * settings. MI_TUNE_FP_XCD_CHUNK maps forward-projection workgroups (4 tasks
+ * an entry cannot reach (default off). They and MI_TUNE_BP_SPLIT_SUBSETS apply
+ * to the column kernels only: families that cover whole runs (the z-shift
+ * symmetry) are back-projected by image tiles, which have no settings. Results
+ * do not depend on these settings. MI_TUNE_FP_XCD_CHUNK maps forward-projection workgroups (4 tasks
  * each) the same way: 0 one contiguous range per XCD, k > 0 chunks of k
  * (default 32).
  * MI_TUNE_BP_SLAB 1 switches the back projection of tables with one plane
  * per axial position (and images of at most 128 planes) to projection-data
- * slabs staged in LDS, one workgroup per image tile (default 0: by image
- * column over the column table, the faster of the two at mMR size);
+ * slabs staged in LDS, one workgroup per image tile (default 0: image tiles
+ * with all planes' rows in LDS, twice as fast at mMR size);
  * MI_TUNE_SLAB_TILE_X / _Y set its tile (default 8 x 8 columns),
  * MI_TUNE_SLAB_COLUMNS_PER_WAVE (2, 4 or 8, default 4) the columns each wave
  * of the tile's workgroup sums, and MI_TUNE_SLAB_LDS_KB (16-160, default 80)
@@ -505,9 +509,10 @@ int mi_batch_synchronize(mi_batch* batch);
  * one-plane tables that merges the column lists of 2 x 2 blocks of image
  * columns, and back-projects one block per wave (each projection-data run
  * gathered once for the block's four columns: 0.58 of the gathers at mMR
- * size, measured no faster); 0 (default) keeps the column kernel. Between a
- * set-up with 1 and the next, 0 and 1 switch the kernel at the next launch.
- * The two give the same sums bit for bit;
+ * size, as fast as the column kernel there and half as fast as image tiles),
+ * beside the column table; 0 (default) builds image tiles. Between a set-up
+ * with 1 and the next, 0 and 1 switch between the blocks and the column kernel
+ * at the next launch. All give the same sums bit for bit;
  * MI_TUNE_BP_QUAD_UNROLL (4, 6 or 8, default 8) sets the merged entries
  * whose gathers each wave keeps in flight.
  * MI_TUNE_BP_SPLIT_SUBSETS 1 back-projects several subsets (a plain back
