@@ -1376,6 +1376,13 @@ bool mi_ctx::build_tile_table(int span) {
   HIPCHECK(hipMemcpy(need, d_need, sizeof(need), hipMemcpyDeviceToHost));
   const int64_t nslots = 4 * static_cast<int64_t>(totals[1]);
   if (need[2]) return false;
+  {
+    // the padded lists and the sort's buffers have to fit; the other tables
+    // need less where the lists are short (a list of one entry is padded to four)
+    size_t free_b = 0, total_b = 0;
+    HIPCHECK(hipMemGetInfo(&free_b, &total_b));
+    if (8 * nslots + 32 * most > static_cast<int64_t>(free_b / 16 * 15)) return false;
+  }
   tile_hdr.alloc((nph + mi::kTileHdrSlack) * mi::kTileWaves);
   mi::launch_tile_headers(groups, group_off, phase_row, total_rows, nph, S, tile_hdr.p, stream);
   // pass 4, subset by subset: every term's list and entry, sorted by list, to
