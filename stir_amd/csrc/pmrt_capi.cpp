@@ -1354,8 +1354,9 @@ bool mi_ctx::build_tile_table(int span) {
   const uint32_t total_rows = totals[1];
   const int64_t nph = totals[0], nlists = nph * S.lines();
   if (nlists >= (int64_t{1} << 31) - 2) return false;
-  tile_row.alloc(static_cast<size_t>(total_rows) + mi::kTileRowSlack);
-  HIPCHECK(hipMemsetAsync(tile_row.p + total_rows, 0, mi::kTileRowSlack * sizeof(int2), stream));
+  const int row_slack = mi::tile_row_slack(A.stride);
+  tile_row.alloc(static_cast<size_t>(total_rows) + row_slack);
+  HIPCHECK(hipMemsetAsync(tile_row.p + total_rows, 0, row_slack * sizeof(int2), stream));
   uint32_t* phase_row = mem.get<uint32_t>(nph);
   mi::launch_tile_rows(d_units, d_unit_off, nsub, ntiles, nunits, nrng, tile_rng.p, rows, tile_phase_off.p,
                        row_off, tile_row.p, phase_row, d_need + 2, stream);

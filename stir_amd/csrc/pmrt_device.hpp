@@ -372,7 +372,41 @@ struct TileShape {
 constexpr int kTileXcdChunk = 1;      // tiles of one XCD's turn
 constexpr int kTileHdrSlack = 3;      // phases that the kernel's header read-ahead may touch past the last
 constexpr int kTileEntSlack = 512;    // entries that its chunk read-ahead may touch past the last
-constexpr int kTileRowSlack = 64 * kTileWaves;  // rows that its read-ahead may touch past the last
+// Rows that the read-ahead may touch past the last one: the kernel for tall
+// images asks for the row wave + kTileWaves * lane of the phase after the last;
+// that for short images for the rows of a wave's first kShortBatch copies there
+// (ShortCopyWalk), 2048 floats of all its copy waves: 1024 rows of the smallest
+// stride, 2.
+constexpr int kShortBatch = 8;  // row list entries of a copy wave requested together
+inline int tile_row_slack(int stride) {
+  const int tall = 64 * kTileWaves, few = (64 * kShortCopyWaves * kShortBatch - 1) / stride + 1;
+  return few > tall ? few : tall;
+}
+// The rows of a phase that lane `lane` of copy wave `wave` copies from: copy i
+// takes the phase's floats 64 (wave + kShortCopyWaves i) + lane, rows of
+// `stride` floats end to end. Its row and place in the row go from copy to copy
+// by a step and a carry. div_stride: ceil(2^32 / stride).
+struct ShortCopyWalk {
+  int stride, row_first, at_first, row_step, at_step;
+  __host__ __device__ static int quotient(int f, uint32_t div_stride) {
+    return static_cast<int>((static_cast<uint64_t>(f) * div_stride) >> 32);
+  }
+  __host__ __device__ ShortCopyWalk(int wave, int lane, int stride, uint32_t div_stride) : stride(stride) {
+    constexpr int kAdvance = kShortCopyWaves * 64;
+    const int f0 = wave * 64 + lane;
+    row_first = quotient(f0, div_stride);
+    at_first = f0 - row_first * stride;
+    row_step = quotient(kAdvance, div_stride);
+    at_step = kAdvance - row_step * stride;
+  }
+  // `at` of the next copy, in [0, stride); whether it passed the row's end
+  __host__ __device__ bool carry(int& at) const {
+    at += at_step;
+    const bool over = at >= stride;
+    at -= over ? stride : 0;
+    return over;
+  }
+};
 struct TileArgs {
   const uint32_t* phase_off;  // first phase of every (tile, subset)
   const uint4* hdr;           // per (phase, wave): first group, groups of its 8 columns (a byte each) or, in

@@ -612,7 +612,6 @@ __device__ inline void short_groups(const int* off, const int* w, const char* ld
 }
 
 constexpr int kShortThreads = kWave * (kTileWaves + kShortCopyWaves);
-constexpr int kShortBatch = 8;  // row list entries of a copy wave requested together
 
 // SUM2: the sum of a phase is added to the voxel's sum as a whole (shorter
 // chains of additions); otherwise all terms one by one, as the column kernel
@@ -643,22 +642,9 @@ __global__ void __launch_bounds__(kShortThreads, 6) bp_tile_short_kernel(TileArg
   if (cw >= 0) {
     const __amdgpu_buffer_rsrc_t all =
         __builtin_amdgcn_make_buffer_rsrc((void*)proj, static_cast<short>(0), static_cast<int>(A.proj_bytes), 0x00020000);
-    // Copy i of the wave takes the phase's floats (cw + kShortCopyWaves i) 64 to
-    // + 63; this lane's row and place in it go from copy to copy by a step and
-    // a carry. (Past the phase's last row a copy writes the next phase's floats
-    // into the buffer's slack.)
-    const int f0 = cw * kWave + lane;
-    const int row_first = static_cast<int>(__umulhi(static_cast<uint32_t>(f0), A.div_stride));
-    const int at_first = f0 - row_first * A.stride;
-    constexpr int kAdvance = kShortCopyWaves * kWave;
-    const int row_step = static_cast<int>(__umulhi(static_cast<uint32_t>(kAdvance), A.div_stride));
-    const int at_step = kAdvance - row_step * A.stride;
-    auto carry = [&](int& at) {  // at in [0, stride) again; whether it passed the end
-      at += at_step;
-      const bool over = at >= A.stride;
-      at -= over ? A.stride : 0;
-      return over;
-    };
+    // (past the phase's last row a copy writes the next phase's floats into the
+    // buffer's slack)
+    const ShortCopyWalk walk(cw, lane, A.stride, A.div_stride);
     int2 ra[kShortBatch], rb[kShortBatch];
     int row = 0, row_at = 0, at = 0;  // of the next request, of the next copy
     auto request = [&](int2 (&r)[kShortBatch], uint32_t base) {
@@ -666,7 +652,7 @@ __global__ void __launch_bounds__(kShortThreads, 6) bp_tile_short_kernel(TileArg
 #pragma unroll
       for (int j = 0; j < kShortBatch; ++j) {
         r[j] = list[row];
-        row += row_step + carry(row_at);
+        row += walk.row_step + walk.carry(row_at);
       }
     };
     auto copy = [&](const int2 (&r)[kShortBatch], int first, int n, float* buf) {
@@ -685,14 +671,14 @@ __global__ void __launch_bounds__(kShortThreads, 6) bp_tile_short_kernel(TileArg
           const int v = ok ? static_cast<int>(4U * static_cast<unsigned>(r[j].x + a)) : -4;  // -4: reads 0
           __builtin_amdgcn_raw_ptr_buffer_load_lds(all, (__attribute__((address_space(3))) void*)(buf + f), 4,
                                                    whole_offset(v), 0, 0, 0);
-          carry(at);
+          walk.carry(at);
         }
       }
     };
     uint32_t row0 = hp[0].w, row1 = hp[kTileWaves].w;
     int nrow = static_cast<int>(__builtin_amdgcn_readfirstlane(row1) - __builtin_amdgcn_readfirstlane(row0));
-    row = row_first;
-    row_at = at_first;
+    row = walk.row_first;
+    row_at = walk.at_first;
     request(ra, row0);
     int which = 0;
     for (uint32_t p = p0; p <= p1; ++p) {
@@ -701,7 +687,7 @@ __global__ void __launch_bounds__(kShortThreads, 6) bp_tile_short_kernel(TileArg
         which ^= 1;
         const int n = nrow * A.stride;
         auto any = [&](int first) { return (cw + kShortCopyWaves * first) * kWave < n; };
-        at = at_first;
+        at = walk.at_first;
         for (int first = 0; any(first); first += 2 * kShortBatch) {
           const bool second = any(first + kShortBatch);
           if (second) request(rb, row0);
@@ -714,8 +700,8 @@ __global__ void __launch_bounds__(kShortThreads, 6) bp_tile_short_kernel(TileArg
         row0 = row1;
         row1 = hp[kTileWaves].w;
         nrow = static_cast<int>(__builtin_amdgcn_readfirstlane(row1) - __builtin_amdgcn_readfirstlane(row0));
-        row = row_first;
-        row_at = at_first;
+        row = walk.row_first;
+        row_at = walk.at_first;
         request(ra, row0);
         __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's rows are in LDS
       }
