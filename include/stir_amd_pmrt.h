@@ -519,14 +519,32 @@ int mi_batch_synchronize(mi_batch* batch);
  * projection of all subsets) in one launch per subset, each continuing the
  * sums the previous one left in the image (the same sums bit for bit as one
  * launch; a working set of one subset's projection data; 2 % faster at mMR
- * size); 0 (default) in one launch. */
+ * size); 0 (default) in one launch.
+ * MI_TUNE_BP_IMAGE_TILES 0 keeps a set-up from building image tiles (column
+ * table or TOF records instead); 1 (default) builds them where they apply; it
+ * takes effect at the next set-up. mi_get_projection_kernels tells which
+ * kernels run. */
 enum { MI_TUNE_BP_TILE_X = 1, MI_TUNE_BP_TILE_Y = 2, MI_TUNE_BP_XCD_REMAP = 3, MI_TUNE_BP_SLOT_SKIP = 4,
        MI_TUNE_FP_XCD_CHUNK = 5, MI_TUNE_BP_SLAB = 6, MI_TUNE_SLAB_TILE_X = 7, MI_TUNE_SLAB_TILE_Y = 8,
        MI_TUNE_SLAB_COLUMNS_PER_WAVE = 9, MI_TUNE_SLAB_LDS_KB = 10, MI_TUNE_TOF_ROWS = 11, MI_TUNE_BP_QUAD = 12,
-       MI_TUNE_BP_QUAD_UNROLL = 13, MI_TUNE_BP_SPLIT_SUBSETS = 14 };
+       MI_TUNE_BP_QUAD_UNROLL = 13, MI_TUNE_BP_SPLIT_SUBSETS = 14, MI_TUNE_BP_IMAGE_TILES = 15 };
 int mi_set_tuning(mi_ctx* ctx, int param, int value);
 
 /* ---- diagnostics ----------------------------------------------------------- */
+/* The kernels that projections of a subset (-1: all subsets) run on after a
+ * set-up. */
+enum { MI_FORWARD_TASKS = 0,      /* a family or pair of families per wave */
+       MI_FORWARD_ROW_GROUPS = 1, /* the families of a basic row packed into waves */
+       MI_FORWARD_TOF_ROWS = 2,   /* stored TOF weights */
+       MI_FORWARD_TOF = 3 };      /* TOF weights computed on the fly */
+enum { MI_BACK_COLUMNS = 0,       /* an image column per wave */
+       MI_BACK_BLOCKS = 1,        /* 2 x 2 columns (MI_TUNE_BP_QUAD) */
+       MI_BACK_SLABS = 2,         /* MI_TUNE_BP_SLAB */
+       MI_BACK_TILES = 3,         /* image tiles, columns of more than 32 planes */
+       MI_BACK_SHORT_TILES = 4,   /* image tiles, up to 32 planes */
+       MI_BACK_TOF_ROWS = 5,      /* stored TOF weights by column */
+       MI_BACK_TOF = 6 };         /* TOF weights computed on the fly */
+int mi_get_projection_kernels(mi_ctx* ctx, int subset, int32_t* forward, int32_t* back);
 /* No counterpart in the reference (its TimedObject timers are CPU/wall clocks,
  * TimedObject.h:45-57). When enabled, every forward- and back-projection kernel
  * launch of the context is bracketed by HIP events recorded on the stream it

@@ -32,7 +32,7 @@ EXPORTED_SYMBOLS = (
     "mi_relative_difference_prior_dev", "mi_batch_set_row_groups", "mi_lm_set_events",
     "mi_prior_hessian_times_input_dev", "mi_basic_view_segments_in_subset", "mi_set_image",
     "mi_forward_project_view_segments", "mi_back_project_view_segments", "mi_quadratic_prior_noalloc_dev",
-    "mi_obj_hessian_times_input_dev",
+    "mi_obj_hessian_times_input_dev", "mi_get_projection_kernels",
 )
 
 MI_PRIOR_NONE, MI_PRIOR_QUADRATIC, MI_PRIOR_RELATIVE_DIFFERENCE = 0, 1, 2
@@ -56,6 +56,11 @@ MI_TUNE_TOF_ROWS = 11
 MI_TUNE_BP_QUAD = 12
 MI_TUNE_BP_QUAD_UNROLL = 13
 MI_TUNE_BP_SPLIT_SUBSETS = 14
+MI_TUNE_BP_IMAGE_TILES = 15
+
+MI_FORWARD_TASKS, MI_FORWARD_ROW_GROUPS, MI_FORWARD_TOF_ROWS, MI_FORWARD_TOF = 0, 1, 2, 3
+MI_BACK_COLUMNS, MI_BACK_BLOCKS, MI_BACK_SLABS, MI_BACK_TILES, MI_BACK_SHORT_TILES = 0, 1, 2, 3, 4
+MI_BACK_TOF_ROWS, MI_BACK_TOF = 5, 6
 
 
 class NativeError(RuntimeError):
@@ -115,6 +120,7 @@ def load():
     L.mi_ctx_destroy.restype = None
     L.mi_set_up.argtypes = [vp, ctypes.POINTER(GeometryStruct), c_int]
     L.mi_get_info.argtypes = [vp, ctypes.POINTER(InfoStruct)]
+    L.mi_get_projection_kernels.argtypes = [vp, c_int, ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_int32)]
     L.mi_subsets_balanced.argtypes = [vp, ctypes.POINTER(c_int)]
     L.mi_subset_view_segments.argtypes = [vp, c_int, _i32p, _i32p, c_int, ctypes.POINTER(c_int)]
     L.mi_get_row.argtypes = [vp, c_int, c_int, c_int, c_int, _i16p, _i16p, _i16p, _f32p, c_int, ctypes.POINTER(c_int)]
@@ -213,6 +219,13 @@ class Context:
         out = InfoStruct()
         check(load().mi_get_info(self._h, ctypes.byref(out)), "mi_get_info")
         return out
+
+    def projection_kernels(self, subset: int = -1):
+        """(forward, back): the MI_FORWARD_* and MI_BACK_* kernels that projections of the subset (-1: all) run on."""
+        f, b = ctypes.c_int32(), ctypes.c_int32()
+        check(load().mi_get_projection_kernels(self._h, int(subset), ctypes.byref(f), ctypes.byref(b)),
+              "mi_get_projection_kernels")
+        return f.value, b.value
 
     def set_tuning(self, param: int, value: int) -> None:
         check(load().mi_set_tuning(self._h, int(param), int(value)), "mi_set_tuning")

@@ -172,6 +172,7 @@ struct mi_ctx {
   void build_quad_table(const uint32_t* d_perm, int64_t n, const int64_t* d_famoff);
   // back projection by image tiles with the runs in LDS (pmrt_tile.hip), the
   // default where build_tile_table accepts the geometry
+  int tiles_enable = 1;  // MI_TUNE_BP_IMAGE_TILES
   bool use_tile = false;
   int64_t tile_entries = 0;
   std::vector<uint32_t> tile_work;  // groups of entries of every tile
@@ -322,6 +323,11 @@ struct mi_ctx {
                       dst_stir, st);
   }
 
+  // MI_FORWARD_*
+  int forward_kernel() const {
+    if (ntof > 1) return tof_fp_w > 0 ? MI_FORWARD_TOF_ROWS : MI_FORWARD_TOF;
+    return use_rows ? MI_FORWARD_ROW_GROUPS : MI_FORWARD_TASKS;
+  }
   // ---- projections on device-layout buffers
   void fp(mi::FpMode mode, const float* d_img, float* d_out, int subset, const mi::FpData& data, hipStream_t st) {
     const int tb = task_off[subset_begin(subset)], te = task_off[subset_end(subset)];
@@ -394,35 +400,48 @@ struct mi_ctx {
     mi::launch_transpose(stage_sino.p + slot, d_proj + blk + static_cast<int64_t>(view) * nt * nax, nax, nt, nt, nax, st);
   }
   DBuf<float> input_img;  // the image of mi_set_image (device layout)
+  // MI_BACK_* of the set-up's tables (nontof as in bp)
+  int back_kernel(bool nontof = false) const {
+    if (ntof > 1 && !nontof) {
+      if (use_tile) return tile.shape.lanes < 64 ? MI_BACK_SHORT_TILES : MI_BACK_TILES;
+      return tof_bp_rec.n ? MI_BACK_TOF_ROWS : MI_BACK_TOF;
+    }
+    if (use_slab) return MI_BACK_SLABS;
+    if (use_tile && ntof == 1) return tile.shape.lanes < 64 ? MI_BACK_SHORT_TILES : MI_BACK_TILES;
+    return use_quad() ? MI_BACK_BLOCKS : MI_BACK_COLUMNS;
+  }
   // nontof: back-project one non-TOF block with the non-TOF values of the
   // table (the sensitivity of TOF data, unless TOF sensitivities are asked for)
   void bp(mi::BpMode mode, const float* d_proj, float* d_img, int subset, const mi::BpData& data, hipStream_t st,
           bool nontof = false) {
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (timing) { e0 = take_event(); e1 = take_event(); HIPCHECK(hipEventRecord(e0, st)); }
-    if (ntof > 1 && !nontof && use_tile)
-      mi::launch_back_project_tile(mode, tile, subset_begin(subset), subset_end(subset), d_proj, d_img, dims, data,
-                                   st);
-    else if (ntof > 1 && !nontof && tof_bp_rec.n)
-      mi::launch_back_project_tof_rows(mode, uniform_ppa, list_off.p, tof_bp_rec.p, tof_bp_w,
-                                       static_cast<int64_t>(tof_bp_rec.n / mi::tof_bp_words(tof_bp_w)) - 1,
-                                       subset_begin(subset), subset_end(subset), d_proj, d_img, dims, tofc, data,
-                                       tof_bp_tuning, st);
-    else if (ntof > 1 && !nontof)
-      mi::launch_back_project_tof(mode, uniform_ppa, list_off.p, entries.p, entry_d.p, subset_begin(subset),
-                                  subset_end(subset), d_proj, d_img, dims, tofc, data, tof_bp_tuning, st);
-    else if (use_slab)
-      mi::launch_back_project_slab(mode, slab, subset_begin(subset), subset_end(subset), d_proj, d_img, dims, data,
-                                   st);
-    else if (use_tile && ntof == 1)
-      mi::launch_back_project_tile(mode, tile, subset_begin(subset), subset_end(subset), d_proj, d_img, dims, data,
-                                   st);
-    else if (use_quad())
-      mi::launch_back_project_quad(mode, quad_off.p, quad_ent.p, subset_begin(subset), subset_end(subset), d_proj,
-                                   d_img, dims, data, bp_tuning, st, block_bins);
-    else
-      mi::launch_back_project(mode, uniform_ppa, list_off.p, entries.p, subset_begin(subset), subset_end(subset), d_proj,
-                              d_img, dims, data, bp_tuning, st, block_bins);
+    const int sb = subset_begin(subset), se = subset_end(subset);
+    switch (back_kernel(nontof)) {
+      case MI_BACK_TILES:
+      case MI_BACK_SHORT_TILES:
+        mi::launch_back_project_tile(mode, tile, sb, se, d_proj, d_img, dims, data, st);
+        break;
+      case MI_BACK_TOF_ROWS:
+        mi::launch_back_project_tof_rows(mode, uniform_ppa, list_off.p, tof_bp_rec.p, tof_bp_w,
+                                         static_cast<int64_t>(tof_bp_rec.n / mi::tof_bp_words(tof_bp_w)) - 1, sb, se,
+                                         d_proj, d_img, dims, tofc, data, tof_bp_tuning, st);
+        break;
+      case MI_BACK_TOF:
+        mi::launch_back_project_tof(mode, uniform_ppa, list_off.p, entries.p, entry_d.p, sb, se, d_proj, d_img, dims,
+                                    tofc, data, tof_bp_tuning, st);
+        break;
+      case MI_BACK_SLABS:
+        mi::launch_back_project_slab(mode, slab, sb, se, d_proj, d_img, dims, data, st);
+        break;
+      case MI_BACK_BLOCKS:
+        mi::launch_back_project_quad(mode, quad_off.p, quad_ent.p, sb, se, d_proj, d_img, dims, data, bp_tuning, st,
+                                     block_bins);
+        break;
+      default:
+        mi::launch_back_project(mode, uniform_ppa, list_off.p, entries.p, sb, se, d_proj, d_img, dims, data, bp_tuning,
+                                st, block_bins);
+    }
     if (timing) { HIPCHECK(hipEventRecord(e1, st)); bp_events.emplace_back(e0, e1); }
   }
 
@@ -1210,7 +1229,9 @@ bool mi_ctx::build_slab_table() {
 // of one element.
 bool mi_ctx::build_tile_table(int span) {
   const mi_geometry& g = plan->geometry();
-  if ((in_batch && dims.nz <= mi::kTileShortPlanes) || slab_enable || quad_enable || dims.nz > 256 || h_fams.empty()) return false;
+  if (!tiles_enable || (in_batch && dims.nz <= mi::kTileShortPlanes) || slab_enable || quad_enable || dims.nz > 256 ||
+      h_fams.empty())
+    return false;
   if (total_bins() >= (int64_t{1} << 31) || (ntof > 1 && tof_fp_w <= 0)) return false;
   const int32_t* rec = ntof > 1 ? tof_fp_rec.p : nullptr;
   const auto& keys = plan->family_keys();
@@ -2675,6 +2696,10 @@ int mi_set_tuning(mi_ctx* ctx, int param, int value) {
         if (value < 0 || value > 1) throw ApiError(MI_ERR_ARGUMENT, "the subset split switch must be 0 or 1");
         ctx->bp_tuning.split_subsets = value;
         break;
+      case MI_TUNE_BP_IMAGE_TILES:
+        if (value < 0 || value > 1) throw ApiError(MI_ERR_ARGUMENT, "the image tile switch must be 0 or 1");
+        ctx->tiles_enable = value;
+        break;
       default: throw ApiError(MI_ERR_ARGUMENT, "unknown tuning parameter");
     }
   });
@@ -2710,6 +2735,16 @@ int mi_get_kernel_timing(mi_ctx* ctx, double* fp_ms, int64_t* fp_launches, doubl
     if (fp_launches) *fp_launches = static_cast<int64_t>(ctx->fp_events.size());
     if (bp_launches) *bp_launches = static_cast<int64_t>(ctx->bp_events.size());
     ctx->release_events();
+  });
+}
+
+int mi_get_projection_kernels(mi_ctx* ctx, int subset, int32_t* forward, int32_t* back) {
+  return guarded([&] {
+    if (!ctx || !forward || !back) throw ApiError(MI_ERR_ARGUMENT, "NULL argument");
+    ctx->require_setup();
+    ctx->check_subset(subset);
+    *forward = ctx->forward_kernel();
+    *back = ctx->back_kernel();
   });
 }
 

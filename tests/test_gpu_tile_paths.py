@@ -1,0 +1,81 @@
+"""Back projections by image tiles, with the kernels that run on either side
+named by the library: tiles (MI_TUNE_BP_IMAGE_TILES 1, the default) against the
+column kernels or stored TOF records (MI_TUNE_BP_IMAGE_TILES 0), GPU.
+
+The geometries and tolerances are those of test_gpu_tile.py, test_gpu_tile_short.py
+and test_gpu_tile_tof.py. An infinite bin at the centre of a direct sinogram
+reaches voxels on both sides, the same ones, and leaves no NaN.
+"""
+import numpy as np
+import pytest
+
+import test_gpu_tile
+import test_gpu_tile_short
+import test_gpu_tile_tof
+from stir_amd import _native
+from stir_amd.geometry import ProjDataInfoCylindrical, RayTracingMatrixParameters, Scanner, VoxelsOnCartesianGrid
+from stir_amd.projectors import ProjectorByBinPairMI355X, ProjMatrixByBinUsingRayTracing
+
+pytestmark = pytest.mark.gpu
+
+NAMES = ([("tall", n) for n in sorted(test_gpu_tile.CASES)] + [("short", n) for n in sorted(test_gpu_tile_short.CASES)] +
+         [("tof", n) for n in sorted(test_gpu_tile_tof.CASES)])
+
+
+def geometry(kind, name):
+    """(projection data, image, parameters, kernel of the tiles, of the other side, the same bits)"""
+    if kind == "tall":
+        rings, crystals, span, mrd, views, tang, nz, ny, nx, vz, pm = test_gpu_tile.CASES[name]
+        sc = Scanner.cylindrical(rings, crystals, 100.0, 4.0, name=name)
+        pdi = ProjDataInfoCylindrical.construct(sc, span=span, max_delta=mrd, num_views=views, num_tangential_poss=tang)
+        return (pdi, VoxelsOnCartesianGrid(nz, ny, nx, vz, 2.5, 2.5), RayTracingMatrixParameters(**pm),
+                _native.MI_BACK_TILES, _native.MI_BACK_COLUMNS, True)
+    if kind == "short":
+        rings, span, mrd, views, nz, ny, nx, vz, ntof, same = test_gpu_tile_short.CASES[name]
+        sc = Scanner(name, rings, 2 * views, 100.0, 0.0, 4.0, 4.0, 0.0, 44, 44, 400.0 if ntof else 0.0,
+                     2500.0 / ntof if ntof else 0.0, ntof)
+        tiles = _native.MI_BACK_SHORT_TILES
+    else:
+        rings, span, mrd, nz, ny, nx, ntof, ps = test_gpu_tile_tof.CASES[name]
+        views, vz, same = 32, 2.0, False
+        sc = Scanner(name, rings, 64, 100.0, 0.0, 4.0, 4.0, 0.0, 44, 44, 400.0, ps, ntof)
+        tiles = _native.MI_BACK_TILES
+    pdi = ProjDataInfoCylindrical.construct(sc, span, mrd, views, 44, False)
+    if ntof:
+        pdi = pdi.with_tof(1)
+    return (pdi, VoxelsOnCartesianGrid(nz, ny, nx, vz, 2.5, 2.5), RayTracingMatrixParameters(), tiles,
+            _native.MI_BACK_TOF_ROWS if ntof else _native.MI_BACK_COLUMNS, same)
+
+
+def make(pdi, img, pm, tiles, num_subsets=4):
+    P = ProjectorByBinPairMI355X(ProjMatrixByBinUsingRayTracing(pm))
+    P.context.set_tuning(_native.MI_TUNE_BP_IMAGE_TILES, tiles)
+    P.set_up(pdi, img, num_subsets=num_subsets)
+    return P
+
+
+@pytest.mark.parametrize("kind,name", NAMES)
+def test_tiles_against_columns(kind, name):
+    pdi, img, pm, tiles, other, same = geometry(kind, name)
+    print(f"[tile paths] {kind} {name}: {pdi.num_bins} bins, image {img.shape}", flush=True)
+    T, C = make(pdi, img, pm, 1), make(pdi, img, pm, 0)
+    for subset in (-1, 3):
+        assert T.context.projection_kernels(subset)[1] == tiles
+        assert C.context.projection_kernels(subset)[1] == other
+    rng = np.random.default_rng(91)
+    terms = pdi.num_views * (2 * pdi.max_segment_num + 1) * 3 * max(T.info().tof_live_span, 1)
+    mean = terms / 100.0
+    for subset in (-1, 0, 3):
+        y = rng.uniform(0.5, 2.0, pdi.num_bins).astype(np.float32)
+        y[rng.uniform(size=pdi.num_bins) > 0.01] = 0.0
+        a, b = T.back_project(y, subset=subset), C.back_project(y, subset=subset)
+        assert b.max() > 0
+        assert test_gpu_tile_short.same_or_close(a, b, same, mean + 16.0 * np.sqrt(mean) + 16.0), subset
+    y = rng.uniform(0.5, 2.0, pdi.num_bins).astype(np.float32)
+    block = pdi.num_bins // max(pdi.num_tof_bins, 1)
+    y[pdi.num_tof_bins // 2 * block + pdi.bin_index(0, 5, pdi.num_axial_poss_of(0) // 2, 1)] = np.inf
+    a, b = T.back_project(y), C.back_project(y)
+    assert np.isinf(b).any()
+    assert not np.isnan(a).any() and np.array_equal(np.isinf(a), np.isinf(b))
+    T.close()
+    C.close()
