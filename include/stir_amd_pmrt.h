@@ -521,9 +521,10 @@ int mi_batch_synchronize(mi_batch* batch);
  * launch; a working set of one subset's projection data; 2 % faster at mMR
  * size); 0 (default) in one launch.
  * MI_TUNE_BP_IMAGE_TILES 0 keeps a set-up from building image tiles (column
- * table or TOF records instead); 1 (default) builds them where they apply; it
- * takes effect at the next set-up. mi_get_projection_kernels tells which
- * kernels run. */
+ * table or TOF records instead), 1 (default) builds them where they are the
+ * faster ones (images of more than 32 planes need enough tiles to fill the
+ * GPU), 2 wherever the geometry allows them; it takes effect at the next
+ * set-up. mi_get_projection_kernels tells which kernels run. */
 enum { MI_TUNE_BP_TILE_X = 1, MI_TUNE_BP_TILE_Y = 2, MI_TUNE_BP_XCD_REMAP = 3, MI_TUNE_BP_SLOT_SKIP = 4,
        MI_TUNE_FP_XCD_CHUNK = 5, MI_TUNE_BP_SLAB = 6, MI_TUNE_SLAB_TILE_X = 7, MI_TUNE_SLAB_TILE_Y = 8,
        MI_TUNE_SLAB_COLUMNS_PER_WAVE = 9, MI_TUNE_SLAB_LDS_KB = 10, MI_TUNE_TOF_ROWS = 11, MI_TUNE_BP_QUAD = 12,

@@ -12,6 +12,7 @@
 #include <string>
 #include <unordered_map>
 #include <deque>
+#include <map>
 #include <vector>
 
 #include "pmrt_device.hpp"
@@ -173,6 +174,7 @@ struct mi_ctx {
   // back projection by image tiles with the runs in LDS (pmrt_tile.hip), the
   // default where build_tile_table accepts the geometry
   int tiles_enable = 1;  // MI_TUNE_BP_IMAGE_TILES
+  int batch_tiles = 0;   // in a batch: the tiles that one launch takes from all its problems
   bool use_tile = false;
   int64_t tile_entries = 0;
   std::vector<uint32_t> tile_work;  // groups of entries of every tile
@@ -193,7 +195,8 @@ struct mi_ctx {
     return static_cast<int64_t>(tile_phase_off.bytes() + tile_hdr.bytes() + tile_row.bytes() + tile_off.bytes() +
                                 tile_order.bytes() + tile_w.bytes());
   }
-  bool build_tile_table(int span);
+  bool build_tile_table(int span, double terms);
+  int min_tiles(double terms) const;
   std::vector<mi::Family> h_fams;
   std::unordered_map<int64_t, int> fam_lookup;  // (seg,view,tang,a0) -> family
   int64_t num_basic_elements = 0;
@@ -796,7 +799,7 @@ void mi_ctx::build_table() {
   release_slab();
   release_tile();
   if (ntof == 1) {
-    if (build_tile_table(1)) {
+    if (build_tile_table(1, 1.0)) {
       use_tile = true;
       return;
     }
@@ -957,13 +960,14 @@ void mi_ctx::build_tof_rows(int64_t n) {
   std::sort(rows.begin(), rows.end());
   for (size_t i = 1; i < rows.size(); ++i)
     if (rows[i - 1].first + rows[i - 1].second > rows[i].first) return;
-  DBuf<int> span;
-  span.alloc(1);
-  HIPCHECK(hipMemsetAsync(span.p, 0, sizeof(int), stream));
-  mi::launch_tof_live_span(entries.p, entry_d.p, n, tofc, span.p, stream);
-  int s = 0;
-  HIPCHECK(hipMemcpyAsync(&s, span.p, sizeof(int), hipMemcpyDeviceToHost, stream));
+  DBuf<unsigned long long> span;  // the widest live range, the sum of all
+  span.alloc(2);
+  HIPCHECK(hipMemsetAsync(span.p, 0, span.bytes(), stream));
+  mi::launch_tof_live_span(entries.p, entry_d.p, n, tofc, reinterpret_cast<int*>(span.p), span.p + 1, stream);
+  unsigned long long hspan[2];
+  HIPCHECK(hipMemcpyAsync(hspan, span.p, sizeof(hspan), hipMemcpyDeviceToHost, stream));
   HIPCHECK(hipStreamSynchronize(stream));
+  const int s = static_cast<int>(hspan[0]);
   tof_live_span = s;
   int fnt, fw, bw;
   if (tof_rows_mode == 1 && ntof <= 12 && s <= mi::kTofFpNarrow) {
@@ -993,7 +997,7 @@ void mi_ctx::build_tof_rows(int64_t n) {
   tof_bp_w = bw;
   // the back projection by image tiles instead of back records (narrow windows
   // only: mode 2 keeps the records)
-  if (tof_rows_mode == 1 && build_tile_table(s)) {
+  if (tof_rows_mode == 1 && build_tile_table(s, static_cast<double>(hspan[1]) / static_cast<double>(n))) {
     use_tile = true;
     HIPCHECK(hipStreamSynchronize(stream));
     entry_d.release();
@@ -1223,14 +1227,63 @@ bool mi_ctx::build_slab_table() {
   return true;
 }
 
+// Tiles of 8 x 8 columns that hold voxels of the field of view: the circle, or
+// the square around it, that the ray tracing is restricted to.
+static int fov_tiles(const mi_geometry& g) {
+  if (g.nx < 1 || g.ny < 1 || g.nx > 1022 || g.ny > 1022) return 0;  // (refused by the plan)
+  const int max_x = g.nx - 1 + g.min_x, max_y = g.ny - 1 + g.min_y;
+  const double r = std::min({-g.min_x, max_x, -g.min_y, max_y}) + 0.5;
+  // distance of the centre to the columns lo .. hi
+  auto dist = [](int lo, int hi) { return lo <= 0 && hi >= 0 ? 0 : std::min(std::abs(lo), std::abs(hi)); };
+  int n = 0;
+  for (int y = g.min_y; y <= max_y; y += 8)
+    for (int x = g.min_x; x <= max_x; x += 8) {
+      const double dx = dist(x, std::min(x + 7, max_x)), dy = dist(y, std::min(y + 7, max_y));
+      if (g.restrict_to_cylindrical_FOV ? dx * dx + dy * dy <= r * r : dx <= r && dy <= r) ++n;
+    }
+  return n;
+}
+
+// The tiles with work from which on the back projection of images of more than
+// kTileShortPlanes planes by tiles is faster than by columns. A tile is one
+// workgroup and takes its time whatever their number, up to three per CU; the
+// column kernels start four columns per workgroup and fill the chip sooner. So
+// the line is a number of tiles: of how many tiles one, alone on its CU, takes
+// as long as the column kernel for the whole image. Measured on square images
+// of 56 to 300 columns a side, where both are as fast (tiles in the field of
+// view), for one plane per axial position, two, and mixed ones:
+//   one plane, 47 to 219 planes: 300 to 390 (45 tiles: a third to a quarter as
+//   fast; 852: 1.3 times);
+//   two: 35 and 46 planes 260, 79 to 219 planes 120 to 150 (a wave of the
+//   column kernel has half of its lanes on the other parity);
+//   mixed: 39 and 47 planes 130 to 140, 65 and 79 planes 80 to 95;
+//   four (z zoom): 2.1 times as fast at 45.
+// TOF, against the stored records of 5 or 13 weights: tiles take a term per
+// live TOF bin, records a gather per weight, so the line goes with the mean
+// number of live bins: 9 bins (4.1 live) one plane 330 to 414, mixed 175 to
+// 230, two planes 185 (35 planes) and 85 to 112 (79 and 127); 3, 5 and 7 bins
+// 160, 178 and 245; records of 13 weights, 13 and 16 bins 180 and 232.
+int mi_ctx::min_tiles(double terms) const {
+  const bool one_slot = dims.nz <= 64;
+  if (ntof == 1) {
+    if (uniform_ppa == 1) return 350;
+    if (uniform_ppa == 2) return one_slot ? 260 : 150;
+    return uniform_ppa == 0 ? (one_slot ? 135 : 95) : 24;
+  }
+  const double per_term = uniform_ppa == 1 ? 92.0 : uniform_ppa == 2 ? (one_slot ? 45.0 : 27.0) : 55.0;
+  return static_cast<int>(per_term * terms * (tof_bp_w > mi::kTofBpNarrow ? 0.45 : 1.0));
+}
+
 // The tile table (pmrt_tile.hip) of a matrix whose families cover whole runs;
-// false where the geometry does not qualify (the column kernels are used
-// then). TOF matrices: from the stored forward records, span the most TOF bins
-// of one element.
-bool mi_ctx::build_tile_table(int span) {
+// false where the geometry does not qualify or the column kernels are faster
+// (they are used then). TOF matrices: from the stored forward records, span the
+// most TOF bins of one element, terms their mean number.
+bool mi_ctx::build_tile_table(int span, double terms) {
   const mi_geometry& g = plan->geometry();
   if (!tiles_enable || (in_batch && dims.nz <= mi::kTileShortPlanes) || slab_enable || quad_enable || dims.nz > 256 ||
       h_fams.empty())
+    return false;
+  if (tiles_enable == 1 && dims.nz > mi::kTileShortPlanes && std::max(fov_tiles(g), batch_tiles) < min_tiles(terms))
     return false;
   if (total_bins() >= (int64_t{1} << 31) || (ntof > 1 && tof_fp_w <= 0)) return false;
   const int32_t* rec = ntof > 1 ? tof_fp_rec.p : nullptr;
@@ -2697,7 +2750,7 @@ int mi_set_tuning(mi_ctx* ctx, int param, int value) {
         ctx->bp_tuning.split_subsets = value;
         break;
       case MI_TUNE_BP_IMAGE_TILES:
-        if (value < 0 || value > 1) throw ApiError(MI_ERR_ARGUMENT, "the image tile switch must be 0 or 1");
+        if (value < 0 || value > 2) throw ApiError(MI_ERR_ARGUMENT, "the image tile switch must be 0, 1 or 2");
         ctx->tiles_enable = value;
         break;
       default: throw ApiError(MI_ERR_ARGUMENT, "unknown tuning parameter");
@@ -3086,12 +3139,17 @@ int mi_batch_create(int device, int n, const mi_geometry* geometries, int num_su
     b->nsub = num_subsets;
     HIPCHECK(hipSetDevice(device));
     HIPCHECK(hipStreamCreate(&b->stream));
+    // the tall images of one slot count share a launch
+    std::map<int, int> tiles;
+    for (int i = 0; i < n; ++i)
+      if (geometries[i].nz > mi::kTileShortPlanes) tiles[(geometries[i].nz - 1) / 64] += fov_tiles(geometries[i]);
     for (int i = 0; i < n; ++i) {
       if (geometries[i].num_tof_bins > 1) throw ApiError(MI_ERR_ARGUMENT, "batched problems are non-TOF");
       mi_ctx* c = nullptr;
       if (mi_ctx_create(device, &c) != MI_OK) throw ApiError(MI_ERR_DEVICE, g_last_error);
       b->probs.push_back(c);
       c->in_batch = true;
+      c->batch_tiles = tiles[(std::max(geometries[i].nz, 1) - 1) / 64];
       if (mi_set_up(c, &geometries[i], num_subsets) != MI_OK)
         throw ApiError(MI_ERR_ARGUMENT, "problem " + std::to_string(i) + ": " + g_last_error);
     }

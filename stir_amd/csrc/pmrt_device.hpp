@@ -214,9 +214,10 @@ constexpr int kTofBpNarrow = 5, kTofBpWide = 13;  // back window widths (8- and 
 constexpr int tof_fp_words(int w) { return 2 + w; }
 constexpr int tof_bp_words(int w) { return 3 + w; }
 // widest live range (khi - klo + 1 over bins with a non-zero weight) of the
-// table entries [0, n) into *d_span (atomic max; *d_span zeroed by the caller)
+// table entries [0, n) into *d_span (atomic max) and the sum of the ranges into
+// *d_total (both zeroed by the caller)
 void launch_tof_live_span(const BpEntry* d_entries, const float* d_entry_d, int64_t n, const TofConsts& tof,
-                          int* d_span, hipStream_t stream);
+                          int* d_span, unsigned long long* d_total, hipStream_t stream);
 // forward records of the families' rows (rows must not overlap); nt, w: the
 // forward kernel's accumulator count and window width; the run lengths are
 // filled in by the second launch

@@ -437,8 +437,9 @@ __device__ inline void live_range(const float (&tw)[NT], int& klo, int& khi) {
 }
 
 __global__ void tof_live_span_kernel(const BpEntry* __restrict__ ent, const float* __restrict__ ent_d, int64_t n,
-                                     TofConsts T, int* __restrict__ span) {
+                                     TofConsts T, int* __restrict__ span, unsigned long long* __restrict__ total) {
   int best = 0;
+  unsigned long long sum = 0;
   for (int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; i < n;
        i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
     float tw[kMaxTofBins];
@@ -446,9 +447,16 @@ __global__ void tof_live_span_kernel(const BpEntry* __restrict__ ent, const floa
     int klo, khi;
     live_range(tw, klo, khi);
     best = max(best, khi - klo + 1);
+    sum += static_cast<unsigned>(max(khi - klo + 1, 0));
   }
-  for (int off = kWave / 2; off > 0; off >>= 1) best = max(best, __shfl_xor(best, off, kWave));
-  if (threadIdx.x % kWave == 0) atomicMax(span, best);
+  for (int off = kWave / 2; off > 0; off >>= 1) {
+    best = max(best, __shfl_xor(best, off, kWave));
+    sum += __shfl_xor(sum, off, kWave);
+  }
+  if (threadIdx.x % kWave == 0) {
+    atomicMax(span, best);
+    atomicAdd(total, sum);
+  }
 }
 
 // one wave per family, lanes over its row; the same weights as fp_tof_task
@@ -841,10 +849,10 @@ unsigned elementwise_blocks(int64_t n) { return static_cast<unsigned>(std::min<i
 }  // namespace
 
 void launch_tof_live_span(const BpEntry* d_entries, const float* d_entry_d, int64_t n, const TofConsts& tof,
-                          int* d_span, hipStream_t stream) {
+                          int* d_span, unsigned long long* d_total, hipStream_t stream) {
   if (n <= 0) return;
   hipLaunchKernelGGL(tof_live_span_kernel, dim3(elementwise_blocks(n)), dim3(256), 0, stream, d_entries, d_entry_d, n,
-                     tof, d_span);
+                     tof, d_span, d_total);
 }
 
 void launch_tof_fp_records(const Family* d_fams, int nfam, const FamilyLor* d_lors, const int2* d_pool,

@@ -1,6 +1,7 @@
 """Back projections by image tiles, with the kernels that run on either side
-named by the library: tiles (MI_TUNE_BP_IMAGE_TILES 1, the default) against the
-column kernels or stored TOF records (MI_TUNE_BP_IMAGE_TILES 0), GPU.
+named by the library: tiles (MI_TUNE_BP_IMAGE_TILES 2: wherever the geometry
+allows them) against the column kernels or stored TOF records
+(MI_TUNE_BP_IMAGE_TILES 0), GPU; and which of them the default takes.
 
 The geometries and tolerances are those of test_gpu_tile.py, test_gpu_tile_short.py
 and test_gpu_tile_tof.py. An infinite bin at the centre of a direct sinogram
@@ -58,7 +59,7 @@ def make(pdi, img, pm, tiles, num_subsets=4):
 def test_tiles_against_columns(kind, name):
     pdi, img, pm, tiles, other, same = geometry(kind, name)
     print(f"[tile paths] {kind} {name}: {pdi.num_bins} bins, image {img.shape}", flush=True)
-    T, C = make(pdi, img, pm, 1), make(pdi, img, pm, 0)
+    T, C = make(pdi, img, pm, 2), make(pdi, img, pm, 0)
     for subset in (-1, 3):
         assert T.context.projection_kernels(subset)[1] == tiles
         assert C.context.projection_kernels(subset)[1] == other
@@ -79,3 +80,39 @@ def test_tiles_against_columns(kind, name):
     assert not np.isnan(a).any() and np.array_equal(np.isinf(a), np.isinf(b))
     T.close()
     C.close()
+
+
+# rings, span, maximum ring difference, ny, nx, TOF bins, whether the default takes tiles: sides whose tiles in the
+# field of view lie on either side of the line for one plane per axial position (350), two (150 of several slots, 260
+# of one), mixed ones (95, 135), TOF (92, 45 and 55 a mean live bin), and never too few of short images
+DEFAULTS = [
+    (40, 5, 20, 96, 96, 0, False), (40, 5, 20, 160, 160, 0, False), (40, 5, 20, 176, 176, 0, True),
+    (40, 5, 20, 60, 600, 0, False), (24, 5, 12, 130, 130, 0, False), (24, 5, 12, 200, 200, 0, True),
+    (40, 1, 4, 96, 96, 0, False), (40, 1, 4, 120, 120, 0, True), (18, 1, 4, 128, 128, 0, False),
+    (18, 1, 4, 150, 150, 0, True), (40, 3, 11, 60, 60, 0, False), (20, 3, 17, 96, 96, 0, False),
+    (20, 3, 17, 112, 112, 0, True), (12, 1, 4, 24, 24, 0, True), (24, 3, 8, 100, 100, 9, False),
+    (24, 3, 8, 260, 260, 9, True),
+]
+
+
+@pytest.mark.parametrize("rings,span,mrd,ny,nx,ntof,tiles", DEFAULTS)
+def test_default_takes_tiles_only_where_they_are_faster(rings, span, mrd, ny, nx, ntof, tiles):
+    sc = Scanner("default", rings, 64, 150.0, 0.0, 4.0, 4.0, 0.0, 30, 30, 400.0 if ntof else 0.0,
+                 200.0 if ntof else 0.0, ntof)
+    pdi = ProjDataInfoCylindrical.construct(sc, span, mrd, 32, 30, False)
+    if ntof:
+        pdi = pdi.with_tof(1)
+    vox = 200.0 / max(nx, ny)
+    img = VoxelsOnCartesianGrid(2 * rings - 1, ny, nx, 2.0, vox, vox)
+    print(f"[tile paths] {rings} rings, span {span}, {ny} x {nx}, {ntof} TOF bins", flush=True)
+    kernels = {True: (_native.MI_BACK_TILES, _native.MI_BACK_SHORT_TILES),
+               False: (_native.MI_BACK_TOF_ROWS if ntof else _native.MI_BACK_COLUMNS,)}
+    y = np.random.default_rng(92).uniform(0.5, 2.0, pdi.num_bins).astype(np.float32)
+    default, other = make(pdi, img, RayTracingMatrixParameters(), 1), make(pdi, img, RayTracingMatrixParameters(),
+                                                                           0 if tiles else 2)
+    assert default.context.projection_kernels()[1] in kernels[tiles]
+    assert other.context.projection_kernels()[1] in kernels[not tiles]
+    a, b = default.back_project(y), other.back_project(y)
+    assert np.abs(a - b).max() <= 1e-5 * b.max()
+    default.close()
+    other.close()
