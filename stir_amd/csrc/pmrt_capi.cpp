@@ -31,10 +31,11 @@ void launch_fill_int2(int2* d, int64_t n, int2 v, hipStream_t stream);
 
 namespace {
 
-// Mean axial positions per family up to which the forward projection runs row
-// groups (milliseconds, row groups against tasks): 8 rings, mean 7: 0.083 / 0.358;
-// 16 rings, span 1, mean 8: 0.47 / 1.23; 24 rings, span 3, mean 24: 0.50 / 0.59;
-// 32 rings, span 7, mean 38: 0.60 / 0.52; 40 rings, span 9, mean 47: 0.77 / 0.62.
+// Mean axial positions per family up to which the forward projection's row
+// groups are made; rows_pay decides which projections run on them. (Microseconds,
+// row groups against tasks, 140 x 140 columns: 8 rings, span 1, mean 4: 245 / 937;
+// 16 rings, span 3, mean 16: 178 / 193; 24 rings, mean 24: 330 / 395. Above 28
+// the best gains are a tenth, and 32 rings, span 5, mean 44, take 245 / 201.)
 constexpr int kRowsMeanAxial = 28;
 
 thread_local std::string g_last_error;
@@ -133,7 +134,9 @@ struct mi_ctx {
   std::vector<std::vector<int>> subset_groups;          // subset of the table -> its groups, ascending
   std::vector<mi::FpTask> h_tasks;
   // forward projection by row groups (pmrt_rows.hip), for short families
-  bool use_rows = false;
+  int rows_enable = 1;        // MI_TUNE_FP_ROW_GROUPS
+  bool use_rows = false;      // the row groups are there
+  std::vector<char> rows_of;  // whether a projection of subset s, or of all (s = nsub), runs on them
   std::vector<int> item_off;  // per subset, size nsub+1
   std::vector<int2> h_row_items;  // of a batch's problem
   DBuf<mi::RowGroup> row_groups;
@@ -327,14 +330,14 @@ struct mi_ctx {
   }
 
   // MI_FORWARD_*
-  int forward_kernel() const {
+  int forward_kernel(int subset) const {
     if (ntof > 1) return tof_fp_w > 0 ? MI_FORWARD_TOF_ROWS : MI_FORWARD_TOF;
-    return use_rows ? MI_FORWARD_ROW_GROUPS : MI_FORWARD_TASKS;
+    return use_rows && rows_of[subset < 0 ? plan->num_subsets() : subset] ? MI_FORWARD_ROW_GROUPS : MI_FORWARD_TASKS;
   }
   // ---- projections on device-layout buffers
   void fp(mi::FpMode mode, const float* d_img, float* d_out, int subset, const mi::FpData& data, hipStream_t st) {
     const int tb = task_off[subset_begin(subset)], te = task_off[subset_end(subset)];
-    if (!use_rows) {
+    if (forward_kernel(subset) != MI_FORWARD_ROW_GROUPS) {
       fp_tasks(mode, tasks.p + tb, te - tb, d_img, d_out, data, st);
       return;
     }
@@ -347,7 +350,7 @@ struct mi_ctx {
   }
   // log-likelihood partial sums that fp() of a subset writes
   int num_partials(int subset) const {
-    const std::vector<int>& off = use_rows ? item_off : task_off;
+    const std::vector<int>& off = forward_kernel(subset) == MI_FORWARD_ROW_GROUPS ? item_off : task_off;
     return off[subset_end(subset)] - off[subset_begin(subset)];
   }
   void fp_tasks(mi::FpMode mode, const mi::FpTask* d_tasks, int ntasks, const float* d_img, float* d_out,
@@ -732,18 +735,47 @@ void mi_ctx::build_tasks() {
   HIPCHECK(hipStreamSynchronize(stream));
 }
 
-// Row groups (pmrt_rows.hip) where the families are short (kRowsMeanAxial).
+// Whether one projection of `items` row group items, with `rows` elements to
+// walk in all, is faster than tasks with `tasks` of them. Row groups start fewer
+// waves, each of which reads several image columns per element where a task
+// reads one; `longest` elements has the longest row. Measured on 250 scanners of
+// 6 to 34 rings with images of 60 to 344 columns a side, whole projections and
+// subsets of them, the gain (0.63 to 4.1) goes with
+//  - tasks / rows, the elements that row groups save (1.3 to 6.4 where they pay);
+//  - the elements that a row has per image column it crosses (two or three
+//    planes at two planes per axial position), which share the column's lines:
+//    as its root;
+//  - the size of the image, which no longer fits the L2 (4 MB) beside the
+//    columns of other waves: the fourth root;
+//  - the rounds of waves that the chip takes, as the eighth root: with less
+//    than one, waves last as long as a row however few they are.
+// The product is 1.3 where both are as fast. On the 340 launches whose families
+// are short the gain is 1.58 in the (geometric) mean, 1.57 with row groups for
+// all of them (losses of up to 37 %) and 1.59 without a mistake; the worst loss
+// left is 11 %, the largest gain left out 28 %.
+static bool rows_pay(double tasks, double rows, int items, int longest, const mi::ImageDims& d, int lors) {
+  if (items <= 0 || rows <= 0 || tasks < 1.2 * rows) return false;
+  const double per_column = longest / (1.45 * lors * std::min(d.nx, d.ny));
+  const double rounds = std::clamp(items / 8192.0, 0.05, 4.5);  // 256 CUs x 32 waves
+  const double mb = std::max(4e-6 * d.ncols * d.nzp, 1.0);
+  return tasks / rows * std::sqrt(per_column) * std::pow(rounds, 0.125) >= 1.3 * std::pow(mb, 0.25);
+}
+
+// Row groups (pmrt_rows.hip) where the families are short (kRowsMeanAxial) and
+// projections are faster with them (rows_pay), or in a batch, whose problems
+// share a launch.
 void mi_ctx::build_row_groups() {
   use_rows = false;
+  rows_of.clear();
   item_off.clear();
   row_groups.release();
   row_fams.release();
   row_items.release();
   // (the image is read as one buffer of less than 2^31 bytes)
-  if (ntof > 1 || h_fams.empty() || static_cast<int64_t>(dims.ncols) * dims.nzp >= (int64_t{1} << 28)) return;
+  if (!rows_enable || ntof > 1 || h_fams.empty() || static_cast<int64_t>(dims.ncols) * dims.nzp >= (int64_t{1} << 28)) return;
   int64_t bins = 0;
   for (const mi::Family& f : h_fams) bins += f.nax;
-  if (bins > int64_t{kRowsMeanAxial} * static_cast<int64_t>(h_fams.size())) return;
+  if (rows_enable == 1 && bins > int64_t{kRowsMeanAxial} * static_cast<int64_t>(h_fams.size())) return;
   const int nsub = plan->num_subsets();
   std::vector<mi::RowGroup> groups;
   std::vector<int32_t> list;
@@ -776,6 +808,26 @@ void mi_ctx::build_row_groups() {
     }
   }
   item_off[nsub] = static_cast<int>(items.size());
+  rows_of.assign(nsub + 1, 0);
+  double all_tasks = 0, all_rows = 0;
+  int all_longest = 0;
+  for (int s = 0; s < nsub; ++s) {
+    double tw = 0, rw = 0;
+    int longest = 0;
+    for (int t = task_off[s]; t < task_off[s + 1]; ++t) tw += h_fams[h_tasks[t].first].row_len;
+    for (int i = item_off[s]; i < item_off[s + 1]; ++i) {
+      const int len = groups[items[i].x].row_len;
+      rw += len;
+      longest = std::max(longest, len);
+    }
+    rows_of[s] = rows_pay(tw, rw, item_off[s + 1] - item_off[s], longest, dims, plan->geometry().num_tangential_LORs);
+    all_tasks += tw;
+    all_rows += rw;
+    all_longest = std::max(all_longest, longest);
+  }
+  rows_of[nsub] = rows_pay(all_tasks, all_rows, item_off[nsub], all_longest, dims, plan->geometry().num_tangential_LORs);
+  if (rows_enable == 2) rows_of.assign(nsub + 1, 1);
+  if (!in_batch && std::find(rows_of.begin(), rows_of.end(), 1) == rows_of.end()) return;
   auto upload = [&](auto& buf, const auto& v) {
     buf.alloc(v.size());
     HIPCHECK(hipMemcpyAsync(buf.p, v.data(), buf.bytes(), hipMemcpyHostToDevice, stream));
@@ -2753,6 +2805,10 @@ int mi_set_tuning(mi_ctx* ctx, int param, int value) {
         if (value < 0 || value > 2) throw ApiError(MI_ERR_ARGUMENT, "the image tile switch must be 0, 1 or 2");
         ctx->tiles_enable = value;
         break;
+      case MI_TUNE_FP_ROW_GROUPS:
+        if (value < 0 || value > 2) throw ApiError(MI_ERR_ARGUMENT, "the row group switch must be 0, 1 or 2");
+        ctx->rows_enable = value;
+        break;
       default: throw ApiError(MI_ERR_ARGUMENT, "unknown tuning parameter");
     }
   });
@@ -2796,7 +2852,7 @@ int mi_get_projection_kernels(mi_ctx* ctx, int subset, int32_t* forward, int32_t
     if (!ctx || !forward || !back) throw ApiError(MI_ERR_ARGUMENT, "NULL argument");
     ctx->require_setup();
     ctx->check_subset(subset);
-    *forward = ctx->forward_kernel();
+    *forward = ctx->forward_kernel(subset);
     *back = ctx->back_kernel();
   });
 }
