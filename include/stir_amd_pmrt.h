@@ -527,13 +527,16 @@ int mi_batch_synchronize(mi_batch* batch);
  * set-up. MI_TUNE_FP_ROW_GROUPS 0, 1 and 2 do the same for the row groups of
  * the forward projection (families of few axial positions; projections of a
  * subset and of all are chosen separately). The results of the forward
- * projection do not depend on it. mi_get_projection_kernels tells which
+ * projection do not depend on it. MI_TUNE_BP_TILE_MEMORY_MB limits the memory
+ * that a set-up takes for image tiles and for making them, in MB (0, the
+ * default: what the device has); where it does not suffice, the column table or
+ * the TOF records are made instead. mi_get_projection_kernels tells which
  * kernels run. */
 enum { MI_TUNE_BP_TILE_X = 1, MI_TUNE_BP_TILE_Y = 2, MI_TUNE_BP_XCD_REMAP = 3, MI_TUNE_BP_SLOT_SKIP = 4,
        MI_TUNE_FP_XCD_CHUNK = 5, MI_TUNE_BP_SLAB = 6, MI_TUNE_SLAB_TILE_X = 7, MI_TUNE_SLAB_TILE_Y = 8,
        MI_TUNE_SLAB_COLUMNS_PER_WAVE = 9, MI_TUNE_SLAB_LDS_KB = 10, MI_TUNE_TOF_ROWS = 11, MI_TUNE_BP_QUAD = 12,
        MI_TUNE_BP_QUAD_UNROLL = 13, MI_TUNE_BP_SPLIT_SUBSETS = 14, MI_TUNE_BP_IMAGE_TILES = 15,
-       MI_TUNE_FP_ROW_GROUPS = 16 };
+       MI_TUNE_FP_ROW_GROUPS = 16, MI_TUNE_BP_TILE_MEMORY_MB = 17 };
 int mi_set_tuning(mi_ctx* ctx, int param, int value);
 
 /* ---- diagnostics ----------------------------------------------------------- */

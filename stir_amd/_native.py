@@ -58,6 +58,7 @@ MI_TUNE_BP_QUAD_UNROLL = 13
 MI_TUNE_BP_SPLIT_SUBSETS = 14
 MI_TUNE_BP_IMAGE_TILES = 15
 MI_TUNE_FP_ROW_GROUPS = 16
+MI_TUNE_BP_TILE_MEMORY_MB = 17
 
 MI_FORWARD_TASKS, MI_FORWARD_ROW_GROUPS, MI_FORWARD_TOF_ROWS, MI_FORWARD_TOF = 0, 1, 2, 3
 MI_BACK_COLUMNS, MI_BACK_BLOCKS, MI_BACK_SLABS, MI_BACK_TILES, MI_BACK_SHORT_TILES = 0, 1, 2, 3, 4

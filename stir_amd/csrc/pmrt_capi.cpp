@@ -98,9 +98,16 @@ struct DBuf {
 struct Arena {
   std::deque<DBuf<char>> blocks;
   size_t used = 0;
+  int64_t limit = 0, taken = 0;  // bytes that may be taken (0: any number), and have been
+  // counts bytes against the limit; past it fails as an allocation does
+  void take(size_t bytes) {
+    taken += static_cast<int64_t>(bytes);
+    if (limit > 0 && taken > limit) throw ApiError(MI_ERR_MEMORY, "memory limit reached");
+  }
   template <class T>
   T* get(size_t count) {
     const size_t bytes = (count * sizeof(T) + 255) / 256 * 256;
+    take(bytes);
     if (blocks.empty() || used + bytes > blocks.back().n) {
       blocks.emplace_back();
       blocks.back().alloc(std::max(bytes, size_t{32} << 20));
@@ -198,8 +205,16 @@ struct mi_ctx {
     return static_cast<int64_t>(tile_phase_off.bytes() + tile_hdr.bytes() + tile_row.bytes() + tile_off.bytes() +
                                 tile_order.bytes() + tile_w.bytes());
   }
+  int tile_memory_mb = 0;  // MI_TUNE_BP_TILE_MEMORY_MB
   bool build_tile_table(int span, double terms);
+  bool make_tile_table(int span, double terms);
   int min_tiles(double terms) const;
+  // device memory that a set-up takes after the tables and a reconstruction on
+  // it: images, projection data, sensitivities
+  int64_t later_bytes() const {
+    return int64_t{4} * dims.ncols * dims.nzp * (6 + plan->num_subsets()) + int64_t{4} * plan->num_voxels() +
+           int64_t{36} * total_bins();
+  }
   std::vector<mi::Family> h_fams;
   std::unordered_map<int64_t, int> fam_lookup;  // (seg,view,tang,a0) -> family
   int64_t num_basic_elements = 0;
@@ -855,7 +870,6 @@ void mi_ctx::build_table() {
       use_tile = true;
       return;
     }
-    release_tile();
   }
   const int nsub = plan->num_subsets();
   const int ncols = dims.ncols;
@@ -1055,7 +1069,6 @@ void mi_ctx::build_tof_rows(int64_t n) {
     entry_d.release();
     return;
   }
-  release_tile();
   tof_bp_rec.alloc((n + 1) * mi::tof_bp_words(bw));  // + the all-zero record read past a list's end
   HIPCHECK(hipMemsetAsync(tof_bp_rec.p + n * mi::tof_bp_words(bw), 0, sizeof(int32_t) * mi::tof_bp_words(bw), stream));
   mi::launch_tof_bp_records(entries.p, entry_d.p, n, tofc, bw, tof_bp_rec.p, stream);
@@ -1331,6 +1344,19 @@ int mi_ctx::min_tiles(double terms) const {
 // (they are used then). TOF matrices: from the stored forward records, span the
 // most TOF bins of one element, terms their mean number.
 bool mi_ctx::build_tile_table(int span, double terms) {
+  try {
+    if (make_tile_table(span, terms)) return true;
+  } catch (const ApiError& e) {
+    // out of memory: the other table may fit
+    if (e.code != MI_ERR_MEMORY) throw;
+    (void)hipGetLastError();
+    HIPCHECK(hipStreamSynchronize(stream));
+  }
+  release_tile();
+  return false;
+}
+
+bool mi_ctx::make_tile_table(int span, double terms) {
   const mi_geometry& g = plan->geometry();
   if (!tiles_enable || (in_batch && dims.nz <= mi::kTileShortPlanes) || slab_enable || quad_enable || dims.nz > 256 ||
       h_fams.empty())
@@ -1399,15 +1425,12 @@ bool mi_ctx::build_tile_table(int span, double terms) {
   most *= span;
   if (most <= 0 || most >= (int64_t{1} << 31)) return false;
   const int ntiles = S.ntx * ((dims.ny + S.ty - 1) / S.ty);
-  if (ntof > 1) {
-    // only where the terms (8 bytes each, padded lists), the rows and the sort's
-    // buffers fit beside everything else
-    size_t free_b = 0, total_b = 0;
-    HIPCHECK(hipMemGetInfo(&free_b, &total_b));
-    const int64_t bytes = 10 * n * span + 32 * most + 4 * (static_cast<int64_t>(ntiles) * nunits);
-    if (bytes > static_cast<int64_t>(free_b / 4 * 3)) return false;
-  }
   Arena mem;
+  mem.limit = int64_t{tile_memory_mb} << 20;
+  auto alloc = [&](auto& buf, size_t count) {
+    mem.take(count * sizeof(*buf.p));
+    buf.alloc(count);
+  };
   auto upload = [&](const auto& v) {
     auto* d = mem.get<typename std::decay_t<decltype(v)>::value_type>(v.size());
     HIPCHECK(hipMemcpyAsync(d, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice, stream));
@@ -1417,7 +1440,7 @@ bool mi_ctx::build_tile_table(int span, double terms) {
   const int2* d_pos = upload(hpos);
   const int32_t* d_unit_off = upload(hunit_off);
   // pass 1: tangential ranges and the zeros a row needs
-  tile_rng.alloc(static_cast<size_t>(ntiles) * nrng);
+  alloc(tile_rng, static_cast<size_t>(ntiles) * nrng);
   mi::launch_fill_int2(tile_rng.p, static_cast<int64_t>(tile_rng.n), make_int2(0x7fffffff, -1), stream);
   int need[3];
   int* d_need = mem.get<int>(3);  // planes after a run's start, planes up to its end, flag
@@ -1458,7 +1481,7 @@ bool mi_ctx::build_tile_table(int span, double terms) {
   uint32_t* slot = mem.get<uint32_t>(static_cast<size_t>(ntiles) * nunits);
   uint32_t *nphase = mem.get<uint32_t>(nst + 1), *nrow = mem.get<uint32_t>(nst + 1);
   uint32_t* row_off = mem.get<uint32_t>(nst + 1);
-  tile_phase_off.alloc(nst + 1);
+  alloc(tile_phase_off, nst + 1);
   HIPCHECK(hipMemsetAsync(nphase + nst, 0, sizeof(uint32_t), stream));
   HIPCHECK(hipMemsetAsync(nrow + nst, 0, sizeof(uint32_t), stream));
   mi::launch_tile_phases(d_units, d_unit_off, nsub, ntiles, nunits, nrng, tile_rng.p, rows, slot, nphase, nrow,
@@ -1481,7 +1504,7 @@ bool mi_ctx::build_tile_table(int span, double terms) {
   const int64_t nph = totals[0], nlists = nph * S.lines();
   if (nlists >= (int64_t{1} << 31) - 2) return false;
   const int row_slack = mi::tile_row_slack(A.stride);
-  tile_row.alloc(static_cast<size_t>(total_rows) + row_slack);
+  alloc(tile_row, static_cast<size_t>(total_rows) + row_slack);
   HIPCHECK(hipMemsetAsync(tile_row.p + total_rows, 0, row_slack * sizeof(int2), stream));
   uint32_t* phase_row = mem.get<uint32_t>(nph);
   mi::launch_tile_rows(d_units, d_unit_off, nsub, ntiles, nunits, nrng, tile_rng.p, rows, tile_phase_off.p,
@@ -1504,19 +1527,24 @@ bool mi_ctx::build_tile_table(int span, double terms) {
   const int64_t nslots = 4 * static_cast<int64_t>(totals[1]);
   if (need[2]) return false;
   {
-    // the padded lists and the sort's buffers have to fit; the other tables
-    // need less where the lists are short (a list of one entry is padded to four)
+    // The padded lists and the sort's buffers have to fit now. What stays (a list
+    // of one entry is padded to four) may be no more than the other table would
+    // take, or has to leave room for what is allocated later.
     size_t free_b = 0, total_b = 0;
     HIPCHECK(hipMemGetInfo(&free_b, &total_b));
-    if (8 * nslots + 32 * most > static_cast<int64_t>(free_b / 16 * 15)) return false;
+    const int64_t now = 8 * nslots + static_cast<int64_t>(sizeof(uint4)) * mi::kTileWaves * nph;
+    if (now + 40 * most > static_cast<int64_t>(free_b / 16 * 15)) return false;
+    const int64_t other = ntof > 1 ? int64_t{4} * mi::tof_bp_words(tof_bp_w) * n
+                                   : static_cast<int64_t>(sizeof(mi::BpEntry)) * n + int64_t{8} * nsub * dims.ncols;
+    if (now + tile_bytes() > other && now + later_bytes() > static_cast<int64_t>(free_b)) return false;
   }
-  tile_hdr.alloc((nph + mi::kTileHdrSlack) * mi::kTileWaves);
+  alloc(tile_hdr, (nph + mi::kTileHdrSlack) * mi::kTileWaves);
   mi::launch_tile_headers(groups, group_off, phase_row, total_rows, nph, S, tile_hdr.p, stream);
   // pass 4, subset by subset: every term's list and entry, sorted by list, to
   // its place
   const int64_t* d_fam_off = upload(fam_off);
-  tile_off.alloc(nslots + mi::kTileEntSlack);
-  tile_w.alloc(nslots + mi::kTileEntSlack);
+  alloc(tile_off, nslots + mi::kTileEntSlack);
+  alloc(tile_w, nslots + mi::kTileEntSlack);
   HIPCHECK(hipMemsetAsync(tile_off.p, 0, tile_off.bytes(), stream));  // padding: weight 0 times the leading zeros
   HIPCHECK(hipMemsetAsync(tile_w.p, 0, tile_w.bytes(), stream));
   {
@@ -1555,7 +1583,7 @@ bool mi_ctx::build_tile_table(int span, double terms) {
   std::vector<int32_t> order(ntiles);
   for (int t = 0; t < ntiles; ++t) order[t] = t;
   std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return work[a] > work[b]; });
-  tile_order.alloc(ntiles);
+  alloc(tile_order, ntiles);
   HIPCHECK(hipMemcpyAsync(tile_order.p, order.data(), tile_order.bytes(), hipMemcpyHostToDevice, stream));
   HIPCHECK(hipStreamSynchronize(stream));
   A.hdr = tile_hdr.p;
@@ -2804,6 +2832,10 @@ int mi_set_tuning(mi_ctx* ctx, int param, int value) {
       case MI_TUNE_BP_IMAGE_TILES:
         if (value < 0 || value > 2) throw ApiError(MI_ERR_ARGUMENT, "the image tile switch must be 0, 1 or 2");
         ctx->tiles_enable = value;
+        break;
+      case MI_TUNE_BP_TILE_MEMORY_MB:
+        if (value < 0) throw ApiError(MI_ERR_ARGUMENT, "the image tiles' memory limit must not be negative");
+        ctx->tile_memory_mb = value;
         break;
       case MI_TUNE_FP_ROW_GROUPS:
         if (value < 0 || value > 2) throw ApiError(MI_ERR_ARGUMENT, "the row group switch must be 0, 1 or 2");

@@ -116,3 +116,26 @@ def test_default_takes_tiles_only_where_they_are_faster(rings, span, mrd, ny, nx
     assert np.abs(a - b).max() <= 1e-5 * b.max()
     default.close()
     other.close()
+
+
+@pytest.mark.parametrize("kind,name", [("tall", "127planes_span11"), ("short", "31planes_many_phases"),
+                                       ("tof", "64planes_9bins")])
+def test_memory_limit_falls_back_to_the_other_table(kind, name):
+    """The table does not fit at any of its allocations: the set-up succeeds with the other one."""
+    pdi, img, pm, tiles, other, same = geometry(kind, name)
+    y = np.random.default_rng(93).uniform(0.5, 2.0, pdi.num_bins).astype(np.float32)
+    ref = make(pdi, img, pm, 0)
+    b = ref.back_project(y)
+    ref.close()
+    P = ProjectorByBinPairMI355X(ProjMatrixByBinUsingRayTracing(pm))
+    P.context.set_tuning(_native.MI_TUNE_BP_IMAGE_TILES, 2)
+    kernels = []
+    for mb in (1, 2, 4, 8, 16, 32, 64, 128, 256, 512, 0, 1):  # one context: a refused table leaves nothing behind
+        P.context.set_tuning(_native.MI_TUNE_BP_TILE_MEMORY_MB, mb)
+        P.set_up(pdi, img, num_subsets=4)
+        kernels.append(P.context.projection_kernels()[1])
+        assert np.abs(P.back_project(y) - b).max() <= 1e-5 * b.max(), mb
+    print(f"[tile paths] {kind} {name}: kernels by limit {kernels}", flush=True)
+    n = kernels.index(tiles)
+    assert n >= 2 and kernels == [other] * n + [tiles] * (11 - n) + [other]
+    P.close()
