@@ -461,7 +461,9 @@ int mi_batch_get_estimate(mi_batch* batch, int problem, float* image);
 int mi_batch_set_launch(mi_batch* batch, int fp_group_max, int fp_widen, int bp_pack, int tile_x, int tile_y);
 /* Forward projection in row groups: the families of one basic row with at
  * most max_axial axial positions (0: none) run up to 64 axial positions per
- * wave with the row's elements loaded once (default 32). */
+ * wave with the row's elements loaded once (default 32). From 28 on, a problem
+ * whose families have at most 28 on average runs all of them so, longer ones
+ * too. */
 int mi_batch_set_row_groups(mi_batch* batch, int max_axial);
 /* Times the candidate launch shapes on subset 0 (no side effects on the
  * estimates) and keeps the fastest; *choice receives its index. */

@@ -78,8 +78,9 @@ class BatchedOSMAPOSL:
     def set_launch(self, fp_group_max: int = 32, fp_widen: bool = False, bp_pack: int = 2, tile_x: int = 32,
                    tile_y: int = 8, row_groups: int = 32) -> None:
         """row_groups: families of at most this many axial positions run in row
-        groups (0: off); the others in lane groups of fp_group_max bins or
-        full waves; bp_pack: columns of images of at most 32 planes in full
+        groups (0: off; from 28 on also the longer ones of a problem whose
+        families have at most 28 on average); the others in lane groups of
+        fp_group_max bins or full waves; bp_pack: columns of images of at most 32 planes in full
         waves (0), lane groups (1) or waves split over table entries (2)."""
         L = _native.load()
         _native.check(L.mi_batch_set_launch(self._h, fp_group_max, int(fp_widen), int(bp_pack), tile_x, tile_y),

@@ -3052,7 +3052,8 @@ void batch_prepare(mi_batch* b) {
     std::vector<int32_t> rg_fam;
     for (int p = 0; p < np; ++p) {
       const mi_ctx* c = b->probs[p];
-      if (c->use_rows && b->fp_rowgroup_max > 0) {  // the groups its own forward projection uses
+      // all families in the problem's own row groups, or by max_axial as the others
+      if (c->use_rows && b->fp_rowgroup_max > 0 && b->fp_rowgroup_max >= std::min(kRowsMeanAxial, c->max_axial)) {
         for (int i = c->item_off[s]; i < c->item_off[s + 1]; ++i)
           row_work.push_back(make_int4(p, c->h_row_items[i].x, c->h_row_items[i].y, 0));
         continue;
