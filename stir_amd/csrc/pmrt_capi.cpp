@@ -95,6 +95,8 @@ struct DBuf {
 };
 // Device memory for the steps of a set-up, in blocks freed together at its
 // end: an allocation and a free cost 0.1 ms, and a table takes twenty of them.
+// A free costs 0.01 ms up to 8 MB and 0.2 to 0.3 ms above, whatever the size, so
+// small blocks by default and one (reserve) for all large buffers.
 struct Arena {
   std::deque<DBuf<char>> blocks;
   size_t used = 0;
@@ -104,15 +106,18 @@ struct Arena {
     taken += static_cast<int64_t>(bytes);
     if (limit > 0 && taken > limit) throw ApiError(MI_ERR_MEMORY, "memory limit reached");
   }
+  // one block for buffers of so many bytes in all (256 more for each)
+  void reserve(size_t bytes) {
+    if (!blocks.empty() && used + bytes <= blocks.back().n) return;
+    blocks.emplace_back();
+    blocks.back().alloc(std::max(bytes, size_t{4} << 20));
+    used = 0;
+  }
   template <class T>
   T* get(size_t count) {
     const size_t bytes = (count * sizeof(T) + 255) / 256 * 256;
     take(bytes);
-    if (blocks.empty() || used + bytes > blocks.back().n) {
-      blocks.emplace_back();
-      blocks.back().alloc(std::max(bytes, size_t{32} << 20));
-      used = 0;
-    }
+    reserve(bytes);
     T* p = reinterpret_cast<T*>(blocks.back().p + used);
     used += bytes;
     return p;
@@ -722,13 +727,16 @@ void mi_ctx::build_tasks() {
   group_vs.clear();
   task_group.assign(h.size(), -1);
   subset_groups.assign(nsub, {});
+  std::vector<int> known(plan->num_viewgrams(), -1);  // groups found, by viewgram
   auto group_of = [&](int fam) {
     int v = keys[fam].view, sg = keys[fam].seg;
+    int& group = known[plan->viewgram_index(sg, v)];
+    if (group >= 0) return group;
     plan->basic_view_segment(v, sg);
     const int64_t key = static_cast<int64_t>(sg + 512) * 65536 + v;
     auto it = vs_group.emplace(key, static_cast<int>(group_vs.size()));
     if (it.second) group_vs.push_back(plan->related_view_segments(v, sg));
-    return it.first->second;
+    return group = it.first->second;
   };
   for (int s = 0; s < nsub; ++s)
     for (int t = task_off[s]; t < task_off[s + 1]; ++t) {
@@ -796,31 +804,40 @@ void mi_ctx::build_row_groups() {
   std::vector<int32_t> list;
   std::vector<int2> items;
   item_off.assign(nsub + 1, 0);
-  std::vector<int> order;
+  // the subset's families by basic row, all of the empty rows as one: lists
+  // linked in family order (a sort of the families took 5 ms of the set-up of
+  // 3.5e5 of them, this 1). A row's families are one segment or +-pair: one length.
+  const auto& keys = plan->family_keys();
+  const int nrows = static_cast<int>(plan->basic_rays().size());
+  std::vector<int> head(nrows + 1), tail(nrows + 1), seen(nrows + 1, -1), next(h_fams.size()), used;
   for (int s = 0; s < nsub; ++s) {
     item_off[s] = static_cast<int>(items.size());
-    // the subset's families by basic row (an empty row starts where the next
-    // row does); a row's families are one segment or +-pair: one length
-    order.clear();
-    for (int f = plan->subset_family_begin(s); f < plan->subset_family_begin(s + 1); ++f) order.push_back(f);
-    std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
-      const mi::Family &A = h_fams[a], &B = h_fams[b];
-      if (A.row_start != B.row_start) return A.row_start < B.row_start;
-      if (A.row_len != B.row_len) return A.row_len < B.row_len;
-      return A.nax < B.nax;
-    });
-    for (size_t i = 0; i < order.size();) {
-      const mi::Family& F = h_fams[order[i]];
-      mi::RowGroup G{F.row_start, F.row_len, static_cast<int32_t>(list.size()), 0, F.nax, 0, {0, 0}};
-      for (; i < order.size(); ++i) {
-        const mi::Family& f = h_fams[order[i]];
-        if (f.row_start != F.row_start || f.row_len != F.row_len || f.nax != F.nax) break;
-        list.push_back(order[i]);
-        ++G.nfam;
+    used.clear();
+    for (int f = plan->subset_family_begin(s); f < plan->subset_family_begin(s + 1); ++f) {
+      const int b = h_fams[f].row_len > 0 ? keys[f].basic_index : nrows;
+      next[f] = -1;
+      if (seen[b] != s) {
+        seen[b] = s;
+        head[b] = f;
+        used.push_back(b);
+      } else {
+        next[tail[b]] = f;
       }
-      for (int b = 0; b < G.nfam * G.nax; b += 64) items.push_back(make_int2(static_cast<int>(groups.size()), b));
-      groups.push_back(G);
+      tail[b] = f;
     }
+    std::sort(used.begin(), used.end());
+    for (const int b : used)
+      for (int f = head[b]; f >= 0;) {
+        const mi::Family& F = h_fams[f];
+        mi::RowGroup G{F.row_start, F.row_len, static_cast<int32_t>(list.size()), 0, F.nax, 0, {0, 0}};
+        for (; f >= 0 && h_fams[f].nax == F.nax; f = next[f]) {
+          list.push_back(f);
+          ++G.nfam;
+        }
+        for (int first = 0; first < G.nfam * G.nax; first += 64)
+          items.push_back(make_int2(static_cast<int>(groups.size()), first));
+        groups.push_back(G);
+      }
   }
   item_off[nsub] = static_cast<int>(items.size());
   rows_of.assign(nsub + 1, 0);
@@ -1548,17 +1565,19 @@ bool mi_ctx::make_tile_table(int span, double terms) {
   HIPCHECK(hipMemsetAsync(tile_off.p, 0, tile_off.bytes(), stream));  // padding: weight 0 times the leading zeros
   HIPCHECK(hipMemsetAsync(tile_w.p, 0, tile_w.bytes(), stream));
   {
-    uint32_t *keys_in = mem.get<uint32_t>(most), *keys_out = mem.get<uint32_t>(most);
-    uint32_t *vals_in = mem.get<uint32_t>(most), *vals_out = mem.get<uint32_t>(most);
-    int2* raw = mem.get<int2>(most);
-    mi::launch_iota(vals_in, most, stream);
     const uint32_t none = static_cast<uint32_t>(nlists);
     int end_bit = 1;
     while ((int64_t{1} << end_bit) <= nlists) ++end_bit;
     size_t tb = 0;
-    HIPCHECK(mi::radix_sort_pairs(nullptr, tb, keys_in, keys_out, vals_in, vals_out, static_cast<int>(most),
+    uint32_t* const no_buffer = nullptr;
+    HIPCHECK(mi::radix_sort_pairs(nullptr, tb, no_buffer, no_buffer, no_buffer, no_buffer, static_cast<int>(most),
                                   end_bit, stream));
+    mem.reserve(24 * most + tb + 6 * 256);
+    uint32_t *keys_in = mem.get<uint32_t>(most), *keys_out = mem.get<uint32_t>(most);
+    uint32_t *vals_in = mem.get<uint32_t>(most), *vals_out = mem.get<uint32_t>(most);
+    int2* raw = mem.get<int2>(most);
     char* tmp = mem.get<char>(std::max<size_t>(tb, 1));
+    mi::launch_iota(vals_in, most, stream);
     for (int s = 0; s < nsub; ++s) {
       const int fb = plan->subset_family_begin(s), fe = plan->subset_family_begin(s + 1);
       const int64_t m = (fam_off[fe] - fam_off[fb]) * span;

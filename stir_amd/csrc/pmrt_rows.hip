@@ -69,14 +69,15 @@ __global__ void __launch_bounds__(kWave) row_group_reach_kernel(RowGroup* __rest
     lo = min(lo, __shfl_xor(lo, o, kWave));
     hi = max(hi, __shfl_xor(hi, o, kWave));
   }
-  if (threadIdx.x != 0) return;
   const int pad = d.nzp - d.nz;
-  int inside = 1;
-  for (int k = 0; k < G.nfam; ++k) {
+  bool inside = true;
+  for (int k = threadIdx.x; k < G.nfam; k += kWave) {  // (the empty rows' group has thousands)
     const Family f = fams[fam_list[G.first + k]];
     const int z0 = f.zadd0 - d.min_z + (f.zsign > 0 ? lo : -hi), z1 = f.zadd0 - d.min_z + (f.zsign > 0 ? hi : -lo);
-    if (z0 < -pad || z1 + f.ppa * (f.nax - 1) >= d.nz + pad) inside = 0;
+    inside = inside && z0 >= -pad && z1 + f.ppa * (f.nax - 1) < d.nz + pad;
   }
+  inside = __all(inside);
+  if (threadIdx.x != 0) return;
   groups[g].inside = inside;
 }
 
