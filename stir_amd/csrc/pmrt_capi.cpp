@@ -11,6 +11,7 @@
 #include <stdexcept>
 #include <string>
 #include <unordered_map>
+#include <utility>
 #include <deque>
 #include <map>
 #include <vector>
@@ -1031,18 +1032,16 @@ void mi_ctx::build_tof_rows(int64_t n) {
   tof_bp_rec.release();
   tof_fp_nt = tof_fp_w = tof_bp_w = tof_live_span = 0;
   if (ntof <= 1 || tof_rows_mode == 0 || h_fams.empty() || n <= 0) return;
-  std::vector<std::pair<int64_t, int64_t>> rows;
-  rows.reserve(h_fams.size());
   int64_t pool_end = 0;
   if (total_bins() >= (int64_t{1} << 31)) return;  // back records hold a bin index in 31 bits
-  for (const mi::Family& f : h_fams) {
+  std::vector<char> taken(plan->basic_rays().size(), 0);
+  const auto& keys = plan->family_keys();
+  for (size_t i = 0; i < h_fams.size(); ++i) {
+    const mi::Family& f = h_fams[i];
     if (f.ppa < 1 || f.ppa > 15) return;
-    rows.emplace_back(f.row_start, f.row_len);
+    if (f.row_len > 0 && std::exchange(taken[keys[i].basic_index], 1)) return;
     pool_end = std::max<int64_t>(pool_end, int64_t{f.row_start} + f.row_len);
   }
-  std::sort(rows.begin(), rows.end());
-  for (size_t i = 1; i < rows.size(); ++i)
-    if (rows[i - 1].first + rows[i - 1].second > rows[i].first) return;
   DBuf<unsigned long long> span;  // the widest live range, the sum of all
   span.alloc(2);
   HIPCHECK(hipMemsetAsync(span.p, 0, span.bytes(), stream));

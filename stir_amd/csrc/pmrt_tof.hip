@@ -851,8 +851,9 @@ unsigned elementwise_blocks(int64_t n) { return static_cast<unsigned>(std::min<i
 void launch_tof_live_span(const BpEntry* d_entries, const float* d_entry_d, int64_t n, const TofConsts& tof,
                           int* d_span, unsigned long long* d_total, hipStream_t stream) {
   if (n <= 0) return;
-  hipLaunchKernelGGL(tof_live_span_kernel, dim3(elementwise_blocks(n)), dim3(256), 0, stream, d_entries, d_entry_d, n,
-                     tof, d_span, d_total);
+  // (every wave ends in two atomics on one address: 2.6e5 waves took 6 ms)
+  hipLaunchKernelGGL(tof_live_span_kernel, dim3(std::min(elementwise_blocks(n), 2048U)), dim3(256), 0, stream, d_entries,
+                     d_entry_d, n, tof, d_span, d_total);
 }
 
 void launch_tof_fp_records(const Family* d_fams, int nfam, const FamilyLor* d_lors, const int2* d_pool,
