@@ -93,7 +93,8 @@ def main():
     ap.add_argument("--bp-quad", action="store_true",
                     help="pair: back-project over 2 x 2 column blocks (MI_TUNE_BP_QUAD; same sums, for comparison)")
     ap.add_argument("--bp-split", action="store_true",
-                    help="pair: back-project all subsets in one launch per subset (MI_TUNE_BP_SPLIT_SUBSETS)")
+                    help="pair: back-project by column, all subsets in one launch per subset (MI_TUNE_BP_SPLIT_SUBSETS "
+                         "acts on the column and block kernels only)")
     args = ap.parse_args()
     if args.gpus != 1:
         print(json.dumps({"error": "--gpus must be 1",
@@ -127,6 +128,7 @@ def main():
         pair.context.set_tuning(_native.MI_TUNE_BP_QUAD, 1)
     if args.bp_split:
         pair.context.set_tuning(_native.MI_TUNE_BP_SPLIT_SUBSETS, 1)
+        pair.context.set_tuning(_native.MI_TUNE_BP_IMAGE_TILES, 0)
     pair.set_up(pdi, img, num_subsets=nsub)
     torch.cuda.synchronize()
     setup_s = time.time() - t0
@@ -170,7 +172,9 @@ def main():
     nvox = int(img.num_voxels)
     dominant = "bp" if bp_avg >= fp_avg else "fp"
     dom_ms = bp_avg if dominant == "bp" else fp_avg
-    kernel = ("bp_quad_kernel" if args.bp_quad else "bp_tile_kernel") if dominant == "bp" else "fp_kernel"
+    bp_names = {_native.MI_BACK_COLUMNS: "bp_kernel", _native.MI_BACK_BLOCKS: "bp_quad_kernel",
+                _native.MI_BACK_TILES: "bp_tile_kernel"}
+    kernel = bp_names[pair.context.projection_kernels()[1]] if dominant == "bp" else "fp_kernel"
     # HBM bytes per launch under this design: the matrix data the kernel
     # streams (back: table + offsets; forward: rows per task + records) plus
     # one read of the input and one write of the output (mi_info)

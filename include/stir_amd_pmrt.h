@@ -483,10 +483,11 @@ int mi_batch_synchronize(mi_batch* batch);
  * k > 1 in chunks of k workgroups (4 columns each) dealt to the XCDs in turn
  * (default 64: half an 8 x 64 tile per chunk); MI_TUNE_BP_SLOT_SKIP skips z slots
  * an entry cannot reach (default off). They and MI_TUNE_BP_SPLIT_SUBSETS apply
- * to the column kernels only: families that cover whole runs (the z-shift
- * symmetry) are back-projected by image tiles, which have no settings. Results
- * do not depend on these settings. MI_TUNE_FP_XCD_CHUNK maps forward-projection workgroups (4 tasks
- * each) the same way: 0 one contiguous range per XCD, k > 0 chunks of k
+ * to the column and block kernels only: families that cover whole runs (the
+ * z-shift symmetry) are mostly back-projected by image tiles
+ * (MI_TUNE_BP_IMAGE_TILES), which have no settings. Results do not depend on
+ * these settings. MI_TUNE_FP_XCD_CHUNK maps the forward projection's workgroups
+ * of 4 tasks the same way: 0 one contiguous range per XCD, k > 0 chunks of k
  * (default 32).
  * MI_TUNE_BP_SLAB 1 switches the back projection of tables with one plane
  * per axial position (and images of at most 128 planes) to projection-data
@@ -520,8 +521,8 @@ int mi_batch_synchronize(mi_batch* batch);
  * MI_TUNE_BP_SPLIT_SUBSETS 1 back-projects several subsets (a plain back
  * projection of all subsets) in one launch per subset, each continuing the
  * sums the previous one left in the image (the same sums bit for bit as one
- * launch; a working set of one subset's projection data; 2 % faster at mMR
- * size); 0 (default) in one launch.
+ * launch; a working set of one subset's projection data; 2 % faster by column
+ * at mMR size, without effect on image tiles); 0 (default) in one launch.
  * MI_TUNE_BP_IMAGE_TILES 0 keeps a set-up from building image tiles (column
  * table or TOF records instead), 1 (default) builds them where they are the
  * faster ones (images of more than 32 planes need enough tiles to fill the

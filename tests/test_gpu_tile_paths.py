@@ -139,3 +139,25 @@ def test_memory_limit_falls_back_to_the_other_table(kind, name):
     n = kernels.index(tiles)
     assert n >= 2 and kernels == [other] * n + [tiles] * (11 - n) + [other]
     P.close()
+
+
+@pytest.mark.parametrize("name", ["64planes", "127planes_span11"])
+def test_one_launch_per_subset_on_columns_and_blocks(name):
+    """MI_TUNE_BP_SPLIT_SUBSETS acts on the column and block kernels: the sums of tiles, bit for bit."""
+    pdi, img, pm, tiles, other, same = geometry("tall", name)
+    y = np.random.default_rng(94).uniform(0.0, 2.0, pdi.num_bins).astype(np.float32)
+    T = make(pdi, img, pm, 2)
+    assert T.context.projection_kernels()[1] == _native.MI_BACK_TILES
+    ref = T.back_project(y)
+    T.close()
+    Q = ProjectorByBinPairMI355X(ProjMatrixByBinUsingRayTracing(pm))
+    Q.context.set_tuning(_native.MI_TUNE_BP_QUAD, 1)
+    Q.set_up(pdi, img, num_subsets=4)
+    for quad, kernel in ((0, _native.MI_BACK_COLUMNS), (1, _native.MI_BACK_BLOCKS)):
+        Q.context.set_tuning(_native.MI_TUNE_BP_QUAD, quad)
+        for split in (0, 1):
+            Q.context.set_tuning(_native.MI_TUNE_BP_SPLIT_SUBSETS, split)
+            assert Q.context.projection_kernels()[1] == kernel
+            got = Q.back_project(y)
+            assert np.array_equal(got.view(np.uint32), ref.view(np.uint32)), (quad, split)
+    Q.close()
