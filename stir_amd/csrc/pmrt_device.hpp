@@ -127,7 +127,11 @@ void launch_expand_rows(const int2* d_pool, int64_t n, const ImageDims& dims, in
 // ---- forward projection by row groups (pmrt_rows.hip): the non-TOF families
 // that share one basic row, `nax` axial positions each
 constexpr int kRowSlack = 16;      // elements after the last row (read-ahead of the forward row loops)
-constexpr int kRowsXcdChunk = 16;  // workgroups of one XCD's turn
+// Workgroups of one XCD's turn. The empty rows are the last items of a subset;
+// turns of 16 gave some XCDs one more turn of work than others in every subset
+// of a small scanner (8 rings, 8 subsets, all of them: 101 us, 87 with turns of
+// 4 and of 1; larger images the same with all three).
+constexpr int kRowsXcdChunk = 4;
 struct RowGroup {
   int32_t row_start, row_len;
   int32_t first, nfam;  // fam_list[first .. first + nfam)
