@@ -17,10 +17,11 @@
 // (flag `inside` 0) tests the plane.
 // Each bin sums its row in row order, as fp_kernel does: the same values bit
 // for bit.
-// Measured: 8 rings x 192 crystals (5.4e5 bins of 116 elements) 0.358 -> 0.083 ms,
-// 16 rings x 288 (span 1) 1.23 -> 0.47 ms, 24 rings x 288 (span 3) 0.59 -> 0.50 ms.
-// From about 38 axial positions on fp_kernel is faster: its waves read one
-// image column per element, these read two or three.
+// Measured, tasks against row groups: 8 rings x 192 crystals (5.4e5 bins of 116
+// elements) 0.356 -> 0.063 ms, 16 rings x 288 (span 1, 128 x 128 columns) 1.21 ->
+// 0.43, 24 rings x 288 (span 3) 0.265 -> 0.207. They lose where families are
+// longer, images larger or a subset small (rows_pay in pmrt_capi.cpp has the
+// line): their waves read two or three image columns per element, tasks one.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>

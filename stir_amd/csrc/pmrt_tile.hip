@@ -44,10 +44,14 @@
 //
 // TOF: every (element, TOF bin it reaches) is an entry of its own, and every
 // TOF bin of a (segment, view) a viewgram with rows of its own: 2.1e9 terms at
-// mMR size with 11 TOF bins (up to 5 per element). 24.4 ms, against 48.2 with
+// mMR size with 11 TOF bins (up to 5 per element). 24.4 ms, against 45.7 with
 // the stored back records, whose five gathers per element also went to L2; per
-// term it costs what the non-TOF kernel does. The table is 17 GB beside 27 GB
-// of records and 200 ms more to make.
+// term it costs what the non-TOF kernel does. The table is 17 GB where the
+// records were 13.5, and takes 0.12 s more to make.
+//
+// One workgroup takes its time however few there are: images of few tiles (60 x
+// 60 columns: 0.25 to 0.8 times as fast) stay with the column kernels
+// (mi_ctx::min_tiles in pmrt_capi.cpp).
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
