@@ -3335,7 +3335,7 @@ int mi_batch_tune(mi_batch* b, int* choice) {
     struct Cand { int rg, gmax, widen, pack, tx, ty; };
     const Cand cands[] = {{32, 32, 0, 2, 32, 8},  {32, 32, 0, 0, 32, 8}, {16, 32, 0, 2, 32, 8}, {0, 32, 0, 2, 32, 8},
                           {0, 0, 0, 0, 32, 8},    {32, 32, 0, 2, 8, 8},  {32, 32, 0, 2, 16, 16}, {32, 32, 0, 1, 32, 8},
-                          {16, 32, 0, 2, 8, 64},  {16, 32, 0, 2, 8, 32}};
+                          {32, 32, 0, 2, 8, 64},  {32, 32, 0, 2, 8, 32}};
     hipEvent_t e0, e1;
     HIPCHECK(hipEventCreate(&e0));
     HIPCHECK(hipEventCreate(&e1));
