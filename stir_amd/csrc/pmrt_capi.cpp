@@ -805,9 +805,9 @@ void mi_ctx::build_row_groups() {
   std::vector<int32_t> list;
   std::vector<int2> items;
   item_off.assign(nsub + 1, 0);
-  // the subset's families by basic row, all of the empty rows as one: lists
-  // linked in family order (a sort of the families took 5 ms of the set-up of
-  // 3.5e5 of them, this 1). A row's families are one segment or +-pair: one length.
+  // the subset's families by basic row, all empty rows as one: lists linked in
+  // family order (sorting 3.5e5 families took 5 ms of a set-up, this takes 2). A
+  // row's families are one segment or +-pair: one length.
   const auto& keys = plan->family_keys();
   const int nrows = static_cast<int>(plan->basic_rays().size());
   std::vector<int> head(nrows + 1), tail(nrows + 1), seen(nrows + 1, -1), next(h_fams.size()), used;
